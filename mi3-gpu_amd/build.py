@@ -21,7 +21,11 @@ OUT = HERE / 'mi3gpu' / 'libmi3hip.so'
 BUILD = HERE / '_build'
 ARCH = os.environ.get('MI3_OFFLOAD_ARCH', 'gfx950')
 
-UNITS = ['runtime.hip', 'potts.hip', 'batch.hip', 'made.hip']
+# (source, object, extra flags)
+UNITS = [(u, Path(u).stem + '.o', []) for u in ('sweep_direct.hip', 'sweep_steps.hip', 'runtime.hip',
+                                                'potts.hip', 'batch.hip', 'made.hip')]
+# the chunk-staged sweep once for each number of state words
+UNITS += [('sweep_chunk.hip', f'sweep_chunk_{kw}.o', [f'-DMI3_KW={kw}']) for kw in range(1, 9)]
 
 CFLAGS = [
     f'--offload-arch={ARCH}', '-O3', '-fPIC', '-std=c++17',
@@ -35,10 +39,10 @@ def build(verbose=False):
     BUILD.mkdir(exist_ok=True)
     procs = []
     objs = []
-    for u in UNITS:
-        obj = BUILD / (Path(u).stem + '.o')
+    for u, o, extra in UNITS:
+        obj = BUILD / o
         objs.append(obj)
-        cmd = ['hipcc', *CFLAGS, '-c', str(CSRC / u), '-o', str(obj)]
+        cmd = ['hipcc', *CFLAGS, *extra, '-c', str(CSRC / u), '-o', str(obj)]
         if verbose:
             print(' '.join(cmd), flush=True)
         procs.append((u, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))

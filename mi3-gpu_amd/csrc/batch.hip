@@ -54,7 +54,9 @@ struct ClassKey {
 
 struct ClassRun {
     std::vector<uint32_t> models;
-    uint32_t wpb = 0;        // chosen walkers per tile
+    uint32_t wpb = 0;        // chosen walkers per tile (the largest: the library's choice)
+    uint32_t run_wpb = 0;    // walkers per tile as run
+    bool direct = false;     // swept without staging
     BatchTile* tiles = nullptr;
     uint32_t ntiles = 0;
     hipStream_t side = nullptr;
@@ -116,14 +118,32 @@ std::vector<uint32_t> tile_options(uint32_t kw) {
 }
 
 // Tiles of a class for a walkers-per-tile choice; larger models first so
-// that the tail of the persistent loop is short.
-int build_tiles(mi3_batch* b, ClassRun& cr, uint32_t wpb) {
+// that the tail of the persistent loop is short.  The largest tile stands for
+// the library's choice, as the single-model sweep makes it: no staging for a
+// class of few walkers, else the smaller of two tiles where it needs no more
+// rounds over the CUs (8 models of 1024-4096 walkers: 4 sweeps took 30.6 ms in
+// tiles of 512, all on the two work-groups of the L=400 model).
+int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
+    uint64_t total = 0;
+    uint32_t qmin = MAX_Q;
+    for (uint32_t m : cr.models) {
+        total += b->N[m];
+        qmin = std::min(qmin, b->q[m]);
+    }
+    const uint32_t ncu = b->ncu ? b->ncu : 256;
+    cr.direct = false;
+    cr.run_wpb = wpb;
+    if (wpb == tile_options(key.kw).back()) {
+        cr.direct = total <= direct_walkers(qmin, ncu);
+        auto rounds = [&](uint32_t w) { return (total / w + ncu - 1) / ncu; };
+        while (cr.run_wpb > 128 && rounds(cr.run_wpb / 2) == rounds(cr.run_wpb)) cr.run_wpb /= 2;
+    }
     std::vector<BatchTile> t;
     std::vector<uint32_t> order = cr.models;
     std::stable_sort(order.begin(), order.end(),
                      [&](uint32_t x, uint32_t y) { return b->L[x] > b->L[y]; });
     for (uint32_t m : order)
-        for (uint32_t blk = 0; blk < b->N[m] / wpb; blk++) t.push_back({m, blk});
+        for (uint32_t blk = 0; blk < b->N[m] / cr.run_wpb; blk++) t.push_back({m, blk});
     if (cr.tiles) hipFree(cr.tiles);
     cr.tiles = nullptr;
     BCHK(b, hipMalloc(&cr.tiles, std::max<size_t>(1, t.size()) * sizeof(BatchTile)));
@@ -135,6 +155,19 @@ int build_tiles(mi3_batch* b, ClassRun& cr, uint32_t wpb) {
 
 uint32_t class_grid(mi3_batch* b, const ClassRun& cr) {
     return std::min<uint32_t>(cr.ntiles, b->ncu ? b->ncu : 256);
+}
+
+// The sweep of one class on stream st.
+hipError_t sweep_class(mi3_batch* b, const ClassKey& key, const ClassRun& cr, uint32_t* counter,
+                       hipStream_t st) {
+    if (cr.direct) {
+        uint32_t qmin = MAX_Q;
+        for (uint32_t m : cr.models) qmin = std::min(qmin, b->q[m]);
+        return launch_sweep_batch_direct(key.kw, qmin, cr.run_wpb, cr.ntiles * cr.run_wpb,
+                                         b->ncu ? b->ncu : 256, b->models, cr.tiles, cr.ntiles, st);
+    }
+    return launch_sweep_batch(key.kw, key.pf, cr.run_wpb, b->models, cr.tiles, cr.ntiles, counter,
+                              class_grid(b, cr), st);
 }
 
 // Per-model descriptors for nsweeps sweeps (nsteps = nsweeps * L).
@@ -196,8 +229,7 @@ int enqueue_round(mi3_batch* b, std::vector<hipEvent_t>& events) {
         ClassRun& cr = kv.second;
         hipStream_t s = cr.side;
         if (hipStreamWaitEvent(s, fork, 0) != hipSuccess) { rc = bfail(b, MI3_EHIP, "fork"); break; }
-        hipError_t e = launch_sweep_batch(kv.first.kw, kv.first.pf, cr.wpb, b->models, cr.tiles,
-                                          cr.ntiles, b->counters + ci, class_grid(b, cr), s);
+        hipError_t e = sweep_class(b, kv.first, cr, b->counters + ci, s);
         if (e != hipSuccess) {
             rc = bfail(b, MI3_EHIP, std::string("batch sweep: ") + hipGetErrorString(e));
             break;
@@ -305,7 +337,7 @@ int mi3_batch_create(int device, uint32_t nmodels, const uint32_t* L, const uint
             if (rc != MI3_OK) break;
             if (hipStreamCreate(&kv.second.side) != hipSuccess) { bad("stream"); break; }
             // default tile: the largest allowed
-            if (build_tiles(b, kv.second, tile_options(kv.first.kw).back()) != MI3_OK)
+            if (build_tiles(b, kv.first, kv.second, tile_options(kv.first.kw).back()) != MI3_OK)
                 bad("tiles");
         }
         if (hipStreamSynchronize(b->stream) != hipSuccess) bad("sync");
@@ -434,7 +466,7 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
         float best = 1e30f;
         uint32_t best_w = cr.wpb;
         for (uint32_t w : tile_options(kv.first.kw)) {
-            rc = build_tiles(b, cr, w);
+            rc = build_tiles(b, kv.first, cr, w);
             if (rc) break;
             // positions for this launch, then the class sweep alone; the
             // step counters advance as after any launch
@@ -445,9 +477,7 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
                                0, b->stream, (const BatchModel*)b->models,
                                (uint32_t* const*)b->pos_ptrs);
             hipEventRecord(e0, b->stream);
-            hipError_t e = launch_sweep_batch(kv.first.kw, kv.first.pf, w, b->models, cr.tiles,
-                                              cr.ntiles, b->counters + ci, class_grid(b, cr),
-                                              b->stream);
+            hipError_t e = sweep_class(b, kv.first, cr, b->counters + ci, b->stream);
             hipEventRecord(e1, b->stream);
             hipLaunchKernelGGL(k_batch_advance, dim3((b->n + 255) / 256), dim3(256), 0, b->stream,
                                (const BatchModel*)b->models, b->steps, b->n);
@@ -463,7 +493,7 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
             }
         }
         if (rc) break;
-        rc = build_tiles(b, cr, best_w);
+        rc = build_tiles(b, kv.first, cr, best_w);
         if (rc) break;
         ci++;
     }
@@ -488,7 +518,7 @@ int mi3_batch_set_tile(mi3_batch* b, uint32_t model, uint32_t wpb) {
     hipSetDevice(b->dev);
     BCHK(b, hipStreamSynchronize(b->stream));
     drop_graph(b);
-    return build_tiles(b, b->classes[k], wpb);
+    return build_tiles(b, k, b->classes[k], wpb);
 }
 
 int mi3_batch_step_count(mi3_batch* b, uint32_t model, uint64_t* steps) {

@@ -20,6 +20,8 @@
 #include "common.h"
 #include "launch.h"
 
+#include <type_traits>
+
 namespace mi3 {
 
 // Native 4-float vector (HIP's float4 is a union-based struct, which keeps
@@ -59,25 +61,6 @@ constexpr int ilog2(int x) { return x <= 1 ? 0 : 1 + ilog2(x / 2); }
 constexpr int SWEEP_G = 8;
 constexpr int SWEEP_P = 1;
 
-// Wave-wide lane masks: bit `lane` set when (lane & m) != 0.
-__device__ __forceinline__ constexpr uint64_t lane_bit_mask(int m) {
-    return m == 16 ? 0xFFFF0000FFFF0000ull
-         : m == 8  ? 0xFF00FF00FF00FF00ull
-         : m == 4  ? 0xF0F0F0F0F0F0F0F0ull
-         : m == 2  ? 0xCCCCCCCCCCCCCCCCull
-                   : 0xAAAAAAAAAAAAAAAAull;
-}
-
-// mask[lane] ? a : b as one v_cndmask.  Written as asm so that the
-// optimizer cannot turn a select between two elements of one register array
-// back into a lane-varying array index (which it lowers to a long
-// compare/select chain).
-__device__ __forceinline__ float lane_select(uint64_t mask, float a, float b) {
-    float r;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(mask));
-    return r;
-}
-
 // Value of v in the partner lane of a reduction level below 16, within a
 // row of 16 lanes, by DPP: m=8 row_ror:8 (lane ^ 8), m=4 row_half_mirror
 // (lane ^ 7: the pair differs in bit 2, and in bits 0-1, which the later
@@ -97,11 +80,13 @@ __device__ __forceinline__ float dpp_partner(float v, int m) {
 // slot j >> (5 - log2 S).  The first level pairs lanes j and j + 16: one
 // v_permlane16_swap exchanges the odd 16-lane rows of v[s] with the even
 // rows of v[s + h], so one add leaves rows 0 and 2 with slot s and rows 1
-// and 3 with slot s + h, with no selects.  Each later level keeps one of two
-// slots by the lane's bit m (v_cndmask with constant lane masks) and adds
-// the other slot's value from the partner lane through DPP.  No LDS.
+// and 3 with slot s + h, with no selects.  Each later level adds the partner
+// lane's value to both slots of a pair (DPP inside the add) and keeps one of
+// them by the lane's bit m.  No LDS, and no inline asm: the wait states that
+// a DPP read needs after its source is written are inserted by the compiler
+// only behind instructions it knows.
 template <int S>
-__device__ __forceinline__ float transposed_sum(float (&v)[S]) {
+__device__ __forceinline__ float transposed_sum(float (&v)[S], uint32_t lane) {
     int n = S;
     if (n > 1) {
         const int h = n / 2;
@@ -116,22 +101,20 @@ __device__ __forceinline__ float transposed_sum(float (&v)[S]) {
         }
         n = h;
     } else {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]),
-                                                        __float_as_uint(v[0]), false, false);
-        v[0] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        // one slot: lane j ^ 16 through ds_swizzle
+        v[0] += swz_xor<16>(v[0]);
     }
 #pragma unroll
     for (int l = 1; l < 5; l++) {
         const int m = 16 >> l;
         if (n > 1) {
             const int h = n / 2;
-            const uint64_t mk = lane_bit_mask(m);
 #pragma unroll
             for (int s = 0; s < S / 2; s++) {
                 if (s < h) {
-                    float send = lane_select(mk, v[s], v[s + h]);
-                    float keep = lane_select(mk, v[s + h], v[s]);
-                    v[s] = keep + dpp_partner(send, m);
+                    const float x = v[s] + dpp_partner(v[s], m);
+                    const float y = v[s + h] + dpp_partner(v[s + h], m);
+                    v[s] = (lane & m) ? y : x;
                 }
             }
             n = h;
@@ -190,24 +173,6 @@ __device__ __forceinline__ void barrier_copies_in_flight() {
     asm volatile("s_barrier" ::: "memory");
 }
 
-// Value of `v` in lane (src + 32*half) of each half-wave, src a compile-time
-// lane number < 32 (ds_swizzle bitmask mode: and 0, or src).
-#define MI3_SWZ_CASE(n) \
-    case n:             \
-        return __builtin_amdgcn_ds_swizzle(v, (n) << 5);
-__device__ __forceinline__ int half_bcast(int v, int src) {
-    switch (src) {
-        MI3_SWZ_CASE(0) MI3_SWZ_CASE(1) MI3_SWZ_CASE(2) MI3_SWZ_CASE(3) MI3_SWZ_CASE(4)
-        MI3_SWZ_CASE(5) MI3_SWZ_CASE(6) MI3_SWZ_CASE(7) MI3_SWZ_CASE(8) MI3_SWZ_CASE(9)
-        MI3_SWZ_CASE(10) MI3_SWZ_CASE(11) MI3_SWZ_CASE(12) MI3_SWZ_CASE(13) MI3_SWZ_CASE(14)
-        MI3_SWZ_CASE(15) MI3_SWZ_CASE(16) MI3_SWZ_CASE(17) MI3_SWZ_CASE(18) MI3_SWZ_CASE(19)
-        MI3_SWZ_CASE(20) MI3_SWZ_CASE(21) MI3_SWZ_CASE(22) MI3_SWZ_CASE(23) MI3_SWZ_CASE(24)
-        MI3_SWZ_CASE(25) MI3_SWZ_CASE(26) MI3_SWZ_CASE(27) MI3_SWZ_CASE(28) MI3_SWZ_CASE(29)
-        MI3_SWZ_CASE(30) default: return __builtin_amdgcn_ds_swizzle(v, 31 << 5);
-    }
-}
-#undef MI3_SWZ_CASE
-
 // ---------------------------------------------------------------------------
 // Chunk ring with overlapping slots, for the 57,344-byte padded chunks of
 // q = 17..21 (7 float4 per thread of 512 staging threads).  Two such chunks
@@ -262,20 +227,6 @@ struct OverlapRing {
 static_assert(OverlapRing::CHB == 7 * 512 * 16, "padded chunk of the PF = 7 class");
 static_assert(OverlapRing::BYTES == 106496 + OverlapRing::CHB, "slots fill the LDS");
 
-template <int KW>
-__device__ __forceinline__ uint32_t select_word_opaque(const uint32_t (&w)[KW], uint32_t idx) {
-    if constexpr (KW == 1) return w[0];
-    if constexpr (KW == 2) return idx ? w[1] : w[0];
-    uint32_t r = w[0];
-#pragma unroll
-    for (int k = 1; k < KW; k++) {
-        uint32_t t = w[k];
-        asm("" : "+v"(t));
-        r = (idx == (uint32_t)k) ? t : r;
-    }
-    return r;
-}
-
 // 128 * byte e of w (e a compile-time constant after unrolling) in one
 // VALU op: a shift with an SDWA byte select on its source.  Left to itself
 // the compiler makes byte 0 a shift and a mask.
@@ -310,12 +261,6 @@ __device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c) 
     return r;
 }
 
-__device__ __forceinline__ uint32_t lane_select_u(uint64_t mask, uint32_t a, uint32_t b) {
-    uint32_t r;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(mask));
-    return r;
-}
-
 // ---------------------------------------------------------------------------
 // Metropolis sweep: nsteps single-site updates per walker.
 //
@@ -327,13 +272,229 @@ __device__ __forceinline__ uint32_t lane_select_u(uint64_t mask, uint32_t a, uin
 // Restates metropolis/DeltaEnergy (mcmc.cl:360-458) with counter-based
 // streams in place of MWC64X.
 //
-// Per step: lane j draws the random numbers of walker slot j >> SH; each
-// lane then fetches, for every slot, the walker's current residue a (from
-// the lane owning site pos, ds_bpermute) and proposal b (ds_swizzle
-// broadcast), gathers J(a, s_m) and J(b, s_m) for its sites chunk by chunk,
-// and one transposed butterfly leaves each lane with the dE of its own slot;
-// it decides, and a ballot tells the owner lane of pos which walkers accepted.
-//
+// Per step: lane j draws the random numbers of walker slot j >> SH; every
+// lane then needs, for every slot, the walker's current residue a (held by
+// the lane owning site pos) and proposal b, gathers J(a, s_m) and J(b, s_m)
+// for its sites chunk by chunk, and one transposed butterfly leaves each lane
+// with the dE of its own slot; it decides, and the owner lane of pos takes the
+// accepted residues.  Three forms share this step and differ in where the
+// gathers read (all give the same sums in the same order, bit for bit):
+//   sweep_block    chunks staged in LDS one at a time, one barrier per chunk:
+//                  rows of couplings too large to hold (q > 8, long chains)
+//   sweep_steps    the whole rows of several steps staged at once, one
+//                  barrier per stage: small alphabets
+//   sweep_direct   no staging, one wave per work-group gathering from L2:
+//                  too few walkers to pay for a staged row
+
+// Value of v in lane e of each row of 16 lanes (DPP row_newbcast).
+#define MI3_RB_CASE(E) \
+    case E:            \
+        return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x150 + E, 0xF, 0xF, false);
+__device__ __forceinline__ uint32_t row_bcast(uint32_t v, int e) {
+    switch (e) {
+        MI3_RB_CASE(0) MI3_RB_CASE(1) MI3_RB_CASE(2) MI3_RB_CASE(3) MI3_RB_CASE(4)
+        MI3_RB_CASE(5) MI3_RB_CASE(6) MI3_RB_CASE(7) MI3_RB_CASE(8) MI3_RB_CASE(9)
+        MI3_RB_CASE(10) MI3_RB_CASE(11) MI3_RB_CASE(12) MI3_RB_CASE(13) MI3_RB_CASE(14)
+        default: return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x15F, 0xF, 0xF, false);
+    }
+}
+#undef MI3_RB_CASE
+
+// The walkers of a wave and what a step does with them around its gathers.
+// QB: q <= 16, so that a residue times q fits a byte.
+template <int KW, int S, bool QB>
+struct Walkers {
+    static constexpr int SH = 5 - ilog2(S);  // lane j reduces and decides slot j >> SH
+    // lanes of a quad that decide the same slot: each draws another pair of steps
+    static constexpr int R = S == 16 ? 2 : 4;
+    static_assert((1 << ilog2(S)) == S && S <= 16, "S must be a power of two <= 16");
+
+    static constexpr int NP = (S + 3) / 4;   // residues of a site, four slots to a word
+
+    uint32_t st[S][KW];       // residues of sites j + 32k, four to a word
+    uint32_t apk[NP];         // this step's current residues, byte s % 4 of word s / 4
+    uint32_t Xe, Xo;          // this lane's draws (steps 2h, 2h+1 of its own pair)
+    uint32_t Pe, Po;          // draws of the current pair of steps
+    int remap;                // bpermute address: row lane e <- the lane deciding slot e
+
+    __device__ __forceinline__ void load(const uint8_t* seq, uint32_t ldseq, uint32_t L,
+                                         uint32_t wfirst, uint32_t lane) {
+        const uint32_t j = lane & 31;
+        remap = (int)((((lane & 15) << SH) & 31) | (lane & 32)) * 4;
+        Xe = Xo = Pe = Po = 0;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+#pragma unroll
+            for (int i = 0; i < KW; i++) {
+                uint32_t word = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    uint32_t m = j + CH * (4 * i + e);
+                    uint32_t v = (m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
+                    word |= v << (8 * e);
+                }
+                st[s][i] = word;
+            }
+            asm volatile("" ::: "memory");
+        }
+    }
+
+    __device__ __forceinline__ void store(uint8_t* seq, uint32_t ldseq, uint32_t L,
+                                          uint32_t wfirst, uint32_t lane) const {
+        const uint32_t j = lane & 31;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+#pragma unroll
+            for (int i = 0; i < KW; i++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    uint32_t m = j + CH * (4 * i + e);
+                    if (m < L) seq[(size_t)m * ldseq + wfirst + s] = (uint8_t)(st[s][i] >> (8 * e));
+                }
+            }
+        }
+    }
+
+    // Draws of step t of the launch (step0 even).  The lanes deciding one
+    // slot share the work: lane i of R draws the steps 2(h + i), 2(h + i) + 1
+    // every R pairs of steps, and a quad permutation hands each pair out.
+    __device__ __forceinline__ uint32_t draws(uint32_t t, uint64_t step0, uint32_t walker,
+                                              uint32_t lane, uint32_t q, uint32_t k0,
+                                              uint32_t k1) {
+        if ((t & 1) == 0) {
+            const uint32_t i = (t >> 1) & (R - 1);
+            if (i == 0) {
+                const uint64_t h = ((step0 + t) >> 1) + (lane & (R - 1));
+                uint4 r = philox4x32_10(make_uint4((uint32_t)h, (uint32_t)(h >> 32), walker,
+                                                   TAG_WALK), k0, k1);
+                Xe = ((r.y >> 8) << 8) | mulhi_range(r.x, q);
+                Xo = ((r.w >> 8) << 8) | mulhi_range(r.z, q);
+            }
+            auto hand = [&](auto ctrl) {
+                Pe = (uint32_t)__builtin_amdgcn_mov_dpp((int)Xe, decltype(ctrl)::value, 0xF, 0xF,
+                                                        false);
+                Po = (uint32_t)__builtin_amdgcn_mov_dpp((int)Xo, decltype(ctrl)::value, 0xF, 0xF,
+                                                        false);
+            };
+            if constexpr (R == 2) {
+                if (i == 0) hand(std::integral_constant<int, 0xA0>{});   // quad 0,0,2,2
+                else hand(std::integral_constant<int, 0xF5>{});          // quad 1,1,3,3
+            } else {
+                if (i == 0) hand(std::integral_constant<int, 0x00>{});
+                else if (i == 1) hand(std::integral_constant<int, 0x55>{});
+                else if (i == 2) hand(std::integral_constant<int, 0xAA>{});
+                else hand(std::integral_constant<int, 0xFF>{});
+            }
+            return Pe;
+        }
+        return Po;
+    }
+
+    // Row addresses of every slot: baseA, baseB = (a, b) * q * 128 + origin
+    // (origin: this lane's column, plus where the couplings of the site
+    // start).  The current residues are packed four slots to a word, so one
+    // ds_bpermute from the owner lane serves four slots; the proposals move
+    // to row lane s once, and each slot's is broadcast by DPP inside the add.
+    // (A ds_bpermute takes the LDS 2.5 times as long as a gather; before, every
+    // slot took one, and two swizzles.)
+    __device__ __forceinline__ void bases(uint32_t pos, uint32_t lane, uint32_t bmine, uint32_t q,
+                                          uint32_t origin, uint32_t (&baseA)[S],
+                                          uint32_t (&baseB)[S]) {
+        const uint32_t kp = pos >> 5, owner = pos & 31;
+        const uint32_t wd = kp >> 2, e0 = kp & 3;
+        const int own_addr = (int)((owner + (lane & 32)) * 4);
+        // (opaque, so that the compiler does not turn the adds of disjoint bit
+        // ranges below into ors, which do not fuse with the products)
+        uint32_t org = origin;
+        asm("" : "+v"(org));
+        const uint32_t bl = (uint32_t)__builtin_amdgcn_ds_bpermute(remap, (int)bmine);
+#pragma unroll
+        for (int i = 0; i < KW; i++) {
+            if (KW == 1 || wd == (uint32_t)i) {
+#pragma unroll
+                for (int g = 0; g < NP; g++) {
+                    uint32_t p;
+                    if constexpr (S == 1)
+                        p = __builtin_amdgcn_ubfe(st[0][i], e0 * 8, 8);
+                    else
+                        p = __builtin_amdgcn_perm(st[4 * g + 1][i], st[4 * g][i],
+                                                  0x0c0c0400u + e0 * 0x00000101u);
+                    if constexpr (S >= 4)
+                        p |= __builtin_amdgcn_perm(st[4 * g + 3][i], st[4 * g + 2][i],
+                                                   0x04000c0cu + e0 * 0x01010000u);
+                    apk[g] = p;
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < NP; g++)
+            apk[g] = (uint32_t)__builtin_amdgcn_ds_bpermute(own_addr, (int)apk[g]);
+        const uint32_t brow = __umul24(bl, q * (CH * 4));
+#pragma unroll
+        for (int s = 0; s < S; s++) baseB[s] = row_bcast(brow, s) + org;
+#pragma unroll
+        for (int g = 0; g < NP; g++) {
+            const uint32_t aq = QB ? apk[g] * q : apk[g];
+#pragma unroll
+            for (int s = 4 * g; s < 4 * g + 4 && s < S; s++)
+                baseA[s] = QB ? byte_x128(aq, s & 3) + org : __umul24(byte_x128(aq, s & 3), q) + org;
+        }
+    }
+
+    // LDS or memory addresses of a slot's gathers from chunk k
+    __device__ __forceinline__ void gather_addr(int s, int k, uint32_t baseA, uint32_t baseB,
+                                                uint32_t& aA, uint32_t& aB) const {
+        const uint32_t off = byte_x128(st[s][k >> 2], k & 3);
+        aA = baseA + off;
+        aB = baseB + off;
+    }
+
+    // Accept or reject: this lane decides for its slot, and the owner lanes
+    // of pos take every slot's residue, the proposal or the current one.
+    // Residues and decisions reach them as packed bytes, so a slot costs one
+    // byte permute there, with no lane mask of its own.
+    __device__ __forceinline__ void accept(uint32_t pos, uint32_t lane, float (&acc)[S],
+                                           uint32_t Pcur, float nbeta) {
+        const uint32_t kp = pos >> 5, owner = pos & 31;
+        const uint32_t wd = kp >> 2, e0 = kp & 3;
+        const float dE = transposed_sum<S>(acc, lane);
+        const float u = (float)(Pcur >> 8) * 0x1.0p-24f;
+        // byte 0 the proposal, byte 1 all ones where it is accepted
+        uint32_t v = (Pcur & 0xffu) | (__expf(nbeta * dE) > u ? 0xff00u : 0u);
+        v = (uint32_t)__builtin_amdgcn_ds_bpermute(remap, (int)v);
+        // row lane 4g: the four slots' proposals and masks
+        const uint32_t y =
+            (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xF5, 0xF, 0xF, false);  // quad 1,1,3,3
+        const uint32_t z = __builtin_amdgcn_perm(y, v, 0x05010400u);
+        const uint32_t y2 =
+            (uint32_t)__builtin_amdgcn_mov_dpp((int)z, 0xAA, 0xF, 0xF, false);  // quad 2,2,2,2
+        const uint32_t bp = __builtin_amdgcn_perm(y2, z, 0x05040100u);
+        const uint32_t mp = __builtin_amdgcn_perm(y2, z, 0x07060302u);
+        uint32_t npk[NP];
+#pragma unroll
+        for (int g = 0; g < NP; g++) {
+            const uint32_t m = row_bcast(mp, 4 * g);
+            npk[g] = (row_bcast(bp, 4 * g) & m) | (apk[g] & ~m);
+        }
+        // owner lanes put byte e of the new residues at pos's byte; the
+        // others keep their word
+        const bool own = (lane & 31) == owner;
+        const uint32_t keep = 0x07060504u & ~(0xffu << (8 * e0));
+        uint32_t sel[S < 4 ? S : 4];
+#pragma unroll
+        for (int e = 0; e < (S < 4 ? S : 4); e++)
+            sel[e] = own ? keep | ((uint32_t)e << (8 * e0)) : 0x07060504u;
+#pragma unroll
+        for (int i = 0; i < KW; i++) {
+            if (KW == 1 || wd == (uint32_t)i) {
+#pragma unroll
+                for (int s = 0; s < S; s++)
+                    st[s][i] = __builtin_amdgcn_perm(st[s][i], npk[s / 4], sel[s & 3]);
+            }
+        }
+    }
+};
+
 // sweep_block runs the walkers of work-group tile `block` (W = 2*S*NWAVES
 // walkers starting at walker block*W); k_sweep is one tile per work-group,
 // k_sweep_batch a persistent loop over the tiles of many models.
@@ -344,23 +505,19 @@ __device__ __forceinline__ void sweep_block(
     uint32_t k1, uint64_t step0, uint32_t walker_base, float nbeta, uint32_t block) {
     constexpr int NT = 64 * NWAVES;
     constexpr int K = 4 * KW;
-    constexpr int SH = 5 - ilog2(S);  // lane j reduces and decides slot j >> SH
-    static_assert((1 << ilog2(S)) == S && S <= 32, "S must be a power of two <= 32");
+    using W = Walkers<KW, S, (PF <= 4)>;
     extern __shared__ f4v lds4[];
     char* ldsb = reinterpret_cast<char*>(lds4);
 
     // the padded chunk is PF float4 per thread of the first DMA_T threads
     // (the chunk layout's unit); waves beyond them take no part in staging
     constexpr int DMA_T = NT < 512 ? NT : 512;
-    constexpr uint32_t chf = PF * DMA_T * 4;  // padded chunk (floats)
-    constexpr uint32_t chb = chf * 4;      // padded chunk (bytes)
+    constexpr uint32_t chb = PF * DMA_T * 16;  // padded chunk (bytes)
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const uint32_t lane = tid & 63;
     const uint32_t j = lane & 31;
-    const bool upper = lane >= 32;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wfirst = block * (2 * S * NWAVES) + (wave * 2 + (upper ? 1 : 0)) * S;
-    const uint32_t myslot = j >> SH;
+    const uint32_t wfirst = block * (2 * S * NWAVES) + (wave * 2 + (lane >> 5)) * S;
     const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * nchunk * chb);
     const uint32_t voff = tid * 16;
     // staging waves: each copies one float4 per lane per pass; a single-pass
@@ -369,27 +526,10 @@ __device__ __forceinline__ void sweep_block(
     // 3-4% faster at q = 3..4 than copying all 8 KB)
     const bool stage = (PF == 1) ? (uint32_t)wave < (q * q + 7) / 8 : wave < DMA_T / 64;
 
-    // walker state: residues of sites j + 32k
-    uint32_t st[S][KW];
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-#pragma unroll
-        for (int kw = 0; kw < KW; kw++) {
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                uint32_t m = j + CH * (4 * kw + e);
-                uint32_t v = (m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
-                word |= v << (8 * e);
-            }
-            st[s][kw] = word;
-        }
-        asm volatile("" ::: "memory");
-    }
-
+    W w;
+    w.load(seq, ldseq, L, wfirst, lane);
     uint32_t baseA[S], baseB[S];  // LDS byte offsets of rows a and b (+ lane column)
     float acc[S];
-    uint32_t Pe = 0, Po = 0;      // this lane's walker draws for steps 2h, 2h+1
 
     if (nsteps == 0) return;
     // site of the current step; the next one is read one step ahead (with
@@ -401,48 +541,19 @@ __device__ __forceinline__ void sweep_block(
     if (stage) chunk_dma<PF, DMA_T>(rJ, voff, pos * nchunk * chb, ldsb, wave);
     wait_vmem();
     __syncthreads();
-    uint32_t buf = 0;
-    const uint32_t qch4 = q * CH * 4;
     const uint32_t j4 = j * 4;
 
-    for (uint32_t t = 0; t < nsteps; t++) {
+    // one step whose chunk 0 is in buffer B0: chunk k is in buffer
+    // (B0 + k) % 2, so that the buffer is a constant offset of each read and
+    // an address is one instruction per gather (the byte dot product of
+    // byte_x128_add)
+    auto step = [&](auto b0c, uint32_t t) __attribute__((always_inline)) {
+        constexpr uint32_t B0 = decltype(b0c)::value;
         const uint32_t pos_after =
             (t + 2 < nsteps) ? __builtin_amdgcn_readfirstlane(pos_list[t + 2]) : 0u;
-        const uint32_t kp = pos >> 5, owner = pos & 31;
-        const uint32_t kwp = kp >> 2, shp = (kp & 3) * 8;
-        if ((t & 1) == 0) {
-            const uint64_t h = (step0 + t) >> 1;
-            uint4 r = philox4x32_10(make_uint4((uint32_t)h, (uint32_t)(h >> 32),
-                                               walker_base + wfirst + myslot, TAG_WALK),
-                                    k0, k1);
-            Pe = ((r.y >> 8) << 8) | mulhi_range(r.x, q);
-            Po = ((r.w >> 8) << 8) | mulhi_range(r.z, q);
-        }
-        const uint32_t Pcur = (t & 1) ? Po : Pe;
-        const uint32_t bmine = Pcur & 0xffu;
-        const int own_addr = (int)((owner + (lane & 32)) * 4);
-        // the proposal as a row offset, scaled by its sender so that every
-        // receiving lane adds only its column
-        const int brow = (int)__umul24(bmine, qch4);
-        // residues a (from the owner lane of pos) and proposals b of every
-        // slot, fetched in groups ahead of their use
-        constexpr int GB = (S < 8) ? S : 8;
-#pragma unroll
-        for (int s0 = 0; s0 < S; s0 += GB) {
-            uint32_t a[GB], b[GB];
-#pragma unroll
-            for (int g = 0; g < GB; g++) {
-                const int s = s0 + g;
-                const uint32_t av = __builtin_amdgcn_ubfe(select_word_opaque<KW>(st[s], kwp), shp, 8);
-                a[g] = (uint32_t)__builtin_amdgcn_ds_bpermute(own_addr, (int)av);
-                b[g] = (uint32_t)half_bcast(brow, s << SH);
-            }
-#pragma unroll
-            for (int g = 0; g < GB; g++) {
-                baseA[s0 + g] = mad_u24(a[g], qch4, j4);
-                baseB[s0 + g] = b[g] + j4;
-            }
-        }
+        const uint32_t Pcur =
+            w.draws(t, step0, walker_base + wfirst + (j >> W::SH), lane, q, k0, k1);
+        w.bases(pos, lane, Pcur & 0xffu, q, j4, baseA, baseB);
         // stream the couplings of site pos, chunk by chunk
 #pragma unroll
         for (int k = 0; k < K; k++) {
@@ -450,6 +561,7 @@ __device__ __forceinline__ void sweep_block(
             if (k == 0 || (uint32_t)k < nchunk) {
                 const bool last_chunk = (uint32_t)k + 1 == nchunk;
                 const bool has_next = !last_chunk || (t + 1 < nsteps);
+                const uint32_t buf = (B0 + k) & 1;
                 if (has_next) {
                     uint32_t npos = last_chunk ? pos_next : pos;
                     uint32_t nc = last_chunk ? 0u : (uint32_t)k + 1;
@@ -473,10 +585,10 @@ __device__ __forceinline__ void sweep_block(
                         for (int g = 0; g < G; g++) {
                             const int s = i * G + g;
                             static_assert(CH * 4 == 128, "row stride of a chunk");
-                            const uint32_t off =
-                                byte_x128(state_word<KW>(st[s], (uint32_t)k >> 2), k & 3);
-                            vA[s] = *reinterpret_cast<const float*>(cb + baseA[s] + off);
-                            vB[s] = *reinterpret_cast<const float*>(cb + baseB[s] + off);
+                            uint32_t aA, aB;
+                            w.gather_addr(s, k, baseA[s], baseB[s], aA, aB);
+                            vA[s] = *reinterpret_cast<const float*>(cb + aA);
+                            vB[s] = *reinterpret_cast<const float*>(cb + aB);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -493,53 +605,200 @@ __device__ __forceinline__ void sweep_block(
                 }
                 wait_vmem();
                 __syncthreads();
-                buf ^= 1;
             }
         }
-        // accept / reject: this lane decides for walker slot `myslot`
-        const float dE = transposed_sum<S>(acc);
-        const float u = (float)(Pcur >> 8) * 0x1.0p-24f;
-        const uint64_t amask = __ballot(__expf(nbeta * dE) > u);
-        // the owner lanes of pos take the proposals their half-wave accepted:
-        // all proposal broadcasts are issued together (one LDS wait), the
-        // state word holding pos is chosen once per step, and each slot's
-        // lane mask takes three scalar operations
-        uint32_t bnew[S];
-        const int bsh = (int)(bmine << shp);  // the proposal at its byte of the word
-#pragma unroll
-        for (int s = 0; s < S; s++) bnew[s] = (uint32_t)half_bcast(bsh, s << SH);
-        const uint32_t keep = ~(0xffu << shp);
-#pragma unroll
-        for (int kw = 0; kw < KW; kw++) {
-            if (kwp == (uint32_t)kw) {
-#pragma unroll
-                for (int s = 0; s < S; s++) {
-                    // bits 0 and 32 of the shifted ballot are the two
-                    // half-waves' decisions for slot s; moved to the owner lanes
-                    const uint64_t m = ((amask >> (s << SH)) & 0x0000000100000001ull) << owner;
-                    const uint32_t nw = (st[s][kw] & keep) | bnew[s];
-                    st[s][kw] = lane_select_u(m, nw, st[s][kw]);
-                }
-            }
-        }
+        w.accept(pos, lane, acc, Pcur, nbeta);
         pos = pos_next;
         pos_next = pos_after;
+    };
+    uint32_t b0 = 0;
+    const uint32_t flip = nchunk & 1;
+    for (uint32_t t = 0; t < nsteps; t++) {
+        if (b0) step(std::integral_constant<uint32_t, 1>{}, t);
+        else step(std::integral_constant<uint32_t, 0>{}, t);
+        b0 ^= flip;
     }
-
-    // write back
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-#pragma unroll
-        for (int kw = 0; kw < KW; kw++) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                uint32_t m = j + CH * (4 * kw + e);
-                if (m < L) seq[(size_t)m * ldseq + wfirst + s] = (uint8_t)(st[s][kw] >> (8 * e));
-            }
-        }
-    }
+    w.store(seq, ldseq, L, wfirst, lane);
 }
 
+// The whole rows of several steps staged at once: a stage holds `nst` steps
+// (nst * nchunk chunks of NPC KB, of which the first ceil(q*q/8) KB are
+// copied), double-buffered, one barrier per stage.  Inside a stage no wave
+// waits for another, so the latencies of one wave's reduction and acceptance
+// overlap the gathers of the others.
+template <int KW, int S, int NWAVES, int NPC>
+__device__ __forceinline__ void sweep_steps(
+    const float* __restrict__ Ju, uint8_t* __restrict__ seq, const uint32_t* __restrict__ pos_list,
+    uint32_t ldseq, uint32_t L, uint32_t q, uint32_t nchunk, uint32_t nsteps, uint32_t k0,
+    uint32_t k1, uint64_t step0, uint32_t walker_base, float nbeta, uint32_t block, uint32_t nst) {
+    constexpr int K = 4 * KW;
+    constexpr uint32_t SLOT = NPC * 1024;     // a chunk in LDS
+    constexpr uint32_t chb = 8192;            // a padded chunk in memory (q <= 8)
+    using W = Walkers<KW, S, true>;
+    extern __shared__ f4v lds4[];
+    char* ldsb = reinterpret_cast<char*>(lds4);
+    const int tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t j = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wfirst = block * (2 * S * NWAVES) + (wave * 2 + (lane >> 5)) * S;
+    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * nchunk * chb);
+    const uint32_t voff = lane * 16;
+    if (nsteps == 0) return;
+    const uint32_t rowb = nchunk * SLOT, stageb = nst * rowb;
+    // KB pieces of a row, dealt to the waves over all steps of a stage
+    const uint32_t npc = (q * q + 7) / 8, rp = nchunk * npc;
+    const uint32_t inv = 65536 / npc + 1;     // r / npc for r < 256
+    auto copy_stage = [&](uint32_t t0, uint32_t buf) {
+        const uint32_t n = nsteps - t0 < nst ? nsteps - t0 : nst;
+        uint32_t g = 0, r = wave;
+        while (r >= rp) {
+            r -= rp;
+            g++;
+        }
+        while (g < n) {
+            const uint32_t pos = __builtin_amdgcn_readfirstlane(pos_list[t0 + g]);
+            const uint32_t k = (r * inv) >> 16, piece = r - k * npc;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rJ, (lds_void*)(ldsb + buf * stageb + g * rowb + k * SLOT + piece * 1024), 16, voff,
+                (pos * nchunk + k) * chb + piece * 1024, 0, 0);
+            r += NWAVES;
+            while (r >= rp) {
+                r -= rp;
+                g++;
+            }
+        }
+    };
+    W w;
+    w.load(seq, ldseq, L, wfirst, lane);
+    uint32_t baseA[S], baseB[S];
+    float acc[S];
+    copy_stage(0, 0);
+    wait_vmem();
+    __syncthreads();
+    uint32_t buf = 0;
+    uint32_t pos = __builtin_amdgcn_readfirstlane(pos_list[0]);
+    for (uint32_t t0 = 0; t0 < nsteps; t0 += nst) {
+        if (t0 + nst < nsteps) copy_stage(t0 + nst, buf ^ 1);
+        const uint32_t t1 = t0 + nst < nsteps ? t0 + nst : nsteps;
+        uint32_t origin = j * 4 + buf * stageb;
+        for (uint32_t t = t0; t < t1; t++) {
+            const uint32_t pos_next =
+                (t + 1 < nsteps) ? __builtin_amdgcn_readfirstlane(pos_list[t + 1]) : 0u;
+            const uint32_t Pcur =
+                w.draws(t, step0, walker_base + wfirst + (j >> W::SH), lane, q, k0, k1);
+            w.bases(pos, lane, Pcur & 0xffu, q, origin, baseA, baseB);
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                if (k == 0 || (uint32_t)k < nchunk) {
+                    const char* cb = ldsb + k * SLOT;
+                    constexpr int G = (S < SWEEP_G) ? S : SWEEP_G;
+#pragma unroll
+                    for (int i = 0; i < S / G; i++) {
+                        float vA[G], vB[G];
+#pragma unroll
+                        for (int g = 0; g < G; g++) {
+                            const int s = i * G + g;
+                            uint32_t aA, aB;
+                            w.gather_addr(s, k, baseA[s], baseB[s], aA, aB);
+                            vA[g] = *reinterpret_cast<const float*>(cb + aA);
+                            vB[g] = *reinterpret_cast<const float*>(cb + aB);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int g = 0; g < G; g++) {
+                            const int s = i * G + g;
+                            if (k == 0) acc[s] = vB[g] - vA[g];
+                            else acc[s] += vB[g] - vA[g];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            w.accept(pos, lane, acc, Pcur, nbeta);
+            pos = pos_next;
+            origin += rowb;
+        }
+        wait_vmem();
+        __syncthreads();
+        buf ^= 1;
+    }
+    w.store(seq, ldseq, L, wfirst, lane);
+}
+
+// No staging: every lane reads the couplings it needs from memory (the rows
+// of a step are shared by all walkers, so they come from L2).  One wave per
+// work-group, no barrier, no LDS.  NC = nchunk, so that the loads of a step
+// are straight-line code and all in flight together.
+template <int NC, int S>
+__device__ __forceinline__ void sweep_direct(
+    const float* __restrict__ Ju, uint8_t* __restrict__ seq, const uint32_t* __restrict__ pos_list,
+    uint32_t ldseq, uint32_t L, uint32_t q, uint32_t chb, uint32_t nsteps, uint32_t k0, uint32_t k1,
+    uint64_t step0, uint32_t walker_base, float nbeta, uint32_t block) {
+    constexpr int KW = (NC + 3) / 4;
+    using W = Walkers<KW, S, false>;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t j = lane & 31;
+    const uint32_t wfirst = block * (2 * S) + (lane >> 5) * S;
+    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * NC * chb);
+    if (nsteps == 0) return;
+    W w;
+    w.load(seq, ldseq, L, wfirst, lane);
+    uint32_t baseA[S], baseB[S];
+    float acc[S];
+    uint32_t pos = __builtin_amdgcn_readfirstlane(pos_list[0]);
+    for (uint32_t t = 0; t < nsteps; t++) {
+        const uint32_t pos_next =
+            (t + 1 < nsteps) ? __builtin_amdgcn_readfirstlane(pos_list[t + 1]) : 0u;
+        const uint32_t Pcur =
+            w.draws(t, step0, walker_base + wfirst + (j >> W::SH), lane, q, k0, k1);
+        w.bases(pos, lane, Pcur & 0xffu, q, j * 4, baseA, baseB);
+        const uint32_t row = pos * NC * chb;
+        float vA[NC][S], vB[NC][S];
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                uint32_t aA, aB;
+                w.gather_addr(s, k, baseA[s], baseB[s], aA, aB);
+                vA[k][s] = __uint_as_float(
+                    __builtin_amdgcn_raw_buffer_load_b32(rJ, aA, row + k * chb, 0));
+                vB[k][s] = __uint_as_float(
+                    __builtin_amdgcn_raw_buffer_load_b32(rJ, aB, row + k * chb, 0));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                if (k == 0) acc[s] = vB[k][s] - vA[k][s];
+                else acc[s] += vB[k][s] - vA[k][s];
+            }
+        }
+        w.accept(pos, lane, acc, Pcur, nbeta);
+        pos = pos_next;
+    }
+    w.store(seq, ldseq, L, wfirst, lane);
+}
+
+template <int KW, int S, int NWAVES, int NPC>
+__global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_sweep_steps(
+    const float* __restrict__ Ju, uint8_t* __restrict__ seq, const uint32_t* __restrict__ pos_list,
+    uint32_t ldseq, uint32_t L, uint32_t q, uint32_t nchunk, uint32_t nsteps, uint32_t k0,
+    uint32_t k1, uint64_t step0, uint32_t walker_base, float nbeta, uint32_t nst) {
+    sweep_steps<KW, S, NWAVES, NPC>(Ju, seq, pos_list, ldseq, L, q, nchunk, nsteps, k0, k1, step0,
+                                    walker_base, nbeta, blockIdx.x, nst);
+}
+
+template <int NC, int S>
+__global__ __launch_bounds__(64) void k_sweep_direct(
+    const float* __restrict__ Ju, uint8_t* __restrict__ seq, const uint32_t* __restrict__ pos_list,
+    uint32_t ldseq, uint32_t L, uint32_t q, uint32_t chb, uint32_t nsteps, uint32_t k0, uint32_t k1,
+    uint64_t step0, uint32_t walker_base, float nbeta) {
+    sweep_direct<NC, S>(Ju, seq, pos_list, ldseq, L, q, chb, nsteps, k0, k1, step0, walker_base,
+                        nbeta, blockIdx.x);
+}
 
 template <int KW, int S, int NWAVES, int PF>
 __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(NWAVES / 4, NWAVES / 4))) void k_sweep(
@@ -548,6 +807,35 @@ __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(NWA
     uint32_t k1, uint64_t step0, uint32_t walker_base, float nbeta) {
     sweep_block<KW, S, NWAVES, PF>(Ju, seq, pos_list, ldseq, L, q, nchunk, nsteps, k0, k1, step0,
                                    walker_base, nbeta, blockIdx.x);
+}
+
+// A model's descriptor with every field wave-uniform (the kernel's own stores
+// to walker memory keep the compiler from proving it).
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
+    // (readfirstlane returns int: widen through uint32_t, or a low word
+    // with bit 31 set would sign-extend over the high word)
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+__device__ __forceinline__ BatchModel uniform_model(const BatchModel& m) {
+    auto u32 = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+    BatchModel r;
+    r.Ju = (const float*)uniform64((uint64_t)m.Ju);
+    r.seq = (uint8_t*)uniform64((uint64_t)m.seq);
+    r.pos = (const uint32_t*)uniform64((uint64_t)m.pos);
+    r.step = (const uint64_t*)uniform64((uint64_t)m.step);
+    r.ld = u32(m.ld);
+    r.L = u32(m.L);
+    r.q = u32(m.q);
+    r.nchunk = u32(m.nchunk);
+    r.nsteps = u32(m.nsteps);
+    r.k0 = u32(m.k0);
+    r.k1 = u32(m.k1);
+    r.walker_base = u32(m.walker_base);
+    r.nbeta = __uint_as_float(u32(__float_as_uint(m.nbeta)));
+    r.pad_ = 0;
+    return r;
 }
 
 // Persistent sweep over the tiles of one (KW, PF) class of a batch of
@@ -565,24 +853,37 @@ k_sweep_batch(const BatchModel* __restrict__ models, const BatchTile* __restrict
         const uint32_t t = __builtin_amdgcn_readfirstlane(s_tile);  // uniform: scalar loads below
         if (t >= ntiles) break;
         const BatchTile tl = tiles[t];
-        const BatchModel& m = models[tl.model];
-        // descriptor fields are uniform; say so (the kernel's own stores to
-        // walker memory keep the compiler from proving it)
-        auto u32 = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane(v); };
-        // (readfirstlane returns int: widen through uint32_t, or a low word
-        // with bit 31 set would sign-extend over the high word)
-        auto ptr = [](const void* p) {
-            const uint64_t v = (uint64_t)p;
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-            return (uint64_t)lo | ((uint64_t)hi << 32);
-        };
-        const uint64_t step0 = ptr((const void*)*m.step);
+        const BatchModel m = uniform_model(models[tl.model]);
+        const uint64_t step0 = uniform64(*m.step);
         sweep_block<KW, S, NWAVES, PF>(
-            (const float*)ptr(m.Ju), (uint8_t*)ptr(m.seq), (const uint32_t*)ptr(m.pos), u32(m.ld),
-            u32(m.L), u32(m.q), u32(m.nchunk), u32(m.nsteps), u32(m.k0), u32(m.k1), step0,
-            u32(m.walker_base), __uint_as_float(u32(__float_as_uint(m.nbeta))), u32(tl.block));
+            m.Ju, m.seq, m.pos, m.ld, m.L, m.q, m.nchunk, m.nsteps, m.k0, m.k1, step0,
+            m.walker_base, m.nbeta, (uint32_t)__builtin_amdgcn_readfirstlane((int)tl.block));
     }
+}
+
+// Unstaged sweep over the walkers of one class of a batch: `sub` waves of
+// 2*S walkers per tile.  Work-groups go to the eight XCDs in turn, so each XCD
+// takes a contiguous range of `per` waves: it sweeps few models, and its L2
+// holds their rows.
+template <int KW, int S>
+__global__ __launch_bounds__(64) void k_sweep_batch_direct(const BatchModel* __restrict__ models,
+                                                           const BatchTile* __restrict__ tiles,
+                                                           uint32_t sub, uint32_t waves,
+                                                           uint32_t per) {
+    const uint32_t v = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (v >= waves) return;
+    const uint32_t t = v / sub;
+    const BatchTile tl = tiles[t];
+    const BatchModel m = uniform_model(models[tl.model]);
+    const uint64_t step0 = uniform64(*m.step);
+    const uint32_t block = tl.block * sub + (v - t * sub);
+    const uint32_t chb = chunk_floats(m.q) * 4;
+#define MI3_NC(NC)                                                                              \
+    if (m.nchunk == NC)                                                                         \
+        sweep_direct<NC, S>(m.Ju, m.seq, m.pos, m.ld, m.L, m.q, chb, m.nsteps, m.k0, m.k1, step0, \
+                            m.walker_base, m.nbeta, block);
+    MI3_NC(4 * KW - 3) MI3_NC(4 * KW - 2) MI3_NC(4 * KW - 1) MI3_NC(4 * KW)
+#undef MI3_NC
 }
 
 // ---------------------------------------------------------------------------

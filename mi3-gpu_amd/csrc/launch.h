@@ -12,7 +12,8 @@ struct SweepArgs {
     uint32_t ld, nwalk, L, q, nchunk, nsteps, k0, k1, walker_base;
     uint64_t step0;
     float nbeta;
-    uint32_t wpb;  // walkers per work-group: 128, 256 or 512 (0 = default)
+    uint32_t wpb;  // walkers per work-group: 128, 256, or 512 / 0 (the library's choice)
+    uint32_t ncu;  // compute units of the device
 };
 
 struct EnergyArgs {
@@ -22,11 +23,8 @@ struct EnergyArgs {
     uint32_t ld, nseq, L, q, nchunk;
 };
 
-// Walkers per work-group of the sweep kernel: 128, 256 or 512 (a request of
-// 512 runs tiles of 256 for L > 384 and q <= 8); the walker count must be a
-// multiple of 512.
+// The walker count must be a multiple of 512.
 constexpr uint32_t SWEEP_WALKERS_PER_BLOCK = 512;
-constexpr uint32_t SWEEP_DEFAULT_WPB = 512;
 
 // Largest q / L the register-resident kernels are instantiated for.
 constexpr uint32_t MAX_Q = 25;
@@ -38,7 +36,7 @@ constexpr uint32_t POTTS_THREADS = 512;
 // float4 loads per thread to stage one chunk of q*q*32 floats; the chunked
 // coupling layout pads every chunk to POTTS_THREADS * pf_class(q) float4 so
 // that staging needs no bounds checks.
-inline uint32_t pf_class(uint32_t q) {
+__host__ __device__ inline uint32_t pf_class(uint32_t q) {
     uint32_t need = (q * q * 32 / 4 + POTTS_THREADS - 1) / POTTS_THREADS;
     if (need <= 1) return 1;
     if (need <= 4) return 4;
@@ -47,7 +45,7 @@ inline uint32_t pf_class(uint32_t q) {
 }
 
 // Floats per (padded) chunk.
-inline uint32_t chunk_floats(uint32_t q) { return pf_class(q) * POTTS_THREADS * 4; }
+__host__ __device__ inline uint32_t chunk_floats(uint32_t q) { return pf_class(q) * POTTS_THREADS * 4; }
 
 // The chunked couplings of an L-site model are addressed with 32-bit byte
 // offsets (buffer resources): true when they fit.
@@ -72,7 +70,27 @@ struct BatchTile {
     uint32_t model, block;
 };
 
+// Largest walker count that is swept without staging (sweep_direct): its
+// time grows with the walkers from the start, a staged tile's only once the
+// CUs are full.  The two meet near 32 walkers a CU for q > 8 (8192 walkers:
+// 6.7 against 7.0 us a step at L=232 q=21, 2.6 against 2.7 at L=93) and
+// near 24 for the cheaper rows of q <= 8 (L=93 q=4: 4096 walkers 0.56 against
+// 0.82, 16384 walkers 1.7 against 0.97).
+inline uint32_t direct_walkers(uint32_t q, uint32_t ncu) { return (q <= 8 ? 24 : 32) * ncu; }
+
+// LDS per chunk in the step-staged sweep, in KB (2 for q <= 4, 8 for q <= 8),
+// or 0 where a row of couplings does not fit 64 KB and the form does not
+// apply.
+inline uint32_t steps_slot_kb(uint32_t q, uint32_t nchunk) {
+    const uint32_t kb = q <= 4 ? 2 : 8;
+    return q <= 8 && nchunk * kb <= 64 ? kb : 0;
+}
+
 // Returns a hipError_t; grid/LDS sizing done inside.
+hipError_t launch_sweep_direct(const SweepArgs& a, hipStream_t st);
+hipError_t launch_sweep_steps(const SweepArgs& a, hipStream_t st);
+template <int KW>
+hipError_t launch_sweep_chunks(const SweepArgs& a, hipStream_t st);
 hipError_t launch_sweep(const SweepArgs& a, hipStream_t st);
 hipError_t launch_energies(const EnergyArgs& a, hipStream_t st);
 
@@ -90,8 +108,30 @@ hipError_t launch_sweep_batch(uint32_t kw, uint32_t pf, uint32_t wpb, const Batc
                               const BatchTile* tiles, uint32_t ntiles, uint32_t* counter,
                               uint32_t grid, hipStream_t st);
 
+template <int KW>
+hipError_t launch_sweep_batch_chunks(uint32_t pf, uint32_t wpb, const BatchModel* models,
+                                     const BatchTile* tiles, uint32_t ntiles, uint32_t* counter,
+                                     uint32_t grid, hipStream_t st);
+
+// The same without staging, for classes of few walkers (`nwalk` in all; q the
+// smallest alphabet of the class).
+hipError_t launch_sweep_batch_direct(uint32_t kw, uint32_t q, uint32_t wpb, uint32_t nwalk,
+                                     uint32_t ncu, const BatchModel* models,
+                                     const BatchTile* tiles, uint32_t ntiles, hipStream_t st);
+
 // Chunked symmetric coupling layout from packed couplings (k_unpack_chunked).
 hipError_t launch_unpack_chunked(const float* J, float* out, uint32_t L, uint32_t q,
                                  uint32_t nchunk, hipStream_t st);
+
+#define MI3_DECL_KW(KW)                                                                       \
+    template <>                                                                               \
+    hipError_t launch_sweep_chunks<KW>(const SweepArgs& a, hipStream_t st);                    \
+    template <>                                                                               \
+    hipError_t launch_sweep_batch_chunks<KW>(uint32_t pf, uint32_t wpb, const BatchModel* models, \
+                                             const BatchTile* tiles, uint32_t ntiles,         \
+                                             uint32_t* counter, uint32_t grid, hipStream_t st);
+MI3_DECL_KW(1) MI3_DECL_KW(2) MI3_DECL_KW(3) MI3_DECL_KW(4)
+MI3_DECL_KW(5) MI3_DECL_KW(6) MI3_DECL_KW(7) MI3_DECL_KW(8)
+#undef MI3_DECL_KW
 
 }  // namespace mi3

@@ -1,4 +1,5 @@
-// Instantiation and launch of the register-resident sweep / energy kernels.
+// Launch rule of the sweep; instantiation and launch of the energy kernels and
+// of the staging probe.
 #include "k_potts.hip"
 #include "launch.h"
 
@@ -8,10 +9,6 @@ namespace {
 constexpr int NWAVES = 8;
 constexpr int NT = 64 * NWAVES;
 
-// Launch shapes (walker slots per half-wave S, waves NW): W = 2*S*NW walkers
-// per work-group.  16 waves of at most 128 registers (4 waves per SIMD) hide
-// the gathers' latency better than 8 waves of 256, wherever the state fits:
-// measured on MI355X at L=120/232/300/450, q=21 and q=4.
 // sequence slots per half-wave of the energy kernel: every staged coupling
 // chunk is read once per sequence, so more sequences per work-group cut the
 // L2 -> LDS traffic per sequence.  16 slots in 16 waves (512 sequences per
@@ -35,20 +32,6 @@ hipError_t set_lds(F kernel, size_t bytes) {
     static_assert(sizeof(F) > 0, "");
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
-template <int KW, int PF, int S, int NW = NWAVES>
-hipError_t sweep_kws(const SweepArgs& a, hipStream_t st) {
-    constexpr uint32_t W = 2 * S * NW;
-    auto kern = k_sweep<KW, S, NW, PF>;
-    size_t lds = 2ull * chunk_floats(a.q) * sizeof(float);
-    hipError_t e = set_lds(kern, lds);
-    if (e != hipSuccess) return e;
-    if (a.nwalk % W) return hipErrorInvalidValue;
-    dim3 grid(a.nwalk / W);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, st, a.Ju, a.seq, a.pos, a.ld, a.L, a.q,
-                       a.nchunk, a.nsteps, a.k0, a.k1, a.step0, a.walker_base, a.nbeta);
-    return hipGetLastError();
 }
 
 template <int KW, int PF>
@@ -90,80 +73,50 @@ hipError_t dispatch(const A& a, hipStream_t st, uint32_t nchunk, uint32_t q) {
 }
 
 template <int KW, int PF>
-struct SweepDisp {
-    static hipError_t run(const SweepArgs& a, hipStream_t st) {
-        uint32_t w = a.wpb ? a.wpb : SWEEP_DEFAULT_WPB;
-        if constexpr (KW >= 5) {
-            // five to eight state words: 8 slots at most fit in 128 registers
-            if (w <= 128) return sweep_kws<KW, PF, 4, 16>(a, st);
-            return sweep_kws<KW, PF, 8, 16>(a, st);
-        } else {
-            if (w <= 128) return sweep_kws<KW, PF, 8, 8>(a, st);
-            if (w <= 256) return sweep_kws<KW, PF, 8, 16>(a, st);
-            // four state words do not fit 16 slots in 128 registers; the
-            // spills still pay for q > 8, not for the small chunks of q <= 8
-            if constexpr (KW == 4 && PF == 1)
-                return sweep_kws<KW, PF, 8, 16>(a, st);
-            else
-                return sweep_kws<KW, PF, 16, 16>(a, st);
-        }
-    }
-};
-template <int KW, int PF>
 struct EnergyDisp {
     static hipError_t run(const EnergyArgs& a, hipStream_t st) { return energies_kw<KW, PF>(a, st); }
 };
 }  // namespace
 
+// Form of the sweep.  A tile asked for by size (128 or 256 walkers) runs
+// chunk-staged; the default goes by what fills the card:
+//   few walkers per CU: no staging at all (direct_walkers);
+//   q <= 8 with rows of up to 64 KB: several steps' rows staged at once;
+//   otherwise chunk by chunk.
 hipError_t launch_sweep(const SweepArgs& a, hipStream_t st) {
-    if (a.nwalk % SWEEP_WALKERS_PER_BLOCK || a.q > MAX_Q || a.L > MAX_L || a.L < 2)
+    if (a.nwalk % SWEEP_WALKERS_PER_BLOCK || a.q > MAX_Q || a.L > MAX_L || a.L < 2 || a.ncu == 0)
         return hipErrorInvalidValue;
-    return dispatch<SweepDisp>(a, st, a.nchunk, a.q);
-}
-
-namespace {
-template <int KW, int PF, int S, int NW = NWAVES>
-hipError_t batch_kws(const BatchModel* models, const BatchTile* tiles, uint32_t ntiles,
-                     uint32_t* counter, uint32_t grid, hipStream_t st) {
-    auto kern = k_sweep_batch<KW, S, NW, PF>;
-    size_t lds = 2ull * PF * POTTS_THREADS * 4 * sizeof(float);  // two padded chunks
-    hipError_t e = set_lds(kern, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, st, models, tiles, ntiles, counter);
-    return hipGetLastError();
-}
-
-template <int KW, int PF>
-hipError_t batch_kw(uint32_t wpb, const BatchModel* models, const BatchTile* tiles,
-                    uint32_t ntiles, uint32_t* counter, uint32_t grid, hipStream_t st) {
-    if constexpr (KW >= 5) {
-        if (wpb == 128) return batch_kws<KW, PF, 4, 16>(models, tiles, ntiles, counter, grid, st);
-        if (wpb == 256) return batch_kws<KW, PF, 8, 16>(models, tiles, ntiles, counter, grid, st);
-        return hipErrorInvalidValue;
-    } else {
-        if (wpb == 128) return batch_kws<KW, PF, 8, 8>(models, tiles, ntiles, counter, grid, st);
-        if (wpb == 256) return batch_kws<KW, PF, 8, 16>(models, tiles, ntiles, counter, grid, st);
-        if (wpb == 512) return batch_kws<KW, PF, 16, 16>(models, tiles, ntiles, counter, grid, st);
-        return hipErrorInvalidValue;
+    if (a.wpb == 0 || a.wpb >= 512) {
+        if (a.nwalk <= direct_walkers(a.q, a.ncu)) return launch_sweep_direct(a, st);
+        if (steps_slot_kb(a.q, a.nchunk)) return launch_sweep_steps(a, st);
     }
+    switch (state_words(a.L)) {
+        case 1: return launch_sweep_chunks<1>(a, st);
+        case 2: return launch_sweep_chunks<2>(a, st);
+        case 3: return launch_sweep_chunks<3>(a, st);
+        case 4: return launch_sweep_chunks<4>(a, st);
+        case 5: return launch_sweep_chunks<5>(a, st);
+        case 6: return launch_sweep_chunks<6>(a, st);
+        case 7: return launch_sweep_chunks<7>(a, st);
+        case 8: return launch_sweep_chunks<8>(a, st);
+    }
+    return hipErrorInvalidValue;
 }
-}  // namespace
 
 hipError_t launch_sweep_batch(uint32_t kw, uint32_t pf, uint32_t wpb, const BatchModel* models,
                               const BatchTile* tiles, uint32_t ntiles, uint32_t* counter,
                               uint32_t grid, hipStream_t st) {
     if (grid == 0 || ntiles == 0) return hipSuccess;
-#define MI3_BCASE(KW_, PF_) \
-    if (kw == KW_ && pf == PF_) return batch_kw<KW_, PF_>(wpb, models, tiles, ntiles, counter, grid, st);
-    MI3_BCASE(1, 1) MI3_BCASE(1, 4) MI3_BCASE(1, 7) MI3_BCASE(1, 10)
-    MI3_BCASE(2, 1) MI3_BCASE(2, 4) MI3_BCASE(2, 7) MI3_BCASE(2, 10)
-    MI3_BCASE(3, 1) MI3_BCASE(3, 4) MI3_BCASE(3, 7) MI3_BCASE(3, 10)
-    MI3_BCASE(4, 1) MI3_BCASE(4, 4) MI3_BCASE(4, 7) MI3_BCASE(4, 10)
-    MI3_BCASE(5, 1) MI3_BCASE(5, 4) MI3_BCASE(5, 7) MI3_BCASE(5, 10)
-    MI3_BCASE(6, 1) MI3_BCASE(6, 4) MI3_BCASE(6, 7) MI3_BCASE(6, 10)
-    MI3_BCASE(7, 1) MI3_BCASE(7, 4) MI3_BCASE(7, 7) MI3_BCASE(7, 10)
-    MI3_BCASE(8, 1) MI3_BCASE(8, 4) MI3_BCASE(8, 7) MI3_BCASE(8, 10)
-#undef MI3_BCASE
+    switch (kw) {
+        case 1: return launch_sweep_batch_chunks<1>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 2: return launch_sweep_batch_chunks<2>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 3: return launch_sweep_batch_chunks<3>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 4: return launch_sweep_batch_chunks<4>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 5: return launch_sweep_batch_chunks<5>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 6: return launch_sweep_batch_chunks<6>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 7: return launch_sweep_batch_chunks<7>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+        case 8: return launch_sweep_batch_chunks<8>(pf, wpb, models, tiles, ntiles, counter, grid, st);
+    }
     return hipErrorInvalidValue;
 }
 

@@ -86,7 +86,7 @@ struct mi3_ctx {
     uint32_t indep_calls = 0;
     uint32_t* pos = nullptr;
     size_t pos_cap = 0;
-    uint32_t wpb = 0;  // sweep walkers per work-group (0 = default)
+    uint32_t wpb = 0;  // sweep walkers per work-group (0, 512 = the library's choice)
     uint32_t ncu = 256;  // compute units of the device
     // derived device data
     std::map<std::string, Chunked> chunked;  // chunked layouts keyed by source buffer
@@ -693,6 +693,7 @@ int mi3_run_mcmc(mi3_ctx* c, float beta) {
     a.step0 = c->step;
     a.nbeta = -beta;
     a.wpb = c->wpb;
+    a.ncu = c->ncu;
     {
         Scope s(c, "mcmc", (size_t)c->N * c->nsteps * (c->L + 1));
         HIPCHK(c, launch_sweep(a, c->stream));
