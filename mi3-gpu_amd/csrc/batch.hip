@@ -225,9 +225,15 @@ int enqueue_round(mi3_batch* b, std::vector<hipEvent_t>& events) {
     BCHK(b, hipEventRecord(fork, b->stream));
     uint32_t ci = 0;
     int rc = MI3_OK;
+    // unstaged classes run one after another (on the first one's stream): side
+    // by side their waves drift apart, the rows they share leave the L2s, and
+    // each takes several times as long (L=301 q=4 and L=400 q=21, 1024 walkers,
+    // 4 sweeps: 1.0 and 3.2 ms alone, 9.2 ms together)
+    hipStream_t direct = nullptr;
     for (auto& kv : b->classes) {
         ClassRun& cr = kv.second;
-        hipStream_t s = cr.side;
+        if (cr.direct && !direct) direct = cr.side;
+        hipStream_t s = cr.direct ? direct : cr.side;
         if (hipStreamWaitEvent(s, fork, 0) != hipSuccess) { rc = bfail(b, MI3_EHIP, "fork"); break; }
         hipError_t e = sweep_class(b, kv.first, cr, b->counters + ci, s);
         if (e != hipSuccess) {

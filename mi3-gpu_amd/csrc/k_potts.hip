@@ -300,6 +300,16 @@ __device__ __forceinline__ uint32_t row_bcast(uint32_t v, int e) {
 }
 #undef MI3_RB_CASE
 
+// Byte permute as asm, for stores to the state word that holds a site: the
+// compiler merges branches on that word, if they hold plain instructions, into
+// one access with a variable index, which moves the state to scratch memory
+// (L=301 q=4 unstaged: 11 us a step against 0.8).
+__device__ __forceinline__ uint32_t perm_apart(uint32_t hi, uint32_t lo, uint32_t sel) {
+    uint32_t r;
+    asm("v_perm_b32 %0, %1, %2, %3" : "=v"(r) : "v"(hi), "v"(lo), "v"(sel));
+    return r;
+}
+
 // The walkers of a wave and what a step does with them around its gathers.
 // QB: q <= 16, so that a residue times q fits a byte.
 template <int KW, int S, bool QB>
@@ -312,16 +322,18 @@ struct Walkers {
     static constexpr int NP = (S + 3) / 4;   // residues of a site, four slots to a word
 
     uint32_t st[S][KW];       // residues of sites j + 32k, four to a word
-    uint32_t apk[NP];         // this step's current residues, byte s % 4 of word s / 4
+    // this step's current residues, byte s % 4 of word s / 4, kept for its end;
+    // fetched again there where the state leaves no registers for them
+    static constexpr bool KEEP = KW * S < 64;
+    uint32_t kept[KEEP ? NP : 1];
     uint32_t Xe, Xo;          // this lane's draws (steps 2h, 2h+1 of its own pair)
-    uint32_t Pe, Po;          // draws of the current pair of steps
     int remap;                // bpermute address: row lane e <- the lane deciding slot e
 
     __device__ __forceinline__ void load(const uint8_t* seq, uint32_t ldseq, uint32_t L,
                                          uint32_t wfirst, uint32_t lane) {
         const uint32_t j = lane & 31;
         remap = (int)((((lane & 15) << SH) & 31) | (lane & 32)) * 4;
-        Xe = Xo = Pe = Po = 0;
+        Xe = Xo = 0;
 #pragma unroll
         for (int s = 0; s < S; s++) {
 #pragma unroll
@@ -355,80 +367,79 @@ struct Walkers {
         }
     }
 
-    // Draws of step t of the launch (step0 even).  The lanes deciding one
-    // slot share the work: lane i of R draws the steps 2(h + i), 2(h + i) + 1
-    // every R pairs of steps, and a quad permutation hands each pair out.
+    // Draw of step t of the launch (step0 even).  The lanes deciding one slot
+    // share the work: lane i of R draws the steps 2(h + i), 2(h + i) + 1 every
+    // R pairs of steps, and a quad permutation hands each out.
     __device__ __forceinline__ uint32_t draws(uint32_t t, uint64_t step0, uint32_t walker,
                                               uint32_t lane, uint32_t q, uint32_t k0,
                                               uint32_t k1) {
-        if ((t & 1) == 0) {
-            const uint32_t i = (t >> 1) & (R - 1);
-            if (i == 0) {
-                const uint64_t h = ((step0 + t) >> 1) + (lane & (R - 1));
-                uint4 r = philox4x32_10(make_uint4((uint32_t)h, (uint32_t)(h >> 32), walker,
-                                                   TAG_WALK), k0, k1);
-                Xe = ((r.y >> 8) << 8) | mulhi_range(r.x, q);
-                Xo = ((r.w >> 8) << 8) | mulhi_range(r.z, q);
-            }
-            auto hand = [&](auto ctrl) {
-                Pe = (uint32_t)__builtin_amdgcn_mov_dpp((int)Xe, decltype(ctrl)::value, 0xF, 0xF,
-                                                        false);
-                Po = (uint32_t)__builtin_amdgcn_mov_dpp((int)Xo, decltype(ctrl)::value, 0xF, 0xF,
-                                                        false);
-            };
-            if constexpr (R == 2) {
-                if (i == 0) hand(std::integral_constant<int, 0xA0>{});   // quad 0,0,2,2
-                else hand(std::integral_constant<int, 0xF5>{});          // quad 1,1,3,3
-            } else {
-                if (i == 0) hand(std::integral_constant<int, 0x00>{});
-                else if (i == 1) hand(std::integral_constant<int, 0x55>{});
-                else if (i == 2) hand(std::integral_constant<int, 0xAA>{});
-                else hand(std::integral_constant<int, 0xFF>{});
-            }
-            return Pe;
+        const uint32_t i = (t >> 1) & (R - 1);
+        if ((t & 1) == 0 && i == 0) {
+            const uint64_t h = ((step0 + t) >> 1) + (lane & (R - 1));
+            uint4 r = philox4x32_10(make_uint4((uint32_t)h, (uint32_t)(h >> 32), walker, TAG_WALK),
+                                    k0, k1);
+            Xe = ((r.y >> 8) << 8) | mulhi_range(r.x, q);
+            Xo = ((r.w >> 8) << 8) | mulhi_range(r.z, q);
         }
-        return Po;
+        const int x = (int)((t & 1) ? Xo : Xe);
+        int p;
+        if constexpr (R == 2) {
+            if (i == 0) p = __builtin_amdgcn_mov_dpp(x, 0xA0, 0xF, 0xF, false);    // quad 0,0,2,2
+            else p = __builtin_amdgcn_mov_dpp(x, 0xF5, 0xF, 0xF, false);           // quad 1,1,3,3
+        } else {
+            if (i == 0) p = __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, false);
+            else if (i == 1) p = __builtin_amdgcn_mov_dpp(x, 0x55, 0xF, 0xF, false);
+            else if (i == 2) p = __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, false);
+            else p = __builtin_amdgcn_mov_dpp(x, 0xFF, 0xF, 0xF, false);
+        }
+        return (uint32_t)p;
+    }
+
+    // Current residues of every slot at site pos, in every lane: four slots to
+    // a word, so one ds_bpermute from the owner lane serves four.
+    __device__ __forceinline__ void residues(uint32_t pos, uint32_t lane,
+                                             uint32_t (&apk)[NP]) const {
+        const uint32_t kp = pos >> 5, owner = pos & 31;
+        const uint32_t wd = kp >> 2, e0 = kp & 3;
+        const int own_addr = (int)((owner + (lane & 32)) * 4);
+#pragma unroll
+        for (int g = 0; g < NP; g++) {
+            uint32_t w[S < 4 ? S : 4];
+#pragma unroll
+            for (int e = 0; e < (S < 4 ? S : 4); e++) w[e] = select_word<KW>(st[4 * g + e], wd);
+            uint32_t p;
+            if constexpr (S == 1)
+                p = __builtin_amdgcn_ubfe(w[0], e0 * 8, 8);
+            else
+                p = __builtin_amdgcn_perm(w[1], w[0], 0x0c0c0400u + e0 * 0x00000101u);
+            if constexpr (S >= 4)
+                p |= __builtin_amdgcn_perm(w[3], w[2], 0x04000c0cu + e0 * 0x01010000u);
+            apk[g] = p;
+        }
+#pragma unroll
+        for (int g = 0; g < NP; g++)
+            apk[g] = (uint32_t)__builtin_amdgcn_ds_bpermute(own_addr, (int)apk[g]);
     }
 
     // Row addresses of every slot: baseA, baseB = (a, b) * q * 128 + origin
     // (origin: this lane's column, plus where the couplings of the site
-    // start).  The current residues are packed four slots to a word, so one
-    // ds_bpermute from the owner lane serves four slots; the proposals move
-    // to row lane s once, and each slot's is broadcast by DPP inside the add.
-    // (A ds_bpermute takes the LDS 2.5 times as long as a gather; before, every
-    // slot took one, and two swizzles.)
+    // start).  The proposals move to row lane s once, and each slot's is
+    // broadcast by DPP inside the add.  (A ds_bpermute takes the LDS 2.5 times
+    // as long as a gather; before, every slot took one, and two swizzles.)
     __device__ __forceinline__ void bases(uint32_t pos, uint32_t lane, uint32_t bmine, uint32_t q,
                                           uint32_t origin, uint32_t (&baseA)[S],
                                           uint32_t (&baseB)[S]) {
-        const uint32_t kp = pos >> 5, owner = pos & 31;
-        const uint32_t wd = kp >> 2, e0 = kp & 3;
-        const int own_addr = (int)((owner + (lane & 32)) * 4);
         // (opaque, so that the compiler does not turn the adds of disjoint bit
         // ranges below into ors, which do not fuse with the products)
         uint32_t org = origin;
         asm("" : "+v"(org));
         const uint32_t bl = (uint32_t)__builtin_amdgcn_ds_bpermute(remap, (int)bmine);
+        uint32_t apk[NP];
+        residues(pos, lane, apk);
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int i = 0; i < KW; i++) {
-            if (KW == 1 || wd == (uint32_t)i) {
-#pragma unroll
-                for (int g = 0; g < NP; g++) {
-                    uint32_t p;
-                    if constexpr (S == 1)
-                        p = __builtin_amdgcn_ubfe(st[0][i], e0 * 8, 8);
-                    else
-                        p = __builtin_amdgcn_perm(st[4 * g + 1][i], st[4 * g][i],
-                                                  0x0c0c0400u + e0 * 0x00000101u);
-                    if constexpr (S >= 4)
-                        p |= __builtin_amdgcn_perm(st[4 * g + 3][i], st[4 * g + 2][i],
-                                                   0x04000c0cu + e0 * 0x01010000u);
-                    apk[g] = p;
-                }
-            }
+            for (int g = 0; g < NP; g++) kept[g] = apk[g];
         }
-#pragma unroll
-        for (int g = 0; g < NP; g++)
-            apk[g] = (uint32_t)__builtin_amdgcn_ds_bpermute(own_addr, (int)apk[g]);
         const uint32_t brow = __umul24(bl, q * (CH * 4));
 #pragma unroll
         for (int s = 0; s < S; s++) baseB[s] = row_bcast(brow, s) + org;
@@ -471,10 +482,16 @@ struct Walkers {
         const uint32_t bp = __builtin_amdgcn_perm(y2, z, 0x05040100u);
         const uint32_t mp = __builtin_amdgcn_perm(y2, z, 0x07060302u);
         uint32_t npk[NP];
+        if constexpr (KEEP) {
+#pragma unroll
+            for (int g = 0; g < NP; g++) npk[g] = kept[g];
+        } else {
+            residues(pos, lane, npk);
+        }
 #pragma unroll
         for (int g = 0; g < NP; g++) {
             const uint32_t m = row_bcast(mp, 4 * g);
-            npk[g] = (row_bcast(bp, 4 * g) & m) | (apk[g] & ~m);
+            npk[g] = (row_bcast(bp, 4 * g) & m) | (npk[g] & ~m);
         }
         // owner lanes put byte e of the new residues at pos's byte; the
         // others keep their word
@@ -489,7 +506,7 @@ struct Walkers {
             if (KW == 1 || wd == (uint32_t)i) {
 #pragma unroll
                 for (int s = 0; s < S; s++)
-                    st[s][i] = __builtin_amdgcn_perm(st[s][i], npk[s / 4], sel[s & 3]);
+                    st[s][i] = perm_apart(st[s][i], npk[s / 4], sel[s & 3]);
             }
         }
     }
@@ -543,12 +560,14 @@ __device__ __forceinline__ void sweep_block(
     __syncthreads();
     const uint32_t j4 = j * 4;
 
-    // one step whose chunk 0 is in buffer B0: chunk k is in buffer
-    // (B0 + k) % 2, so that the buffer is a constant offset of each read and
-    // an address is one instruction per gather (the byte dot product of
-    // byte_x128_add)
-    auto step = [&](auto b0c, uint32_t t) __attribute__((always_inline)) {
-        constexpr uint32_t B0 = decltype(b0c)::value;
+    // one step whose chunk 0 is in buffer b0: chunk k is in buffer (b0 + k) % 2.
+    // For up to two state words the step is compiled for either b0, so that
+    // the buffer is a constant offset of each read and an address one plain
+    // add (half the time of a three-operand one); two copies of the longer
+    // steps spill registers.
+    constexpr bool TWICE = KW <= 2;
+    auto step = [&](auto b0c, uint32_t b0v, uint32_t t) __attribute__((always_inline)) {
+        const uint32_t b0 = TWICE ? decltype(b0c)::value : b0v;
         const uint32_t pos_after =
             (t + 2 < nsteps) ? __builtin_amdgcn_readfirstlane(pos_list[t + 2]) : 0u;
         const uint32_t Pcur =
@@ -561,7 +580,7 @@ __device__ __forceinline__ void sweep_block(
             if (k == 0 || (uint32_t)k < nchunk) {
                 const bool last_chunk = (uint32_t)k + 1 == nchunk;
                 const bool has_next = !last_chunk || (t + 1 < nsteps);
-                const uint32_t buf = (B0 + k) & 1;
+                const uint32_t buf = (b0 + k) & 1;
                 if (has_next) {
                     uint32_t npos = last_chunk ? pos_next : pos;
                     uint32_t nc = last_chunk ? 0u : (uint32_t)k + 1;
@@ -614,8 +633,8 @@ __device__ __forceinline__ void sweep_block(
     uint32_t b0 = 0;
     const uint32_t flip = nchunk & 1;
     for (uint32_t t = 0; t < nsteps; t++) {
-        if (b0) step(std::integral_constant<uint32_t, 1>{}, t);
-        else step(std::integral_constant<uint32_t, 0>{}, t);
+        if (TWICE && b0) step(std::integral_constant<uint32_t, 1>{}, b0, t);
+        else step(std::integral_constant<uint32_t, 0>{}, b0, t);
         b0 ^= flip;
     }
     w.store(seq, ldseq, L, wfirst, lane);
