@@ -21,101 +21,156 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // ---------------------------------------------------------------------------
 // C = alpha * op(A) op(B) + beta * C + bias[col], optionally relu; fp32 C
 // and/or bf16 Cb.  op(A) is M x K (A row-major M x K, or K x M if TA),
-// op(B) is K x N (B row-major K x N, or N x K if TB).  Work-group tile
-// 128 x 128 (4 waves of 64 x 64 = 2 x 2 v_mfma_f32_32x32x16_bf16), K step
-// 32 staged through LDS as [row][k] for A and [col][k] for B.  Requires
-// M, N, K, lda, ldb multiples of 8 and 16-byte aligned A, B (host-checked).
-constexpr int GT = 128, GK = 32, GKP = GK + 8;   // tile, k step, padded LDS row
+// op(B) is K x N (B row-major K x N, or N x K if TB).  Requires M, N, K, lda,
+// ldb multiples of 8 and 16-byte aligned A, B (host-checked).
+//
+// Work-group tile BM x BN, 4 waves (2 x 2), each a (BM/2) x (BN/2) block of
+// v_mfma_f32_32x32x16_bf16 tiles; K in steps of 64, both operands in LDS as
+// [row or column][k], double-buffered, the next step's global loads in flight
+// during this step's products, one barrier a step.  An operand whose memory is
+// k-major is transposed on the way: a thread loads 4 (or, in the small tile, 2)
+// k-rows of 8 columns and interleaves them in registers (byte permutes), so LDS
+// takes 8- or 4-byte stores, not one 2-byte store per element (4872 x 512 x 4096, A k-major: 560 us
+// before).  LDS rows are 128 bytes; the 16-byte pieces of row r are permuted
+// by r ^ (r >> 3), which spreads both the stores and the reads over the banks.
+// Products accumulate in ascending k, 16 at a time, whatever the tile.
+constexpr int GK = 64;   // k step
 
-template <bool TA, bool TB>
+template <int ROWS>
+struct GemmStage {
+    static constexpr int CHUNKS = ROWS * GK / 8 / 256;   // 16-byte loads per thread
+    uint4 v[CHUNKS];
+    // LDS byte address of piece kc (8 k) of row r
+    __device__ static __forceinline__ uint32_t at(int r, int kc) {
+        return (uint32_t)(r * (GK * 2) + ((kc ^ ((r ^ (r >> 3)) & 7)) << 4));
+    }
+    // T: the operand's memory is k-major (K rows of `rows`), else row-major
+    template <bool T>
+    __device__ __forceinline__ void load(const bf16* __restrict__ X, int ld, int r0, int rows,
+                                         int k0, int K, int tid) {
+#pragma unroll
+        for (int c = 0; c < CHUNKS; c++) {
+            uint4 x = make_uint4(0, 0, 0, 0);
+            if (!T) {
+                const int i = tid + 256 * c, r = r0 + (i >> 3), k = k0 + (i & 7) * 8;
+                if (r < rows && k < K)
+                    x = *reinterpret_cast<const uint4*>(X + (size_t)r * ld + k);
+            } else {
+                // rows 8*rb .. 8*rb + 7 of CHUNKS neighbouring k
+                const int r = r0 + 8 * (tid % (ROWS / 8));
+                const int k = k0 + CHUNKS * (tid / (ROWS / 8)) + c;
+                if (r < rows && k < K)
+                    x = *reinterpret_cast<const uint4*>(X + (size_t)k * ld + r);
+            }
+            v[c] = x;
+        }
+    }
+    template <bool T>
+    __device__ __forceinline__ void store(char* lds, int tid) const {
+        if (!T) {
+#pragma unroll
+            for (int c = 0; c < CHUNKS; c++) {
+                const int i = tid + 256 * c;
+                *reinterpret_cast<uint4*>(lds + at(i >> 3, i & 7)) = v[c];
+            }
+        } else {
+            static_assert(CHUNKS == 4 || CHUNKS == 2, "k-rows of a thread");
+            const int rb = tid % (ROWS / 8), kq = tid / (ROWS / 8);
+            const uint32_t* q0 = reinterpret_cast<const uint32_t*>(v);
+#pragma unroll
+            for (int p = 0; p < 4; p++) {   // rows 8*rb + 2p and 2p + 1
+                const int r = 8 * rb + 2 * p;
+                const uint32_t a0 = q0[p], a1 = q0[4 + p];
+                const uint32_t lo = __builtin_amdgcn_perm(a1, a0, 0x05040100u);
+                const uint32_t hi = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
+                if constexpr (CHUNKS == 4) {
+                    const uint32_t a2 = q0[8 + p], a3 = q0[12 + p];
+                    *reinterpret_cast<uint2*>(lds + at(r, kq >> 1) + (kq & 1) * 8) =
+                        make_uint2(lo, __builtin_amdgcn_perm(a3, a2, 0x05040100u));
+                    *reinterpret_cast<uint2*>(lds + at(r + 1, kq >> 1) + (kq & 1) * 8) =
+                        make_uint2(hi, __builtin_amdgcn_perm(a3, a2, 0x07060302u));
+                } else {
+                    *reinterpret_cast<uint32_t*>(lds + at(r, kq >> 2) + (kq & 3) * 4) = lo;
+                    *reinterpret_cast<uint32_t*>(lds + at(r + 1, kq >> 2) + (kq & 3) * 4) = hi;
+                }
+            }
+        }
+    }
+};
+
+template <bool TA, bool TB, int BM, int BN>
 __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, float alpha,
                                                    const bf16* __restrict__ A, int lda,
                                                    const bf16* __restrict__ B, int ldb,
                                                    float beta, float* __restrict__ C, int ldc,
                                                    bf16* __restrict__ Cb, int ldcb,
                                                    const float* __restrict__ bias, int relu) {
-    __shared__ __attribute__((aligned(16))) bf16 As[GT][GKP];
-    __shared__ __attribute__((aligned(16))) bf16 Bs[GT][GKP];
+    constexpr int MT = BM / 64, NT = BN / 64;   // 32x32 tiles of a wave
+    __shared__ __attribute__((aligned(16))) char As[2][BM * GK * 2];
+    __shared__ __attribute__((aligned(16))) char Bs[2][BN * GK * 2];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
     const int lr = lane & 31, lg = lane >> 5;
-    f32x16 acc[2][2];
+    f32x16 acc[MT][NT];
 #pragma unroll
-    for (int x = 0; x < 2; x++)
+    for (int x = 0; x < MT; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++)
+        for (int y = 0; y < NT; y++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[x][y][e] = 0.f;
-    const uint4 zero = make_uint4(0, 0, 0, 0);
 
+    GemmStage<BM> a;
+    GemmStage<BN> b;
+    a.template load<TA>(A, lda, m0, M, 0, K, tid);
+    b.template load<!TB>(B, ldb, n0, N, 0, K, tid);
+    a.template store<TA>(As[0], tid);
+    b.template store<!TB>(Bs[0], tid);
+    __syncthreads();
+    int buf = 0;
     for (int k0 = 0; k0 < K; k0 += GK) {
-        // stage A' (GT rows x GK k) and B' (GK k x GT cols): 512 chunks of
-        // 8 bf16 each, two per thread
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const int c = tid + 256 * r;
-            if (!TA) {
-                const int m = c >> 2, kk = (c & 3) * 8;
-                uint4 v = zero;
-                if (m0 + m < M && k0 + kk < K)
-                    v = *reinterpret_cast<const uint4*>(A + (size_t)(m0 + m) * lda + k0 + kk);
-                *reinterpret_cast<uint4*>(&As[m][kk]) = v;
-            } else {
-                const int k = c >> 4, mm = (c & 15) * 8;
-                uint4 v = zero;
-                if (k0 + k < K && m0 + mm < M)
-                    v = *reinterpret_cast<const uint4*>(A + (size_t)(k0 + k) * lda + m0 + mm);
-                const bf16* e8 = reinterpret_cast<const bf16*>(&v);
-#pragma unroll
-                for (int e = 0; e < 8; e++) As[mm + e][k] = e8[e];
-            }
-            if (TB) {
-                const int n = c >> 2, kk = (c & 3) * 8;
-                uint4 v = zero;
-                if (n0 + n < N && k0 + kk < K)
-                    v = *reinterpret_cast<const uint4*>(B + (size_t)(n0 + n) * ldb + k0 + kk);
-                *reinterpret_cast<uint4*>(&Bs[n][kk]) = v;
-            } else {
-                const int k = c >> 4, nn = (c & 15) * 8;
-                uint4 v = zero;
-                if (k0 + k < K && n0 + nn < N)
-                    v = *reinterpret_cast<const uint4*>(B + (size_t)(k0 + k) * ldb + n0 + nn);
-                const bf16* e8 = reinterpret_cast<const bf16*>(&v);
-#pragma unroll
-                for (int e = 0; e < 8; e++) Bs[nn + e][k] = e8[e];
-            }
+        const bool more = k0 + GK < K;
+        if (more) {
+            a.template load<TA>(A, lda, m0, M, k0 + GK, K, tid);
+            b.template load<!TB>(B, ldb, n0, N, k0 + GK, K, tid);
         }
-        __syncthreads();
 #pragma unroll
         for (int kk = 0; kk < GK; kk += 16) {
-            bf16x8 a[2], b[2];
+            bf16x8 fa[MT], fb[NT];
 #pragma unroll
-            for (int x = 0; x < 2; x++)
-                a[x] = *reinterpret_cast<const bf16x8*>(&As[64 * wm + 32 * x + lr][kk + 8 * lg]);
+            for (int x = 0; x < MT; x++)
+                fa[x] = *reinterpret_cast<const bf16x8*>(
+                    As[buf] + GemmStage<BM>::at(wm + 32 * x + lr, (kk >> 3) + lg));
 #pragma unroll
-            for (int y = 0; y < 2; y++)
-                b[y] = *reinterpret_cast<const bf16x8*>(&Bs[64 * wn + 32 * y + lr][kk + 8 * lg]);
+            for (int y = 0; y < NT; y++)
+                fb[y] = *reinterpret_cast<const bf16x8*>(
+                    Bs[buf] + GemmStage<BN>::at(wn + 32 * y + lr, (kk >> 3) + lg));
 #pragma unroll
-            for (int x = 0; x < 2; x++)
+            for (int x = 0; x < MT; x++)
 #pragma unroll
-                for (int y = 0; y < 2; y++)
-                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x], b[y], acc[x][y], 0, 0, 0);
+                for (int y = 0; y < NT; y++)
+                    acc[x][y] =
+                        __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[x], fb[y], acc[x][y], 0, 0, 0);
+        }
+        if (more) {
+            a.template store<TA>(As[buf ^ 1], tid);
+            b.template store<!TB>(Bs[buf ^ 1], tid);
         }
         __syncthreads();
+        buf ^= 1;
     }
     // D layout of a 32x32 tile: value e of lane l is row 8*(e/4) + 4*(l/32) + e%4,
     // column l%32
 #pragma unroll
-    for (int x = 0; x < 2; x++)
+    for (int x = 0; x < MT; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++) {
-            const int col = n0 + 64 * wn + 32 * y + lr;
+        for (int y = 0; y < NT; y++) {
+            const int col = n0 + wn + 32 * y + lr;
             if (col >= N) continue;
             const float bc = bias ? bias[col] : 0.f;
 #pragma unroll
             for (int e = 0; e < 16; e++) {
-                const int row = m0 + 64 * wm + 32 * x + 8 * (e >> 2) + 4 * lg + (e & 3);
+                const int row = m0 + wm + 32 * x + 8 * (e >> 2) + 4 * lg + (e & 3);
                 if (row >= M) continue;
                 float v = alpha * acc[x][y][e] + bc;
                 if (beta != 0.f) v += beta * C[(size_t)row * ldc + col];
@@ -127,92 +182,194 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, float al
 }
 
 // h1[b][k] = b1[k] + sum_i W1t[(q*i + s_i)*H + k]  (W1t: (L*q, H), masked);
-// h1b = bf16(relu(h1)).  One thread per (b, k), k fastest.
-__global__ void k_made_embed(const uint8_t* __restrict__ seq, uint32_t ld, uint32_t B, uint32_t L,
-                             uint32_t q, uint32_t H, const float* __restrict__ W1t,
-                             const float* __restrict__ b1, float* __restrict__ h1,
-                             bf16* __restrict__ h1b) {
+// h1b = bf16(relu(h1)).  A thread forms V neighbouring units of EMB
+// neighbouring sequences, sites in order: EMB independent sums of V-wide
+// loads keep the gathered rows (bound by L2) in flight.
+constexpr int EMB = 4;
+template <int V>
+__global__ __launch_bounds__(256) void k_made_embed(const uint8_t* __restrict__ seq, uint32_t ld,
+                                                    uint32_t B, uint32_t L, uint32_t q, uint32_t H,
+                                                    const float* __restrict__ W1t,
+                                                    const float* __restrict__ b1,
+                                                    float* __restrict__ h1,
+                                                    bf16* __restrict__ h1b) {
+    typedef float fv __attribute__((ext_vector_type(V)));
+    typedef bf16 bv __attribute__((ext_vector_type(V)));
+    const uint32_t nk = H / V, nb = (B + EMB - 1) / EMB;
     const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (uint64_t)B * H) return;
-    const uint32_t b = (uint32_t)(idx / H), k = (uint32_t)(idx - (uint64_t)b * H);
-    float v = b1[k];
-    for (uint32_t i = 0; i < L; i++) v += W1t[(size_t)(q * i + seq[(size_t)i * ld + b]) * H + k];
-    h1[idx] = v;
-    h1b[idx] = (bf16)fmaxf(v, 0.f);
+    if (idx >= (uint64_t)nb * nk) return;
+    const uint32_t bg = (uint32_t)(idx / nk), k = (uint32_t)(idx - (uint64_t)bg * nk) * V;
+    // sequences past the batch repeat its last one and are not stored
+    uint32_t col[EMB];
+    fv v[EMB];
+#pragma unroll
+    for (int e = 0; e < EMB; e++) {
+        const uint32_t b = bg * EMB + e;
+        col[e] = b < B ? b : B - 1;
+        v[e] = *reinterpret_cast<const fv*>(b1 + k);
+    }
+#pragma unroll 4
+    for (uint32_t i = 0; i < L; i++) {
+        fv w[EMB];
+#pragma unroll
+        for (int e = 0; e < EMB; e++)
+            w[e] = *reinterpret_cast<const fv*>(
+                W1t + (size_t)(q * i + seq[(size_t)i * ld + col[e]]) * H + k);
+#pragma unroll
+        for (int e = 0; e < EMB; e++) v[e] += w[e];
+    }
+#pragma unroll
+    for (int e = 0; e < EMB; e++) {
+        const uint32_t b = bg * EMB + e;
+        if (b >= B) break;
+        *reinterpret_cast<fv*>(h1 + (size_t)b * H + k) = v[e];
+        bv r;
+#pragma unroll
+        for (int x = 0; x < V; x++) r[x] = (bf16)fmaxf(v[e][x], 0.f);
+        *reinterpret_cast<bv*>(h1b + (size_t)b * H + k) = r;
+    }
 }
 
-// dW1t[(q*i + a)*H + k] = sum over b with s_i(b) == a of dh1[b][k]: one
-// work-group per (site i, 256 units); thread k keeps its q sums in an LDS
-// column of its own and walks the batch in order, adding dh1[b][k] into the
-// row of the letter s_i(b) (a wave-uniform scalar load), so each sequence
-// costs one LDS read and write instead of a select over every letter.
-// Writes every entry, so no zeroing is needed; deterministic.
-constexpr int EG_T = 256, EG_QMAX = 25;
-__global__ __launch_bounds__(EG_T) void k_made_embed_grad(const uint8_t* __restrict__ seq,
-                                                          uint32_t ld, uint32_t B, uint32_t L,
-                                                          uint32_t q, uint32_t H,
-                                                          const float* __restrict__ dh1,
-                                                          float* __restrict__ dW1t) {
-    __shared__ float acc[EG_QMAX][EG_T];
-    const uint32_t nkb = (H + EG_T - 1) / EG_T;
-    const uint32_t i = blockIdx.x / nkb, k = (blockIdx.x % nkb) * EG_T + threadIdx.x;
-    for (uint32_t a = 0; a < q; a++) acc[a][threadIdx.x] = 0.f;
-    const uint8_t* si = seq + (size_t)i * ld;
-    if (k < H) {
-        // eight sequences per step: their letters and gradients are loaded
-        // before the eight additions (in batch order)
-        constexpr int U = 8;
-        uint32_t b = 0;
-        for (; b + U <= B; b += U) {
-            uint32_t sv[U];
-            float gv[U];
+// dW1t[(q*i + a)*H + k] = sum over b with s_i(b) == a of dh1[b][k], in batch
+// order: one wave per (EG_SITES sites, 64 units), whose lane k keeps its q sums
+// of each site in an LDS column of its own and adds dh1[b][k] into the row of
+// the letter s_i(b) (wave-uniform).  Bound by the chain of LDS read, add and
+// write, so EG_G sequences go through it together: their sums are read at
+// once, a sequence whose letter an earlier one of the group holds takes that
+// one's result, and the writes follow in order; and the sites' chains run side
+// by side on one load of the gradient.  Writes every entry, so no zeroing is
+// needed; deterministic.  (One sequence at a time, one site: 273 us at 4096 x
+// 232 x 512 units.)
+constexpr int EG_SITES = 2, EG_G = 4, EG_QMAX = 25;
+__global__ __launch_bounds__(64) void k_made_embed_grad(const uint8_t* __restrict__ seq,
+                                                        uint32_t ld, uint32_t B, uint32_t L,
+                                                        uint32_t q, uint32_t H,
+                                                        const float* __restrict__ dh1,
+                                                        float* __restrict__ dW1t) {
+    extern __shared__ float eg_acc[];   // [site][letter][64]
+    const uint32_t nkb = (H + 63) / 64;
+    const uint32_t i0 = blockIdx.x / nkb * EG_SITES;
+    const uint32_t lane = threadIdx.x, k = (blockIdx.x % nkb) * 64 + lane;
+    const bool on = k < H;
+    const float* gk = dh1 + (on ? k : 0);
+    for (uint32_t a = 0; a < EG_SITES * q; a++) eg_acc[a * 64 + lane] = 0.f;
+    // one group: letters (as row offsets) su[site][], gradients gu[]
+    auto add_group = [&](const uint32_t (&su)[EG_SITES][EG_G], const float* gu) {
+        float r[EG_SITES][EG_G];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                sv[u] = si[b + u];
-                gv[u] = dh1[(size_t)(b + u) * H + k];
+        for (int t = 0; t < EG_SITES; t++)
+#pragma unroll
+            for (int u = 0; u < EG_G; u++) r[t][u] = eg_acc[t * q * 64 + su[t][u] + lane];
+#pragma unroll
+        for (int u = 0; u < EG_G; u++)
+#pragma unroll
+            for (int t = 0; t < EG_SITES; t++) {
+                // the latest earlier sequence of the group with this letter
+                float v = r[t][u];
+#pragma unroll
+                for (int p = 0; p < u; p++) v = su[t][p] == su[t][u] ? r[t][p] : v;
+                r[t][u] = v + gu[u];
             }
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const uint32_t s = __builtin_amdgcn_readfirstlane(sv[u]);
-                acc[s < q ? s : q - 1][threadIdx.x] += gv[u];
+        for (int u = 0; u < EG_G; u++)
+#pragma unroll
+            for (int t = 0; t < EG_SITES; t++) eg_acc[t * q * 64 + su[t][u] + lane] = r[t][u];
+    };
+    constexpr int U = 4 * EG_G;   // gradients loaded ahead
+    for (uint32_t c0 = 0; c0 < B; c0 += 64) {
+        // the letters of 64 sequences, a lane each
+        const uint32_t n = B - c0 < 64 ? B - c0 : 64;
+        uint32_t sv[EG_SITES];
+#pragma unroll
+        for (int t = 0; t < EG_SITES; t++) {
+            const uint32_t i = i0 + t < L ? i0 + t : L - 1;
+            const uint32_t s = lane < n ? seq[(size_t)i * ld + c0 + lane] : 0u;
+            sv[t] = (s < q ? s : q - 1) * 64;
+        }
+        uint32_t u0 = 0;
+        for (; u0 + U <= n; u0 += U) {
+            float g[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) g[u] = gk[(size_t)(c0 + u0 + u) * H];
+#pragma unroll
+            for (int h = 0; h < U; h += EG_G) {
+                uint32_t su[EG_SITES][EG_G];
+#pragma unroll
+                for (int t = 0; t < EG_SITES; t++)
+#pragma unroll
+                    for (int u = 0; u < EG_G; u++)
+                        su[t][u] = __builtin_amdgcn_readlane(sv[t], u0 + h + u);
+                add_group(su, g + h);
             }
         }
-        for (; b < B; b++) {
-            const uint32_t s = __builtin_amdgcn_readfirstlane(si[b]);
-            acc[s < q ? s : q - 1][threadIdx.x] += dh1[(size_t)b * H + k];
+        for (; u0 < n; u0++) {
+            const float g = gk[(size_t)(c0 + u0) * H];
+#pragma unroll
+            for (int t = 0; t < EG_SITES; t++)
+                eg_acc[t * q * 64 + __builtin_amdgcn_readlane(sv[t], u0) + lane] += g;
         }
-        for (uint32_t a = 0; a < q; a++) dW1t[(size_t)(q * i + a) * H + k] = acc[a][threadIdx.x];
     }
+    if (!on) return;
+#pragma unroll
+    for (int t = 0; t < EG_SITES; t++)
+        if (i0 + t < L)
+            for (uint32_t a = 0; a < q; a++)
+                dW1t[(size_t)(q * (i0 + t) + a) * H + k] = eg_acc[(t * q + a) * 64 + lane];
 }
 
 // Per sequence b (one work-group): nll[b] = -sum_j log softmax(logits_j)[s_j]
 // and dlogits = gscale * (softmax - onehot), written bf16 (and fp32 if
-// dlf != null).  Threads stride over the sites; the block sum is a fixed
-// tree, so nll is deterministic.
+// dlf != null).  The sequence's logits go through LDS, so that memory is read
+// and written in whole lines (V values a thread) while each thread works on
+// its sites' q letters (read and written by their own threads, 84 bytes apart,
+// before: 727 us at 4096 x 232 x 21); threads stride over the sites, and the
+// block sum is a fixed tree, so nll is deterministic.
+template <int V>
 __global__ __launch_bounds__(256) void k_made_xent(const float* __restrict__ logits,
                                                    const uint8_t* __restrict__ seq, uint32_t ld,
                                                    uint32_t B, uint32_t L, uint32_t q, float gscale,
                                                    float* __restrict__ nll, bf16* __restrict__ dlb,
                                                    float* __restrict__ dlf) {
+    typedef float fv __attribute__((ext_vector_type(V)));
+    typedef bf16 bv __attribute__((ext_vector_type(V)));
+    extern __shared__ __attribute__((aligned(16))) float xrow[];   // 256 sites x q
     __shared__ float red[256];
     const uint32_t b = blockIdx.x, tid = threadIdx.x;
     const size_t row = (size_t)b * L * q;
     float part = 0.f;
-    for (uint32_t j = tid; j < L; j += 256) {
-        const float* z = logits + row + (size_t)j * q;
-        float mx = -INFINITY;
-        for (uint32_t a = 0; a < q; a++) mx = fmaxf(mx, z[a]);
-        float se = 0.f;
-        for (uint32_t a = 0; a < q; a++) se += expf(z[a] - mx);
-        const float lse = mx + logf(se);
-        const uint32_t s = seq[(size_t)j * ld + b];
-        part += lse - z[s];
+    for (uint32_t j0 = 0; j0 < L; j0 += 256) {
+        const uint32_t n = (L - j0 < 256 ? L - j0 : 256) * q;
+        const size_t at = row + (size_t)j0 * q;
+        for (uint32_t e = tid * V; e < n; e += 256 * V)
+            *reinterpret_cast<fv*>(xrow + e) = *reinterpret_cast<const fv*>(logits + at + e);
+        __syncthreads();
+        const uint32_t j = j0 + tid;
+        if (j < L) {
+            float* z = xrow + tid * q;
+            float mx = -INFINITY;
+            for (uint32_t a = 0; a < q; a++) mx = fmaxf(mx, z[a]);
+            float se = 0.f;
+            for (uint32_t a = 0; a < q; a++) se += expf(z[a] - mx);
+            const float lse = mx + logf(se);
+            const uint32_t s = seq[(size_t)j * ld + b];
+            part += lse - z[s];
+            if (dlb || dlf)
+                for (uint32_t a = 0; a < q; a++)
+                    z[a] = gscale * (expf(z[a] - lse) - (a == s ? 1.f : 0.f));
+        }
+        __syncthreads();
         if (dlb || dlf) {
-            for (uint32_t a = 0; a < q; a++) {
-                const float g = gscale * (expf(z[a] - lse) - (a == s ? 1.f : 0.f));
-                if (dlb) dlb[row + (size_t)j * q + a] = (bf16)g;
-                if (dlf) dlf[row + (size_t)j * q + a] = g;
+            for (uint32_t e = tid * V; e < n; e += 256 * V) {
+                const fv g = *reinterpret_cast<const fv*>(xrow + e);
+                if (dlf) *reinterpret_cast<fv*>(dlf + at + e) = g;
+                if (dlb) {
+                    bv r;
+#pragma unroll
+                    for (int x = 0; x < V; x++) r[x] = (bf16)g[x];
+                    *reinterpret_cast<bv*>(dlb + at + e) = r;
+                }
             }
+            __syncthreads();
         }
     }
     red[tid] = part;
@@ -552,8 +709,9 @@ __global__ void k_adam(uint64_t n, float* __restrict__ p, const float* __restric
 // takes 32 columns with 8 row lanes each: row lane t sums rows t, t + 8, ...
 // in order (each load instruction reads 8 rows x 128 contiguous bytes), then
 // the 8 partial sums are added in a fixed order, so the result is
-// deterministic.
-constexpr int CS_COLS = 32, CS_ROWL = 8;
+// deterministic.  Bound by the latency of its loads, CS_U of which are in
+// flight (one at a time: 440 us at 4096 x 4872).
+constexpr int CS_COLS = 32, CS_ROWL = 8, CS_U = 32;
 __global__ __launch_bounds__(CS_COLS * CS_ROWL) void k_colsum(uint32_t rows, uint32_t cols,
                                                               const float* __restrict__ x,
                                                               float* __restrict__ out) {
@@ -561,8 +719,17 @@ __global__ __launch_bounds__(CS_COLS * CS_ROWL) void k_colsum(uint32_t rows, uin
     const uint32_t cl = threadIdx.x % CS_COLS, t = threadIdx.x / CS_COLS;
     const uint32_t c = blockIdx.x * CS_COLS + cl;
     float s = 0.f;
-    if (c < cols)
-        for (uint32_t r = t; r < rows; r += CS_ROWL) s += x[(size_t)r * cols + c];
+    if (c < cols) {
+        uint32_t r = t;
+        for (; r + (CS_U - 1) * CS_ROWL < rows; r += CS_U * CS_ROWL) {
+            float v[CS_U];
+#pragma unroll
+            for (int u = 0; u < CS_U; u++) v[u] = x[(size_t)(r + u * CS_ROWL) * cols + c];
+#pragma unroll
+            for (int u = 0; u < CS_U; u++) s += v[u];
+        }
+        for (; r < rows; r += CS_ROWL) s += x[(size_t)r * cols + c];
+    }
     part[t][cl] = s;
     __syncthreads();
     if (t == 0 && c < cols) {

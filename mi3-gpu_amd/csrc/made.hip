@@ -31,6 +31,9 @@ int launched() {
 bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 }  // namespace
 
+// 128 x 128 GEMM tiles that fill 256 CUs twice.
+static constexpr int64_t GEMM_LARGE_TILES = 512;
+
 extern "C" {
 
 const char* mi3_made_last_error(void) { return g_made_error.c_str(); }
@@ -47,17 +50,26 @@ int mi3_gemm_bf16(void* stream, int transA, int transB, int M, int N, int K, flo
         (transB && ldb < K) || (C && ldc < N) || (Cb && ldcb < N))
         return mfail(MI3_EINVAL, "gemm: leading dimension too small");
     if (beta != 0.f && !C) return mfail(MI3_EINVAL, "gemm: beta needs C");
-    dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
     const bf16* a = static_cast<const bf16*>(A);
     const bf16* b = static_cast<const bf16*>(B);
     bf16* cb = static_cast<bf16*>(Cb);
-#define MI3_G(TA_, TB_)                                                                       \
-    hipLaunchKernelGGL((k_gemm_bf16<TA_, TB_>), grid, dim3(256), 0, S(stream), M, N, K, alpha, \
-                       a, lda, b, ldb, beta, C, ldc, cb, ldcb, bias, relu)
-    if (!transA && !transB) MI3_G(false, false);
-    else if (!transA && transB) MI3_G(false, true);
-    else if (transA && !transB) MI3_G(true, false);
-    else MI3_G(true, true);
+    // 128 x 128 tiles where they give every CU two; else 64 x 64, which read
+    // LDS twice as often per product but are four times as many (4872 x 512 over
+    // K = 4096: 156 against 616)
+    auto tiles = [&](int t) { return (int64_t)((N + t - 1) / t) * ((M + t - 1) / t); };
+    const int t = tiles(128) >= GEMM_LARGE_TILES ? 128 : 64;
+    const dim3 grid((N + t - 1) / t, (M + t - 1) / t);
+#define MI3_G(TA_, TB_)                                                                        \
+    if (t == 128)                                                                              \
+        hipLaunchKernelGGL((k_gemm_bf16<TA_, TB_, 128, 128>), grid, dim3(256), 0, S(stream), M, N, \
+                           K, alpha, a, lda, b, ldb, beta, C, ldc, cb, ldcb, bias, relu);      \
+    else                                                                                       \
+        hipLaunchKernelGGL((k_gemm_bf16<TA_, TB_, 64, 64>), grid, dim3(256), 0, S(stream), M, N, \
+                           K, alpha, a, lda, b, ldb, beta, C, ldc, cb, ldcb, bias, relu)
+    if (!transA && !transB) { MI3_G(false, false); }
+    else if (!transA && transB) { MI3_G(false, true); }
+    else if (transA && !transB) { MI3_G(true, false); }
+    else { MI3_G(true, true); }
 #undef MI3_G
     return launched();
 }
@@ -67,8 +79,15 @@ int mi3_made_embed(void* stream, const uint8_t* seq, uint32_t ld, uint32_t B, ui
                    void* h1b) {
     if (!seq || !W1t || !b1 || !h1 || !h1b || ld < B || q < 2 || q > MAX_Q)
         return mfail(MI3_EINVAL, "made_embed: bad arguments");
-    hipLaunchKernelGGL(k_made_embed, dim3(blocks((uint64_t)B * H)), dim3(256), 0, S(stream), seq,
-                       ld, B, L, q, H, W1t, b1, h1, static_cast<bf16*>(h1b));
+    if (B == 0 || H == 0) return MI3_OK;
+    const uint64_t nb = (B + EMB - 1) / EMB;
+    bf16* hb = static_cast<bf16*>(h1b);
+    if (H % 4 == 0 && al16(W1t) && al16(b1) && al16(h1) && al16(h1b))
+        hipLaunchKernelGGL(k_made_embed<4>, dim3(blocks(nb * (H / 4))), dim3(256), 0, S(stream),
+                           seq, ld, B, L, q, H, W1t, b1, h1, hb);
+    else
+        hipLaunchKernelGGL(k_made_embed<1>, dim3(blocks(nb * H)), dim3(256), 0, S(stream), seq, ld,
+                           B, L, q, H, W1t, b1, h1, hb);
     return launched();
 }
 
@@ -79,7 +98,9 @@ int mi3_made_embed_grad(void* stream, const uint8_t* seq, uint32_t ld, uint32_t 
     if (!seq || !dh1 || !dW1t || ld < B || q < 2 || q > MAX_Q)
         return mfail(MI3_EINVAL, "made_embed_grad: bad arguments");
     if (L == 0 || H == 0) return MI3_OK;
-    hipLaunchKernelGGL(k_made_embed_grad, dim3(L * ((H + EG_T - 1) / EG_T)), dim3(EG_T), 0,
+    const size_t lds = (size_t)EG_SITES * q * 64 * sizeof(float);
+    hipLaunchKernelGGL(k_made_embed_grad,
+                       dim3((L + EG_SITES - 1) / EG_SITES * ((H + 63) / 64)), dim3(64), lds,
                        S(stream), seq, ld, B, L, q, H, dh1, dW1t);
     return launched();
 }
@@ -89,8 +110,12 @@ int mi3_made_xent(void* stream, const float* logits, const uint8_t* seq, uint32_
                   float* dlogits) {
     if (!logits || !seq || !nll || ld < B || q < 2 || q > MAX_Q || B == 0)
         return mfail(MI3_EINVAL, "made_xent: bad arguments");
-    hipLaunchKernelGGL(k_made_xent, dim3(B), dim3(256), 0, S(stream), logits, seq, ld, B, L, q,
-                       gscale, nll, static_cast<bf16*>(dlogits_bf16), dlogits);
+    const size_t lds = (size_t)(L < 256 ? L : 256) * q * sizeof(float);   // logits of 256 sites
+    bf16* dlb = static_cast<bf16*>(dlogits_bf16);
+    auto kern = ((uint64_t)L * q % 4 == 0 && al16(logits) && al16(dlogits) && al16(dlb))
+                    ? k_made_xent<4> : k_made_xent<1>;
+    hipLaunchKernelGGL(kern, dim3(B), dim3(256), lds, S(stream), logits, seq, ld, B, L, q, gscale,
+                       nll, dlb, dlogits);
     return launched();
 }
 
