@@ -231,90 +231,114 @@ __global__ __launch_bounds__(256) void k_made_embed(const uint8_t* __restrict__ 
 }
 
 // dW1t[(q*i + a)*H + k] = sum over b with s_i(b) == a of dh1[b][k], in batch
-// order: one wave per (EG_SITES sites, 64 units), whose lane k keeps its q sums
-// of each site in an LDS column of its own and adds dh1[b][k] into the row of
-// the letter s_i(b) (wave-uniform).  Bound by the chain of LDS read, add and
-// write, so EG_G sequences go through it together: their sums are read at
-// once, a sequence whose letter an earlier one of the group holds takes that
-// one's result, and the writes follow in order; and the sites' chains run side
-// by side on one load of the gradient.  Writes every entry, so no zeroing is
-// needed; deterministic.  (One sequence at a time, one site: 273 us at 4096 x
-// 232 x 512 units.)
-constexpr int EG_SITES = 2, EG_G = 4, EG_QMAX = 25;
-__global__ __launch_bounds__(64) void k_made_embed_grad(const uint8_t* __restrict__ seq,
-                                                        uint32_t ld, uint32_t B, uint32_t L,
-                                                        uint32_t q, uint32_t H,
-                                                        const float* __restrict__ dh1,
-                                                        float* __restrict__ dW1t) {
-    extern __shared__ float eg_acc[];   // [site][letter][64]
-    const uint32_t nkb = (H + 63) / 64;
-    const uint32_t i0 = blockIdx.x / nkb * EG_SITES;
-    const uint32_t lane = threadIdx.x, k = (blockIdx.x % nkb) * 64 + lane;
+// order.  One work-group per (site, 64*V units): it sorts EG_CHUNK sequences
+// at a time by their letter at the site (a stable counting sort: the groups of
+// 64 sequences are ranked by ballots, and their counts prefixed), and each
+// wave sums the rows of every EG_WAVES-th letter in registers, several loads
+// in flight.  Bound by the reads of dh1 (once per site) from L2; the sums of
+// all letters in LDS instead are a chain of dependent read, add and write per
+// sequence (4096 x 232 x 512 units: 273 us, 328 us in groups of four).  Writes
+// every entry, so no zeroing is needed; deterministic.
+constexpr int EG_WAVES = 4, EG_CHUNK = 2048, EG_GROUPS = EG_CHUNK / 64, EG_QMAX = 25;
+constexpr int EG_LPW = (EG_QMAX + EG_WAVES - 1) / EG_WAVES;   // letters of a wave
+template <int V>
+__global__ __launch_bounds__(64 * EG_WAVES) void k_made_embed_grad(
+    const uint8_t* __restrict__ seq, uint32_t ld, uint32_t B, uint32_t L, uint32_t q, uint32_t H,
+    const float* __restrict__ dh1, float* __restrict__ dW1t) {
+    typedef float fv __attribute__((ext_vector_type(V)));
+    __shared__ uint16_t list[EG_CHUNK];             // sequences of the chunk by letter
+    __shared__ uint32_t cnt[EG_GROUPS][32];         // per group and letter: count, then place
+    __shared__ uint32_t off[33];                    // first place of each letter
+    const uint32_t nkb = (H + 64 * V - 1) / (64 * V);
+    const uint32_t i = blockIdx.x / nkb;
+    const uint32_t lane = threadIdx.x & 63, k = ((blockIdx.x % nkb) * 64 + lane) * V;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool on = k < H;
     const float* gk = dh1 + (on ? k : 0);
-    for (uint32_t a = 0; a < EG_SITES * q; a++) eg_acc[a * 64 + lane] = 0.f;
-    // one group: letters (as row offsets) su[site][], gradients gu[]
-    auto add_group = [&](const uint32_t (&su)[EG_SITES][EG_G], const float* gu) {
-        float r[EG_SITES][EG_G];
+    const uint8_t* si = seq + (size_t)i * ld;
+    fv acc[EG_LPW];
 #pragma unroll
-        for (int t = 0; t < EG_SITES; t++)
+    for (int x = 0; x < EG_LPW; x++) acc[x] = (fv)0.f;
+    for (uint32_t c0 = 0; c0 < B; c0 += EG_CHUNK) {
+        const uint32_t n = B - c0 < EG_CHUNK ? B - c0 : EG_CHUNK;
+        // ranks within groups of 64 (sequences past the batch: letter q)
+        uint32_t s[EG_GROUPS / EG_WAVES], rank[EG_GROUPS / EG_WAVES];
 #pragma unroll
-            for (int u = 0; u < EG_G; u++) r[t][u] = eg_acc[t * q * 64 + su[t][u] + lane];
-#pragma unroll
-        for (int u = 0; u < EG_G; u++)
-#pragma unroll
-            for (int t = 0; t < EG_SITES; t++) {
-                // the latest earlier sequence of the group with this letter
-                float v = r[t][u];
-#pragma unroll
-                for (int p = 0; p < u; p++) v = su[t][p] == su[t][u] ? r[t][p] : v;
-                r[t][u] = v + gu[u];
+        for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
+            const uint32_t g = wave * (EG_GROUPS / EG_WAVES) + x, b = g * 64 + lane;
+            s[x] = q;
+            if (b < n) {
+                s[x] = si[c0 + b];
+                if (s[x] >= q) s[x] = q - 1;
             }
-#pragma unroll
-        for (int u = 0; u < EG_G; u++)
-#pragma unroll
-            for (int t = 0; t < EG_SITES; t++) eg_acc[t * q * 64 + su[t][u] + lane] = r[t][u];
-    };
-    constexpr int U = 4 * EG_G;   // gradients loaded ahead
-    for (uint32_t c0 = 0; c0 < B; c0 += 64) {
-        // the letters of 64 sequences, a lane each
-        const uint32_t n = B - c0 < 64 ? B - c0 : 64;
-        uint32_t sv[EG_SITES];
-#pragma unroll
-        for (int t = 0; t < EG_SITES; t++) {
-            const uint32_t i = i0 + t < L ? i0 + t : L - 1;
-            const uint32_t s = lane < n ? seq[(size_t)i * ld + c0 + lane] : 0u;
-            sv[t] = (s < q ? s : q - 1) * 64;
+            rank[x] = 0;
+            uint32_t c = 0;
+            for (uint32_t a = 0; a < q; a++) {
+                const uint64_t m = __ballot(s[x] == a);
+                const uint32_t r = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                rank[x] = s[x] == a ? r : rank[x];
+                c = lane == a ? (uint32_t)__popcll(m) : c;
+            }
+            if (lane < 32) cnt[g][lane] = c;
         }
-        uint32_t u0 = 0;
-        for (; u0 + U <= n; u0 += U) {
-            float g[U];
+        __syncthreads();
+        // places: letters in order, within a letter the groups in order
+        if (threadIdx.x < 32) {
+            uint32_t t = 0;
+            for (uint32_t g = 0; g < EG_GROUPS; g++) t += cnt[g][threadIdx.x];
+            uint32_t before = 0;
+            for (uint32_t a = 0; a < q; a++) {
+                const uint32_t ta = __shfl(t, a, 32);
+                before += a < threadIdx.x ? ta : 0u;
+            }
+            off[threadIdx.x] = before;
+            for (uint32_t g = 0; g < EG_GROUPS; g++) {
+                const uint32_t c = cnt[g][threadIdx.x];
+                cnt[g][threadIdx.x] = before;
+                before += c;
+            }
+            if (threadIdx.x == 31) off[32] = before;
+        }
+        __syncthreads();
 #pragma unroll
-            for (int u = 0; u < U; u++) g[u] = gk[(size_t)(c0 + u0 + u) * H];
+        for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
+            const uint32_t g = wave * (EG_GROUPS / EG_WAVES) + x;
+            if (s[x] < q) list[cnt[g][s[x]] + rank[x]] = (uint16_t)(g * 64 + lane);
+        }
+        __syncthreads();
 #pragma unroll
-            for (int h = 0; h < U; h += EG_G) {
-                uint32_t su[EG_SITES][EG_G];
+        for (int x = 0; x < EG_LPW; x++) {
+            const uint32_t a = wave + EG_WAVES * x;
+            if (a >= q) continue;
+            const uint32_t e1 = __builtin_amdgcn_readfirstlane(off[a + 1]);
+            for (uint32_t e0 = __builtin_amdgcn_readfirstlane(off[a]); e0 < e1; e0 += 64) {
+                const uint32_t m = e1 - e0 < 64 ? e1 - e0 : 64;
+                const uint32_t mine = lane < m ? list[e0 + lane] : 0u;
+                constexpr int U = 8;
+                uint32_t u0 = 0;
+                for (; u0 + U <= m; u0 += U) {
+                    fv g[U];
 #pragma unroll
-                for (int t = 0; t < EG_SITES; t++)
+                    for (int u = 0; u < U; u++)
+                        g[u] = *reinterpret_cast<const fv*>(
+                            gk + (size_t)(c0 + __builtin_amdgcn_readlane(mine, u0 + u)) * H);
 #pragma unroll
-                    for (int u = 0; u < EG_G; u++)
-                        su[t][u] = __builtin_amdgcn_readlane(sv[t], u0 + h + u);
-                add_group(su, g + h);
+                    for (int u = 0; u < U; u++) acc[x] += g[u];
+                }
+                for (; u0 < m; u0++)
+                    acc[x] += *reinterpret_cast<const fv*>(
+                        gk + (size_t)(c0 + __builtin_amdgcn_readlane(mine, u0)) * H);
             }
         }
-        for (; u0 < n; u0++) {
-            const float g = gk[(size_t)(c0 + u0) * H];
-#pragma unroll
-            for (int t = 0; t < EG_SITES; t++)
-                eg_acc[t * q * 64 + __builtin_amdgcn_readlane(sv[t], u0) + lane] += g;
-        }
+        __syncthreads();
     }
     if (!on) return;
 #pragma unroll
-    for (int t = 0; t < EG_SITES; t++)
-        if (i0 + t < L)
-            for (uint32_t a = 0; a < q; a++)
-                dW1t[(size_t)(q * (i0 + t) + a) * H + k] = eg_acc[(t * q + a) * 64 + lane];
+    for (int x = 0; x < EG_LPW; x++) {
+        const uint32_t a = wave + EG_WAVES * x;
+        if (a < q) *reinterpret_cast<fv*>(dW1t + (size_t)(q * i + a) * H + k) = acc[x];
+    }
 }
 
 // Per sequence b (one work-group): nll[b] = -sum_j log softmax(logits_j)[s_j]

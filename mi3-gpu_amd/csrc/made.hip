@@ -98,10 +98,12 @@ int mi3_made_embed_grad(void* stream, const uint8_t* seq, uint32_t ld, uint32_t 
     if (!seq || !dh1 || !dW1t || ld < B || q < 2 || q > MAX_Q)
         return mfail(MI3_EINVAL, "made_embed_grad: bad arguments");
     if (L == 0 || H == 0) return MI3_OK;
-    const size_t lds = (size_t)EG_SITES * q * 64 * sizeof(float);
-    hipLaunchKernelGGL(k_made_embed_grad,
-                       dim3((L + EG_SITES - 1) / EG_SITES * ((H + 63) / 64)), dim3(64), lds,
-                       S(stream), seq, ld, B, L, q, H, dh1, dW1t);
+    if (H % 4 == 0 && al16(dh1) && al16(dW1t))
+        hipLaunchKernelGGL(k_made_embed_grad<4>, dim3(L * ((H + 255) / 256)), dim3(64 * EG_WAVES), 0,
+                           S(stream), seq, ld, B, L, q, H, dh1, dW1t);
+    else
+        hipLaunchKernelGGL(k_made_embed_grad<1>, dim3(L * ((H + 63) / 64)), dim3(64 * EG_WAVES), 0,
+                           S(stream), seq, ld, B, L, q, H, dh1, dW1t);
     return launched();
 }
 

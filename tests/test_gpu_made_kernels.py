@@ -36,9 +36,10 @@ def test_gemm_tile_edges(gpu_ok, M, N, K, ta, tb):
 
 
 # (L, q, B, H): vector and scalar forms, batches that end inside a group of 4
-# sequences, 16 gradients or 64 letters, more than 256 sites, odd numbers of sites
+# sequences, 64 or 2048 letters, more than 256 sites, odd numbers of sites
 @pytest.mark.parametrize("L,q,B,H", [(2, 2, 1, 1), (5, 3, 7, 30), (16, 21, 64, 64), (33, 25, 70, 68),
-                                     (257, 4, 300, 32), (300, 7, 33, 130)])
+                                     (257, 4, 300, 32), (300, 7, 33, 130),
+                                     (3, 20, 2050, 260)])
 def test_embedding_and_softmax(gpu_ok, L, q, B, H):
     from mi3gpu._lib import lib
     rng = np.random.default_rng(L)
