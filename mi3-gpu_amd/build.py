@@ -22,10 +22,11 @@ BUILD = HERE / '_build'
 ARCH = os.environ.get('MI3_OFFLOAD_ARCH', 'gfx950')
 
 # (source, object, extra flags)
-UNITS = [(u, Path(u).stem + '.o', []) for u in ('sweep_direct.hip', 'sweep_steps.hip', 'runtime.hip',
-                                                'potts.hip', 'batch.hip', 'made.hip')]
-# the chunk-staged sweep once for each number of state words
-UNITS += [('sweep_chunk.hip', f'sweep_chunk_{kw}.o', [f'-DMI3_KW={kw}']) for kw in range(1, 9)]
+UNITS = [(u, Path(u).stem + '.o', []) for u in ('sweep_direct.hip', 'sweep_steps.hip', 'energies_rows.hip',
+                                                'runtime.hip', 'potts.hip', 'batch.hip', 'made.hip')]
+# the chunk-staged kernels once for each number of state words
+UNITS += [(f'{k}_chunk.hip', f'{k}_chunk_{kw}.o', [f'-DMI3_KW={kw}'])
+          for kw in range(8, 0, -1) for k in ('sweep', 'energies')]
 
 CFLAGS = [
     f'--offload-arch={ARCH}', '-O3', '-fPIC', '-std=c++17',

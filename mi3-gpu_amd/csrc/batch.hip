@@ -120,8 +120,9 @@ std::vector<uint32_t> tile_options(uint32_t kw) {
 // Tiles of a class for a walkers-per-tile choice; larger models first so
 // that the tail of the persistent loop is short.  The largest tile stands for
 // the library's choice, as the single-model sweep makes it: no staging for a
-// class of few walkers, else the smaller of two tiles where it needs no more
-// rounds over the CUs (8 models of 1024-4096 walkers: 4 sweeps took 30.6 ms in
+// class of few walkers (more than a single model's, since classes without
+// staging follow one another), else smaller tiles where they leave most of the
+// card free (8 models of 1024-4096 walkers: 4 sweeps took 30.6 ms in
 // tiles of 512, all on the two work-groups of the L=400 model).
 int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
     uint64_t total = 0;
@@ -134,9 +135,8 @@ int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
     cr.direct = false;
     cr.run_wpb = wpb;
     if (wpb == tile_options(key.kw).back()) {
-        cr.direct = total <= direct_walkers(qmin, ncu);
-        auto rounds = [&](uint32_t w) { return (total / w + ncu - 1) / ncu; };
-        while (cr.run_wpb > 128 && rounds(cr.run_wpb / 2) == rounds(cr.run_wpb)) cr.run_wpb /= 2;
+        cr.direct = total <= (uint64_t)(qmin <= 8 ? 24 : 32) * ncu;
+        cr.run_wpb = chunk_tile((uint32_t)std::min<uint64_t>(total, 1u << 30), wpb, ncu);
     }
     std::vector<BatchTile> t;
     std::vector<uint32_t> order = cr.models;

@@ -253,14 +253,6 @@ __device__ __forceinline__ uint32_t byte_x128(uint32_t w, int e) {
     return r;
 }
 
-// a * b + c for 24-bit a, b in one op (the compiler turns the add of
-// disjoint bit ranges into an or, which then stays a separate instruction).
-__device__ __forceinline__ uint32_t mad_u24(uint32_t a, uint32_t b, uint32_t c) {
-    uint32_t r;
-    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 // ---------------------------------------------------------------------------
 // Metropolis sweep: nsteps single-site updates per walker.
 //
@@ -329,20 +321,70 @@ struct Walkers {
     uint32_t Xe, Xo;          // this lane's draws (steps 2h, 2h+1 of its own pair)
     int remap;                // bpermute address: row lane e <- the lane deciding slot e
 
+    // A lane's S walkers are neighbours in a row of the sequence buffer: where
+    // rows are aligned for it, one S-byte load per site fetches all of them (the
+    // byte loads, S times as many, took a fifth of the energies' time at L=93
+    // q=4), and byte permutes turn four sites' loads into S words.
+    static constexpr bool WIDE = S >= 4;
+    __device__ static __forceinline__ bool rows_aligned(const uint8_t* seq, uint32_t ldseq) {
+        return (((uint32_t)(uintptr_t)seq | ldseq) & (S - 1)) == 0;
+    }
+    // 4 x 4 bytes transposed: word i holds byte i of a, b, c, d (and back)
+    __device__ static __forceinline__ void transpose4(uint32_t& a, uint32_t& b, uint32_t& c,
+                                                      uint32_t& d) {
+        const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u);
+        const uint32_t ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+        const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u);
+        const uint32_t cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+        a = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+        b = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+        c = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+        d = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+    }
+
+    // (walkers from `end` on read as residue 0)
     __device__ __forceinline__ void load(const uint8_t* seq, uint32_t ldseq, uint32_t L,
-                                         uint32_t wfirst, uint32_t lane) {
+                                         uint32_t wfirst, uint32_t lane,
+                                         uint32_t end = 0xffffffffu) {
         const uint32_t j = lane & 31;
         remap = (int)((((lane & 15) << SH) & 31) | (lane & 32)) * 4;
         Xe = Xo = 0;
+        if constexpr (WIDE) {
+            if (rows_aligned(seq, ldseq)) {
+                typedef uint32_t wv __attribute__((ext_vector_type(S / 4)));
+#pragma unroll
+                for (int i = 0; i < KW; i++) {
+                    uint32_t v[4][S / 4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t m = j + CH * (4 * i + e);
+                        wv x = (wv)0u;
+                        if (m < L && wfirst < end)
+                            x = *reinterpret_cast<const wv*>(seq + (size_t)m * ldseq + wfirst);
+#pragma unroll
+                        for (int d = 0; d < S / 4; d++) v[e][d] = x[d];
+                    }
+#pragma unroll
+                    for (int d = 0; d < S / 4; d++) {
+                        transpose4(v[0][d], v[1][d], v[2][d], v[3][d]);
+#pragma unroll
+                        for (int g = 0; g < 4; g++)
+                            st[4 * d + g][i] = wfirst + 4 * d + g < end ? v[g][d] : 0u;
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int s = 0; s < S; s++) {
+            const bool valid = wfirst + s < end;
 #pragma unroll
             for (int i = 0; i < KW; i++) {
                 uint32_t word = 0;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     uint32_t m = j + CH * (4 * i + e);
-                    uint32_t v = (m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
+                    uint32_t v = (valid && m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
                     word |= v << (8 * e);
                 }
                 st[s][i] = word;
@@ -354,6 +396,30 @@ struct Walkers {
     __device__ __forceinline__ void store(uint8_t* seq, uint32_t ldseq, uint32_t L,
                                           uint32_t wfirst, uint32_t lane) const {
         const uint32_t j = lane & 31;
+        if constexpr (WIDE) {
+            if (rows_aligned(seq, ldseq)) {
+                typedef uint32_t wv __attribute__((ext_vector_type(S / 4)));
+#pragma unroll
+                for (int i = 0; i < KW; i++) {
+                    uint32_t v[4][S / 4];
+#pragma unroll
+                    for (int d = 0; d < S / 4; d++) {
+#pragma unroll
+                        for (int g = 0; g < 4; g++) v[g][d] = st[4 * d + g][i];
+                        transpose4(v[0][d], v[1][d], v[2][d], v[3][d]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const uint32_t m = j + CH * (4 * i + e);
+                        wv x;
+#pragma unroll
+                        for (int d = 0; d < S / 4; d++) x[d] = v[e][d];
+                        if (m < L) *reinterpret_cast<wv*>(seq + (size_t)m * ldseq + wfirst) = x;
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int s = 0; s < S; s++) {
 #pragma unroll
@@ -449,6 +515,24 @@ struct Walkers {
 #pragma unroll
             for (int s = 4 * g; s < 4 * g + 4 && s < S; s++)
                 baseA[s] = QB ? byte_x128(aq, s & 3) + org : __umul24(byte_x128(aq, s & 3), q) + org;
+        }
+    }
+
+    // Row addresses a * q * 128 + origin of every slot's residue at site pos.
+    __device__ __forceinline__ void row_bases(uint32_t pos, uint32_t lane, uint32_t q,
+                                              uint32_t origin, uint32_t (&base)[S]) const {
+        uint32_t org = origin;
+        asm("" : "+v"(org));   // as in bases()
+        uint32_t apk[NP];
+        residues(pos, lane, apk);
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            if constexpr (QB) {
+                if (s % 4 == 0) apk[s / 4] *= q;
+                base[s] = byte_x128(apk[s / 4], s & 3) + org;
+            } else {
+                base[s] = __umul24(byte_x128(apk[s / 4], s & 3), q) + org;
+            }
         }
     }
 
@@ -950,194 +1034,300 @@ __global__ __launch_bounds__(64 * NWAVES) void k_stage_probe(const float* __rest
 
 // ---------------------------------------------------------------------------
 // Batch energies E(s) = sum_{i<m} J_{i,m}(s_i, s_m) of nseq sequences.
-// Restates getEnergies (mcmc.cl:249-345); same layout and staging as the
-// sweep, streaming for each row i only the chunks holding m > i.
+// Restates getEnergies (mcmc.cl:249-345); the sweep's layout, with, for each
+// row i, only the chunks holding partners m > i.  As the sweep, in three forms:
+// chunks staged one at a time, the rows of a stage staged at once (q <= 8), and
+// unstaged (few sequences).
+
+// Sum of the gathers of chunk k over the lane's slots.  MASK: the diagonal
+// chunk, where only partners m > i count, as a 0/1 factor (fma(v, 1, acc) is
+// acc + v exactly).  The other chunks add without it for up to two state words
+// (an add takes half the time of an fma); beyond, two copies spill.
+template <bool MASK, int KW, int S, bool QB>
+__device__ __forceinline__ void energy_chunk(const Walkers<KW, S, QB>& w, int k, const char* cb,
+                                             const uint32_t (&base)[S], float keep,
+                                             float (&acc)[S]) {
+    constexpr int G = (S < 16) ? S : 16;
+#pragma unroll
+    for (int s0 = 0; s0 < S; s0 += G) {
+        float v[G];
+#pragma unroll
+        for (int g = 0; g < G; g++)
+            v[g] = *reinterpret_cast<const float*>(
+                cb + (base[s0 + g] + byte_x128(w.st[s0 + g][k >> 2], k & 3)));
+#pragma unroll
+        for (int g = 0; g < G; g++)
+            acc[s0 + g] = MASK ? __fmaf_rn(v[g], keep, acc[s0 + g]) : acc[s0 + g] + v[g];
+    }
+}
+
+template <int KW, int S, bool QB>
+__device__ __forceinline__ void store_energies(const float (&acc)[S], float* E, uint32_t wfirst,
+                                               uint32_t lane, uint32_t nseq) {
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        const float e = half_wave_sum(acc[s]);
+        if ((lane & 31) == 0 && wfirst + s < nseq) E[wfirst + s] = e;
+    }
+}
+
 template <int KW, int S, int NWAVES, int PF, bool OVL>
 __global__ __launch_bounds__(64 * NWAVES) void k_energies(
     const float* __restrict__ Ju, const uint8_t* __restrict__ seq, float* __restrict__ E,
     uint32_t ldseq, uint32_t nseq, uint32_t L, uint32_t q, uint32_t nchunk) {
     constexpr int NT = 64 * NWAVES;
     constexpr int K = 4 * KW;
+    using W = Walkers<KW, S, (PF <= 4)>;
     extern __shared__ f4v lds4[];
 
     // the padded chunk is PF float4 per thread of the first DMA_T threads
     // (the chunk layout's unit); waves beyond them take no part in staging
     constexpr int DMA_T = NT < 512 ? NT : 512;
-    constexpr uint32_t chf = PF * DMA_T * 4;  // padded chunk (floats)
+    // (a tile of fewer than 512 threads copies a chunk in several passes)
+    constexpr int PASS = 512 / DMA_T;
+    constexpr uint32_t chb = PF * 512 * 16;  // padded chunk (bytes)
     const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    const uint32_t lane = tid & 63;
     const uint32_t j = lane & 31;
-    const bool upper = lane >= 32;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t wfirst = blockIdx.x * (2 * S * NWAVES) + (wave * 2 + (upper ? 1 : 0)) * S;
-
-    uint32_t st[S][KW];
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-        const bool valid = wfirst + s < nseq;
-#pragma unroll
-        for (int kw = 0; kw < KW; kw++) {
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                uint32_t m = j + CH * (4 * kw + e);
-                uint32_t v = (valid && m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
-                word |= v << (8 * e);
-            }
-            st[s][kw] = word;
-        }
-        asm volatile("" ::: "memory");
-    }
+    const uint32_t wfirst = blockIdx.x * (2 * S * NWAVES) + (wave * 2 + (lane >> 5)) * S;
+    W w;
+    w.load(seq, ldseq, L, wfirst, lane, nseq);
     float acc[S];
 #pragma unroll
     for (int s = 0; s < S; s++) acc[s] = 0.f;
-    // row offsets of the slots: in LDS bytes, so that a gather address is
-    // one SDWA shift of the partner residue and one add, for up to 16 slots
-    // per half-wave (3.05 against 4.67 ms at L=300 q=8, 7.9 against 10.2 ms
-    // at L=400 q=21); in floats for 32 slots, where byte offsets took 3.4
-    // against 2.5 ms at L=232 q=21 (no launch shape uses 32 slots now)
-    constexpr bool BYTE_ADDR = S <= 16;
     uint32_t base[S];
 
-    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * nchunk * chf * 4);
+    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * nchunk * chb);
     const uint32_t voff = tid * 16;
     // staging waves, as in the sweep
     const bool stage = (PF == 1) ? (uint32_t)wave < (q * q + 7) / 8 : wave < DMA_T / 64;
     char* ldsb = reinterpret_cast<char*>(lds4);
-    if (L >= 2) {
-        // OVL: copy cursor (row ci, chunk ck) two units ahead of the gathers
-        // and the byte offset of the unit one ahead; at the last unit the
-        // cursor stays, so copies past the end repeat it into unread slots
-        uint32_t ci = 0, ck = 0, off_next = 0;
-        auto advance = [&]() {
-            const bool wrap = ck + 1 >= nchunk;
-            const bool stay = wrap && ci + 2 >= L;
-            ck = stay ? ck : (wrap ? (ci + 2) >> 5 : ck + 1);
-            ci = (wrap && !stay) ? ci + 1 : ci;
-        };
-        if constexpr (OVL) {
-            static_assert(PF == 7 && DMA_T == 512, "overlapping ring: chunks of q = 17..21");
-            // unit (0, 0) whole into slot 0, then the early part of the next
-            if (wave < 8) {
-                OverlapRing::copy<OverlapRing::EARLY_OPS>(rJ, voff, 0, ldsb, 0,
-                                                          OverlapRing::early_first(0), wave);
-                OverlapRing::copy<OverlapRing::LATE_OPS>(rJ, voff, 0, ldsb, 0,
-                                                         OverlapRing::late_first(0), wave);
-            }
-            advance();
-            off_next = (ci * nchunk + ck) * chf * 4;
-            if (wave < 8)
-                OverlapRing::copy<OverlapRing::EARLY_OPS>(rJ, voff, off_next, ldsb, 1,
-                                                          OverlapRing::early_first(1), wave);
-            advance();
-            wait_vmem_upto<OverlapRing::EARLY_OPS>();
-            barrier_copies_in_flight();
-        } else {
-            // first unit: row 0, chunk 0
-            if (stage) chunk_dma<PF, DMA_T>(rJ, voff, 0, ldsb, wave);
-            wait_vmem();
-            __syncthreads();
+    // OVL: copy cursor (row ci, chunk ck) two units ahead of the gathers
+    // and the byte offset of the unit one ahead; at the last unit the
+    // cursor stays, so copies past the end repeat it into unread slots
+    uint32_t ci = 0, ck = 0, off_next = 0;
+    auto advance = [&]() {
+        const bool wrap = ck + 1 >= nchunk;
+        const bool stay = wrap && ci + 2 >= L;
+        ck = stay ? ck : (wrap ? (ci + 2) >> 5 : ck + 1);
+        ci = (wrap && !stay) ? ci + 1 : ci;
+    };
+    if constexpr (OVL) {
+        static_assert(PF == 7 && DMA_T == 512, "overlapping ring: chunks of q = 17..21");
+        // unit (0, 0) whole into slot 0, then the early part of the next
+        if (wave < 8) {
+            OverlapRing::copy<OverlapRing::EARLY_OPS>(rJ, voff, 0, ldsb, 0,
+                                                      OverlapRing::early_first(0), wave);
+            OverlapRing::copy<OverlapRing::LATE_OPS>(rJ, voff, 0, ldsb, 0,
+                                                     OverlapRing::late_first(0), wave);
         }
-        uint32_t buf = 0;
-        const uint32_t qch = q * CH;
-        for (uint32_t i = 0; i + 1 < L; i++) {
-            const uint32_t kp = i >> 5, owner = i & 31;
-            const uint32_t kwp = kp >> 2, shp = (kp & 3) * 8;
-            const uint32_t c0 = (i + 1) >> 5;
-            // each slot's residue at site i, from the owner lane of its
-            // half-wave (one ds_bpermute per slot; two v_readlane and a
-            // select per slot took 9-19% longer), then its row offset
-            const int own_addr = (int)((owner + (lane & 32)) * 4);
+        advance();
+        off_next = (ci * nchunk + ck) * chb;
+        if (wave < 8)
+            OverlapRing::copy<OverlapRing::EARLY_OPS>(rJ, voff, off_next, ldsb, 1,
+                                                      OverlapRing::early_first(1), wave);
+        advance();
+        wait_vmem_upto<OverlapRing::EARLY_OPS>();
+        barrier_copies_in_flight();
+    } else {
+        // first unit: row 0, chunk 0
+        if (stage) chunk_dma<PF * PASS, DMA_T>(rJ, voff, 0, ldsb, wave);
+        wait_vmem();
+        __syncthreads();
+    }
+    uint32_t ring = 0;
+    // one row whose chunk k is in buffer (p + k) % 2; as the sweep's step,
+    // compiled for either p where that does not spill
+    constexpr bool TWICE = KW <= 2 && !OVL;
+    auto row = [&](auto pc, uint32_t pv, uint32_t i) __attribute__((always_inline)) {
+        const uint32_t p = TWICE ? decltype(pc)::value : pv;
+        const uint32_t kp = i >> 5, c0 = (i + 1) >> 5;
+        w.row_bases(i, lane, q, j * 4, base);
+        const float keep = (c0 != kp || j > (i & 31)) ? 1.f : 0.f;
 #pragma unroll
-            for (int s = 0; s < S; s++) {
-                const uint32_t av = __builtin_amdgcn_ubfe(select_word<KW>(st[s], kwp), shp, 8);
-                base[s] = (uint32_t)__builtin_amdgcn_ds_bpermute(own_addr, (int)av);
-            }
-#pragma unroll
-            for (int s = 0; s < S; s++)
-                base[s] = BYTE_ADDR ? mad_u24(base[s], qch * 4, j * 4) : mad_u24(base[s], qch, j);
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                if ((uint32_t)k >= c0 && (uint32_t)k < nchunk) {
-                    const char* cbb;
-                    if constexpr (OVL) {
-                        // late part of the next unit, early part of the one after
-                        if (wave < 8) {
-                            OverlapRing::copy<OverlapRing::LATE_OPS>(
-                                rJ, voff, off_next, ldsb, (buf + 1) & 3,
-                                OverlapRing::late_first((buf + 1) & 3), wave);
-                            OverlapRing::copy<OverlapRing::EARLY_OPS>(
-                                rJ, voff, (ci * nchunk + ck) * chf * 4, ldsb, (buf + 2) & 3,
-                                OverlapRing::early_first((buf + 2) & 3), wave);
-                        }
-                        off_next = (ci * nchunk + ck) * chf * 4;
-                        advance();
-                        cbb = ldsb + OverlapRing::base(buf);
-                    } else {
-                        const bool last_chunk = (uint32_t)k + 1 == nchunk;
-                        const bool has_next = !last_chunk || (i + 2 < L);
-                        if (has_next) {
-                            uint32_t ni = last_chunk ? i + 1 : i;
-                            uint32_t nc = last_chunk ? ((i + 2) >> 5) : (uint32_t)k + 1;
-                            if (stage)
-                                chunk_dma<PF, DMA_T>(rJ, voff, (ni * nchunk + nc) * chf * 4,
-                                                     ldsb + (buf ^ 1) * chf * 4, wave);
-                        }
-                        cbb = ldsb + buf * chf * 4;
+        for (int k = 0; k < K; k++) {
+            if ((uint32_t)k >= c0 && (uint32_t)k < nchunk) {
+                const char* cb;
+                if constexpr (OVL) {
+                    // late part of the next unit, early part of the one after
+                    if (wave < 8) {
+                        OverlapRing::copy<OverlapRing::LATE_OPS>(
+                            rJ, voff, off_next, ldsb, (ring + 1) & 3,
+                            OverlapRing::late_first((ring + 1) & 3), wave);
+                        OverlapRing::copy<OverlapRing::EARLY_OPS>(
+                            rJ, voff, (ci * nchunk + ck) * chb, ldsb, (ring + 2) & 3,
+                            OverlapRing::early_first((ring + 2) & 3), wave);
                     }
-                    const float* cb = reinterpret_cast<const float*>(cbb);
-                    if constexpr (S > 16) {
-                        // the state is loop-invariant: without this the
-                        // compiler hoists the S*K extracted residues out of
-                        // the loops, which at 32 slots spills registers
-#pragma unroll
-                        for (int s = 0; s < S; s++)
-#pragma unroll
-                            for (int kw = 0; kw < KW; kw++) asm volatile("" : "+v"(st[s][kw]));
+                    off_next = (ci * nchunk + ck) * chb;
+                    advance();
+                    cb = ldsb + OverlapRing::base(ring);
+                } else {
+                    const uint32_t buf = (p + k) & 1;
+                    const bool last_chunk = (uint32_t)k + 1 == nchunk;
+                    const bool has_next = !last_chunk || (i + 2 < L);
+                    if (has_next) {
+                        const uint32_t ni = last_chunk ? i + 1 : i;
+                        const uint32_t nc = last_chunk ? ((i + 2) >> 5) : (uint32_t)k + 1;
+                        if (stage)
+                            chunk_dma<PF * PASS, DMA_T>(rJ, voff, (ni * nchunk + nc) * chb,
+                                                        ldsb + (buf ^ 1) * chb, wave);
                     }
-                    // on the diagonal chunk only partners m > i count: a 0/1
-                    // factor (fma(v, 1, acc) == acc + v exactly)
-                    const float keep = ((uint32_t)k != kp || j > owner) ? 1.f : 0.f;
-                    constexpr int G = (S < 16) ? S : 16;
-#pragma unroll
-                    for (int s0 = 0; s0 < S; s0 += G) {
-                        float v[G];
-#pragma unroll
-                        for (int g = 0; g < G; g++) {
-                            const uint32_t w = state_word<KW>(st[s0 + g], (uint32_t)k >> 2);
-                            if constexpr (BYTE_ADDR) {
-                                v[g] = *reinterpret_cast<const float*>(
-                                    cbb + base[s0 + g] + byte_x128(w, k & 3));
-                            } else {
-                                const uint32_t sm = (w >> ((k & 3) * 8)) & 0xffu;
-                                v[g] = cb[base[s0 + g] + sm * CH];
-                            }
-                        }
-#pragma unroll
-                        for (int g = 0; g < G; g++) acc[s0 + g] = __fmaf_rn(v[g], keep, acc[s0 + g]);
-                    }
-                    if constexpr (OVL) {
-                        // the next unit has landed (only the early part of
-                        // the one after may be in flight)
-                        wait_vmem_upto<OverlapRing::EARLY_OPS>();
-                        barrier_copies_in_flight();
-                        buf = (buf + 1) & 3;
-                    } else {
-                        wait_vmem();
-                        __syncthreads();
-                        buf ^= 1;
-                    }
+                    cb = ldsb + buf * chb;
+                }
+                if constexpr (KW <= 2) {
+                    if ((uint32_t)k == c0) energy_chunk<true>(w, k, cb, base, keep, acc);
+                    else energy_chunk<false>(w, k, cb, base, keep, acc);
+                } else {
+                    energy_chunk<true>(w, k, cb, base, (uint32_t)k == c0 ? keep : 1.f, acc);
+                }
+                if constexpr (OVL) {
+                    // the next unit has landed (only the early part of
+                    // the one after may be in flight)
+                    wait_vmem_upto<OverlapRing::EARLY_OPS>();
+                    barrier_copies_in_flight();
+                    ring = (ring + 1) & 3;
+                } else {
+                    wait_vmem();
+                    __syncthreads();
                 }
             }
         }
+    };
+    uint32_t p = 0;
+    for (uint32_t i = 0; i + 1 < L; i++) {
+        if (TWICE && p) row(std::integral_constant<uint32_t, 1>{}, p, i);
+        else row(std::integral_constant<uint32_t, 0>{}, p, i);
+        // the next row's first chunk follows this row's last
+        p = (p + nchunk + ((i + 2) >> 5)) & 1;
     }
     // copies issued past the last unit
     if constexpr (OVL) wait_vmem();
+    store_energies<KW, S, (PF <= 4)>(acc, E, wfirst, lane, nseq);
+}
+
+// Rows staged `nrow` at a time (all chunks of a row, NPC KB each; of the first
+// row's chunks those before its diagonal are not read), one barrier per stage.
+template <int KW, int S, int NWAVES, int NPC>
+__global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_energies_rows(
+    const float* __restrict__ Ju, const uint8_t* __restrict__ seq, float* __restrict__ E,
+    uint32_t ldseq, uint32_t nseq, uint32_t L, uint32_t q, uint32_t nchunk, uint32_t nrow) {
+    constexpr int K = 4 * KW;
+    constexpr uint32_t SLOT = NPC * 1024, chb = 8192;
+    extern __shared__ f4v lds4[];
+    char* ldsb = reinterpret_cast<char*>(lds4);
+    const int tid = threadIdx.x;
+    const uint32_t lane = tid & 63;
+    const uint32_t j = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wfirst = blockIdx.x * (2 * S * NWAVES) + (wave * 2 + (lane >> 5)) * S;
+    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * nchunk * chb);
+    const uint32_t voff = lane * 16;
+    const uint32_t rowb = nchunk * SLOT, stageb = nrow * rowb;
+    const uint32_t npc = (q * q + 7) / 8, rp = nchunk * npc;
+    const uint32_t inv = 65536 / npc + 1;     // r / npc for r < 256
+    auto copy_stage = [&](uint32_t i0, uint32_t buf) {
+        const uint32_t n = L - 1 - i0 < nrow ? L - 1 - i0 : nrow;
+        uint32_t g = 0, r = wave;
+        while (r >= rp) {
+            r -= rp;
+            g++;
+        }
+        while (g < n) {
+            const uint32_t k = (r * inv) >> 16, piece = r - k * npc;
+            if (k >= (i0 + g + 1) >> 5)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rJ, (lds_void*)(ldsb + buf * stageb + g * rowb + k * SLOT + piece * 1024), 16,
+                    voff, ((i0 + g) * nchunk + k) * chb + piece * 1024, 0, 0);
+            r += NWAVES;
+            while (r >= rp) {
+                r -= rp;
+                g++;
+            }
+        }
+    };
+    Walkers<KW, S, true> w;
+    w.load(seq, ldseq, L, wfirst, lane, nseq);
+    float acc[S];
 #pragma unroll
-    for (int s = 0; s < S; s++) {
-        float e = half_wave_sum(acc[s]);
-        if (j == 0 && wfirst + s < nseq) E[wfirst + s] = e;
+    for (int s = 0; s < S; s++) acc[s] = 0.f;
+    uint32_t base[S];
+    copy_stage(0, 0);
+    wait_vmem();
+    __syncthreads();
+    uint32_t buf = 0;
+    for (uint32_t i0 = 0; i0 + 1 < L; i0 += nrow) {
+        if (i0 + nrow + 1 < L) copy_stage(i0 + nrow, buf ^ 1);
+        const uint32_t i1 = i0 + nrow < L - 1 ? i0 + nrow : L - 1;
+        uint32_t origin = j * 4 + buf * stageb;
+        for (uint32_t i = i0; i < i1; i++) {
+            const uint32_t kp = i >> 5, c0 = (i + 1) >> 5;
+            w.row_bases(i, lane, q, origin, base);
+            const float keep = (c0 != kp || j > (i & 31)) ? 1.f : 0.f;
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                if ((uint32_t)k < c0 || (uint32_t)k >= nchunk) continue;
+                if constexpr (KW <= 2) {
+                    if ((uint32_t)k == c0)
+                        energy_chunk<true>(w, k, ldsb + k * SLOT, base, keep, acc);
+                    else
+                        energy_chunk<false>(w, k, ldsb + k * SLOT, base, keep, acc);
+                } else {
+                    energy_chunk<true>(w, k, ldsb + k * SLOT, base,
+                                       (uint32_t)k == c0 ? keep : 1.f, acc);
+                }
+            }
+            origin += rowb;
+        }
+        wait_vmem();
+        __syncthreads();
+        buf ^= 1;
     }
+    store_energies<KW, S, true>(acc, E, wfirst, lane, nseq);
+}
+
+// No staging: one wave per work-group, ROWS neighbouring rows at a time (of one
+// chunk, so that they share its partners), all their gathers of a chunk in
+// flight.  Lanes whose partner does not count read the row all the same.
+template <int NC>
+__global__ __launch_bounds__(64) void k_energies_direct(
+    const float* __restrict__ Ju, const uint8_t* __restrict__ seq, float* __restrict__ E,
+    uint32_t ldseq, uint32_t nseq, uint32_t L, uint32_t q, uint32_t chb) {
+    constexpr int KW = (NC + 3) / 4, S = 1, ROWS = 4;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t j = lane & 31;
+    const uint32_t wfirst = blockIdx.x * 2 + (lane >> 5);
+    const __amdgpu_buffer_rsrc_t rJ = make_rsrc(Ju, L * NC * chb);
+    Walkers<KW, S, false> w;
+    w.load(seq, ldseq, L, wfirst, lane, nseq);
+    float acc[1] = {0.f};
+    for (uint32_t i0 = 0; i0 + 1 < L; i0 += ROWS) {
+        const uint32_t kp = i0 >> 5;
+        uint32_t base[ROWS][S];
+        float keep[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            // rows past the last repeat it and count nothing
+            const uint32_t i = i0 + r + 1 < L ? i0 + r : L - 2;
+            w.row_bases(i, lane, q, j * 4 + i * NC * chb, base[r]);
+            keep[r] = i == i0 + r ? 1.f : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < NC; k++) {
+            if ((uint32_t)k < kp) continue;
+            float v[ROWS];
+#pragma unroll
+            for (int r = 0; r < ROWS; r++)
+                v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    rJ, base[r][0] + byte_x128(w.st[0][k >> 2], k & 3), k * chb, 0));
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                const float f = (uint32_t)k != kp || j > ((i0 + r) & 31) ? keep[r] : 0.f;
+                acc[0] = __fmaf_rn(v[r], f, acc[0]);
+            }
+        }
+    }
+    store_energies<KW, S, false>(acc, E, wfirst, lane, nseq);
 }
 
 }  // namespace mi3

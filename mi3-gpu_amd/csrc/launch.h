@@ -21,6 +21,7 @@ struct EnergyArgs {
     const uint8_t* seq;
     float* E;
     uint32_t ld, nseq, L, q, nchunk;
+    uint32_t ncu;  // compute units of the device
 };
 
 // The walker count must be a multiple of 512.
@@ -70,13 +71,31 @@ struct BatchTile {
     uint32_t model, block;
 };
 
-// Largest walker count that is swept without staging (sweep_direct): its
-// time grows with the walkers from the start, a staged tile's only once the
-// CUs are full.  The two meet near 32 walkers a CU for q > 8 (8192 walkers:
-// 6.7 against 7.0 us a step at L=232 q=21, 2.6 against 2.7 at L=93) and
-// near 24 for the cheaper rows of q <= 8 (L=93 q=4: 4096 walkers 0.56 against
-// 0.82, 16384 walkers 1.7 against 0.97).
-inline uint32_t direct_walkers(uint32_t q, uint32_t ncu) { return (q <= 8 ? 24 : 32) * ncu; }
+// Largest walker count that is swept without staging (sweep_direct).  Alone on
+// the card it is the fastest form up to some 32 walkers a CU, but its time
+// grows with the walkers from the start, and with the work of other streams
+// beside it, where a staged tile leaves their CUs alone; the line lies where
+// three contexts sweeping at once lose nothing either (us a step and context,
+// three at once / one alone, unstaged against the staged form taken instead:
+// L=93 q=21, 2048 walkers 0.95 / 0.77 against 0.95 / 2.7, 4096 1.9 / 1.3 against
+// 0.95 / 2.7; L=232 q=21, 1024 walkers 2.1 / 1.2 against 2.5 / 7.0; L=93 q=4, 2048
+// walkers 0.22 / 0.50 against 0.32 / 0.85, 4096 0.41 / 0.55 against 0.32 / 0.85).
+inline uint32_t direct_walkers(uint32_t q, uint32_t ncu) { return (q <= 8 ? 12 : 6) * ncu; }
+
+// Largest sequence count whose energies are taken without staging, by the same
+// measure (us, three contexts at once / one alone: L=232 q=21, 2048 sequences 187 /
+// 163 against 324 / 960, 4096 770 / 266 against 321 / 950; L=93 q=4, 4096 sequences
+// 14 / 17 against 18 / 48, 8192 27 / 32 against 19 / 48).
+inline uint32_t direct_sequences(uint32_t q, uint32_t ncu) { return (q <= 8 ? 16 : 8) * ncu; }
+
+// Walkers (or sequences) per work-group of the chunk-staged kernels, `most` or
+// less: half as many take 0.7-0.97 of the time, on twice the CUs, so tiles are
+// halved only while they occupy at most a quarter of the card.
+inline uint32_t chunk_tile(uint32_t n, uint32_t most, uint32_t ncu) {
+    uint32_t w = most;
+    while (w > 128 && (n + w / 2 - 1) / (w / 2) <= ncu / 4) w /= 2;
+    return w;
+}
 
 // LDS per chunk in the step-staged sweep, in KB (2 for q <= 4, 8 for q <= 8),
 // or 0 where a row of couplings does not fit 64 KB and the form does not
@@ -92,6 +111,10 @@ hipError_t launch_sweep_steps(const SweepArgs& a, hipStream_t st);
 template <int KW>
 hipError_t launch_sweep_chunks(const SweepArgs& a, hipStream_t st);
 hipError_t launch_sweep(const SweepArgs& a, hipStream_t st);
+hipError_t launch_energies_direct(const EnergyArgs& a, hipStream_t st);
+hipError_t launch_energies_rows(const EnergyArgs& a, hipStream_t st);
+template <int KW>
+hipError_t launch_energies_chunks(const EnergyArgs& a, hipStream_t st);
 hipError_t launch_energies(const EnergyArgs& a, hipStream_t st);
 
 // The sweep's coupling-row staging alone (k_stage_probe) for the sites of
@@ -124,6 +147,8 @@ hipError_t launch_unpack_chunked(const float* J, float* out, uint32_t L, uint32_
                                  uint32_t nchunk, hipStream_t st);
 
 #define MI3_DECL_KW(KW)                                                                       \
+    template <>                                                                               \
+    hipError_t launch_energies_chunks<KW>(const EnergyArgs& a, hipStream_t st);                \
     template <>                                                                               \
     hipError_t launch_sweep_chunks<KW>(const SweepArgs& a, hipStream_t st);                    \
     template <>                                                                               \

@@ -791,6 +791,7 @@ int mi3_calc_energies(mi3_ctx* c, const char* seqbuf, const char* Jbuf, const ch
     a.L = c->L;
     a.q = c->q;
     a.nchunk = c->nchunk;
+    a.ncu = c->ncu;
     Scope s(c, "getEnergies", (size_t)nseq * (c->L + 4));
     HIPCHK(c, launch_energies(a, c->stream));
     eb->version++;

@@ -30,24 +30,14 @@ hipError_t sweep_kws(const SweepArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Tile of the chunk-staged sweep.  128 and 256 walkers are as the caller
-// asked.  At the default (512) the smaller of two tiles is taken where it
-// needs no more rounds of work-groups over the CUs: a step costs a tile of
-// 128, 256 or 512 walkers 7.0, 7.5 and 9.1 us at L=232 q=21 (2.7, 2.9 and
-// 3.9 us at L=93), so halving the tile pays only while the card has CUs to
-// spare.
-inline uint32_t chunk_tile(const SweepArgs& a) {
-    if (a.wpb == 128 || a.wpb == 256) return a.wpb;
-    auto rounds = [&](uint32_t w) { return (a.nwalk / w + a.ncu - 1) / a.ncu; };
-    uint32_t w = 512;
-    while (w > 128 && rounds(w / 2) == rounds(w)) w /= 2;
-    return w;
-}
-
 template <int KW, int PF>
 struct SweepDisp {
     static hipError_t run(const SweepArgs& a, hipStream_t st) {
-        const uint32_t w = chunk_tile(a);
+        // 128 and 256 walkers as the caller asked; at the default by the rule
+        // (a step of 128, 256 or 512 walkers: 7.0, 7.2 and 8.2 us at L=232 q=21, 2.7,
+        // 2.9 and 3.8 us at L=93)
+        const uint32_t w =
+            (a.wpb == 128 || a.wpb == 256) ? a.wpb : chunk_tile(a.nwalk, 512, a.ncu);
         if constexpr (KW >= 5) {
             // five to eight state words: 8 slots at most fit in 128 registers
             if (w <= 128) return sweep_kws<KW, PF, 4, 16>(a, st);

@@ -21,21 +21,24 @@ hipError_t run_shape(const SweepArgs& a, hipStream_t st, uint32_t stage_kb) {
     return hipGetLastError();
 }
 
-// Shape (slots x waves) by how many walkers a CU gets; us per step at q=4:
-//   up to 64:  4 x 4 (32 walkers a work-group): L=93, 16384 walkers 0.97, against
-//              1.15 for 8 x 4, 1.75 for 16 x 4 and 3.65 chunk-staged
-//   up to 256: 8 x 8: 65536 walkers 1.98, against 2.17 for 16 x 8
-//   beyond:    16 x 8 for up to two state words: 2^18 walkers 6.5 at L=93 and
-//              13.4 at L=232, against 7.5 and 16.1 chunk-staged; 8 slots for longer
-//              chains (22.8 against 24.8 at L=300).
+// Shape (slots x waves) by how many walkers a CU gets (us a step, three contexts
+// at once / one alone):
+//   up to 64 (32 for q > 4): 4 x 4, 32 walkers a work-group: L=93 q=4, 16384 walkers
+//              0.54 / 1.0, 0.54 / 1.2 for 8 x 8, 1.2 / 3.7 chunk-staged; at q=8
+//              0.97 / 1.5, so 8 x 8 there (0.67 / 1.5)
+//   up to 128: 8 x 8: 32768 walkers 0.81 / 1.3, 0.96 / 2.1 for 16 x 8
+//   beyond:    16 x 8 for up to two state words: 65536 walkers 1.43 / 2.3, 1.64 / 2.1
+//              for 8 x 8; 2^18 alone 5.6 at L=93 and 13.4 at L=232, against 7.2 and
+//              16.1 chunk-staged; 8 slots for longer chains (22.8 against 24.8 at
+//              L=300)
 // Two work-groups of 8 waves share a CU while their stages fit beside each
 // other; longer rows take 16 waves.
 template <int KW, int NPC>
 hipError_t run_kw(const SweepArgs& a, hipStream_t st) {
     const bool wide = 4ull * a.nchunk * NPC * 1024 > 163840;
-    if (a.nwalk <= 64 * a.ncu) return run_shape<KW, 4, 4, NPC>(a, st, 16);
+    if (a.nwalk <= (NPC == 2 ? 64 : 32) * a.ncu) return run_shape<KW, 4, 4, NPC>(a, st, 16);
     if constexpr (KW <= 2) {
-        if (a.nwalk > 256 * a.ncu)
+        if (a.nwalk > 128 * a.ncu)
             return wide ? run_shape<KW, 16, 16, NPC>(a, st, 64) : run_shape<KW, 16, 8, NPC>(a, st, 32);
     }
     return wide ? run_shape<KW, 8, 16, NPC>(a, st, 64) : run_shape<KW, 8, 8, NPC>(a, st, 32);

@@ -11,10 +11,10 @@ pytestmark = pytest.mark.gpu
 
 # (L, q, walkers, steps): lengths at the edges of chunks (32), state words
 # (128) and staged rows; walker counts at the edges of the forms and tiles of a
-# 256-CU card (unstaged up to 6144 or 8192; then 16384, 65536)
-CASES = [(2, 2, 512, 7), (32, 4, 512, 41), (33, 25, 1024, 33), (129, 3, 2048, 20), (160, 21, 2560, 17),
-         (97, 9, 8192, 12), (1024, 4, 512, 9),                      # unstaged
-         (31, 2, 6656, 65), (93, 8, 8704, 30), (256, 6, 16384, 9), (385, 4, 6656, 11),
+# 256-CU card
+CASES = [(2, 2, 512, 7), (32, 4, 512, 41), (33, 25, 1024, 33), (129, 3, 3072, 20), (160, 21, 1536, 17),
+         (97, 9, 1024, 12), (1024, 4, 512, 9),                      # unstaged
+         (160, 21, 2048, 17), (31, 2, 3584, 65), (93, 8, 8192, 30), (93, 8, 8704, 30), (256, 6, 16384, 9), (385, 4, 6656, 11),
          (33, 4, 16896, 37), (225, 8, 66048, 6), (128, 7, 66048, 9), (300, 3, 66048, 5),
          (1000, 4, 16896, 5),                                       # steps staged
          (65, 9, 8704, 21), (300, 5, 8704, 9), (40, 21, 66048, 12), (70, 16, 131584, 6),
