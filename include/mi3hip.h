@@ -202,8 +202,10 @@ int mi3_calc_energies(mi3_ctx *ctx, const char *seqbuf, const char *Jbuf, const 
  * (mcmc.cl:464-516). */
 int mi3_calc_bicounts(mi3_ctx *ctx, const char *seqbuf, uint32_t nseq);
 
-/* Number of parts mi3_calc_bicounts splits nseq sequences into (partial
- * counts of the parts are added with integer atomics when it is above 1).
+/* Number of parts that mi3_calc_bicounts plans for nseq sequences: with 1, a wave
+ * counts all sequences for its block of the table; above 1, blocks are shared
+ * by at most that many waves and one more, whose counts are added with integer
+ * atomics.
  * A query of the launch plan behind calcBicounts (mcmcGPU.py:501-518); the
  * reference's countBivariate has no split (mcmc.cl:464-516). */
 int mi3_bicount_split(mi3_ctx *ctx, uint32_t nseq, uint32_t *ksplit);

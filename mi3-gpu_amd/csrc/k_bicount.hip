@@ -1,15 +1,16 @@
-// Bimarginal counts as an int8 one-hot Gram product on the matrix cores.
+// Bimarginal counts as a one-hot Gram product on the matrix cores, in 4-bit
+// floats.
 //
 // With X[n][r] = [s_{n, r/q} == r % q] (N x L*q, one-hot, never stored),
 // count_{ij}(a, b) = (X^T X)[i*q + a][j*q + b] for i < j.  Each wave owns a
-// 128 x 128 block of the flattened L*q x L*q Gram matrix (4 x 4 tiles of
-// v_mfma_i32_32x32x32_i8), builds its int8 operands on the fly from the
-// site-major residue bytes (16 sequences per lane per k-step, read from an
-// LDS copy of the block's sites that LDS DMA refills 4 to 16 k-steps at a
-// time, one load per site and 16 bytes instead of one per row), contracts
-// over its range of sequences with int32 accumulation, and scatters the
-// i < j entries into the packed (L(L-1)/2, q*q) uint32 table.  Integer accumulation makes
-// the result exact whatever the summation order.
+// T x T block of the flattened L*q x L*q Gram matrix (tiles of
+// v_mfma_scale_f32_32x32x64_f8f6f4 with e2m1 operands, twice the rate of the
+// 8-bit ones), builds its operands on the fly from residues packed to bit
+// planes (32 sequences per lane per k-step of 64), contracts over its range of
+// sequences and scatters the i < j entries into the packed (L(L-1)/2, q*q)
+// uint32 table.  Every product is 0 or 1 and a wave sums at most 2^23 sequences
+// before it stores, so the float32 sums are exact integers and the result does
+// not depend on the order of any addition.
 // Replaces countBivariate (mcmc.cl:464-516); matches np.bincount per pair
 // (getMarginals.py:80-86).
 #include "common.h"
@@ -17,83 +18,69 @@
 namespace mi3 {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
-// bytes of `v` equal to `a` -> 0x01, others -> 0x00
-__device__ __forceinline__ uint32_t eq_bytes(uint32_t v, uint32_t a4) {
-    uint32_t x = v ^ a4;
-    uint32_t t = ((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x;
-    return (~t & 0x80808080u) >> 7;
-}
-
-// One-hot operand of row r (site r/q, residue r%q) for 16 sequences
-// starting at n: 16 int8 values in 4 dwords.
-__device__ __forceinline__ v4i onehot16(const uint8_t* __restrict__ seq, uint32_t ldseq,
-                                        uint32_t site, uint32_t a4, bool valid, uint32_t n,
-                                        uint32_t nseq) {
-    v4i r = {0, 0, 0, 0};
-    if (valid) {
-        const uint8_t* p = seq + (size_t)site * ldseq + n;
-        uint4 v;
-        if (n + 16 <= nseq) {
-            v = *reinterpret_cast<const uint4*>(p);
-            r[0] = (int)eq_bytes(v.x, a4);
-            r[1] = (int)eq_bytes(v.y, a4);
-            r[2] = (int)eq_bytes(v.z, a4);
-            r[3] = (int)eq_bytes(v.w, a4);
-        } else {
-            // ragged tail: bytes past nseq contribute nothing
-            uint32_t w[4] = {0, 0, 0, 0};
-            for (uint32_t e = 0; e < 16; e++) {
-                if (n + e < nseq && p[e] == (uint8_t)(a4 & 0xff)) w[e >> 2] |= 1u << (8 * (e & 3));
-            }
-            r[0] = (int)w[0]; r[1] = (int)w[1]; r[2] = (int)w[2]; r[3] = (int)w[3];
+// Residues packed for the operands: bit planes.  A unit is 128 sequences of a
+// site in 16 * PL consecutive bytes, [plane][half] of 64 bits; a lane's 32
+// sequences of the unit's first k-step are the low word of its half, those of
+// the second the high word.
+//   PL = 3 (q <= 7), PL = 5 (q <= 25).
+// A residue equals a letter where every plane agrees with the letter's bit: PL
+// instructions for 32 sequences.  Sequences past the end are all ones, which is
+// no residue.  The bits of a word are in the same order at every site, which is
+// all that a sum over sequences needs.
+template <int PL>
+__global__ __launch_bounds__(256) void k_pack_residues(const uint8_t* __restrict__ seq,
+                                                       uint32_t ldseq, uint32_t nseq,
+                                                       uint32_t nunits, uint8_t* __restrict__ out) {
+    // thread: 64 sequences of a site
+    const uint32_t c = blockIdx.x * 256 + threadIdx.x, site = blockIdx.y;
+    if (c >= nunits * 2) return;
+    const uint4* row = reinterpret_cast<const uint4*>(seq + (size_t)site * ldseq);
+    uint32_t w[2][8];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) {
+        const uint32_t n = c * 64 + k * 16;
+        uint4 v = make_uint4(~0u, ~0u, ~0u, ~0u);
+        if (n < nseq) v = row[n / 16];   // rows are multiples of 16 bytes long
+        uint32_t x[4] = {v.x, v.y, v.z, v.w};
+        if (n < nseq && n + 16 > nseq) {
+#pragma unroll
+            for (uint32_t e = 0; e < 16; e++)
+                if (n + e >= nseq) x[e >> 2] |= 0xffu << (8 * (e & 3));
         }
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++) w[k >> 1][(k & 1) * 4 + e] = x[e];
     }
-    return r;
+    uint2* o = reinterpret_cast<uint2*>(out + ((size_t)site * nunits + (c >> 1)) * (16 * PL) +
+                                        (c & 1) * 8);
+#pragma unroll
+    for (int p = 0; p < PL; p++) {
+        uint32_t m[2] = {0u, 0u};
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) m[h] |= ((w[h][e] >> p) & 0x01010101u) << e;
+        o[2 * p] = make_uint2(m[0], m[1]);
+    }
 }
 
-// grid: ksplit waves per (row block rb, col block cb), rb <= cb, blocks of
-// 128 (256 int32 accumulators per lane, held in AGPRs), so every one-hot
-// operand built from a 16-byte load feeds 4 matrix instructions.  The
-// sequence range is split over the ksplit waves of a block, whose partial
-// counts are added with integer atomics (exact in any order; the table must
-// be zeroed first).  Residue bytes are loaded two k-steps ahead of use.
-//
-// Operands: row operands are -128 (0x80) where the residue matches, column
-// operands +1, so each co-occurrence adds -128 and count = -acc / 128
-// (|acc| <= 128 * nseq < 2^31 for nseq < 2^24).  With residues < 32 every
-// byte of x = v ^ a is below 0x80, so 0x80808080 - x borrows nothing across
-// bytes and its top bit per byte is set exactly where v == a; it is formed
-// in one v_xad_u32 as (v ^ ~a) + 0x80808081.  Rows past L*q compare against
-// 0x7f, which no residue equals.
-__device__ __forceinline__ uint32_t match_hi(uint32_t v, uint32_t na4) {
-    return (v ^ na4) + 0x80808081u;
+// Staging: STAGE units of the sites that a block's rows and columns touch (at
+// most T/q + 2 each), double-buffered; one LDS DMA instruction moves 16 bytes
+// per lane.  An odd number of 16-byte pieces per site keeps the sites that one
+// read touches (at most 17) in different banks.  The host takes the longer stage
+// (5 units, else 3) whose buffers fit 40 KiB, so that four waves share a CU.
+constexpr uint32_t BC_PLANES_Q = 7;   // largest q of three planes
+constexpr uint32_t BC_UNIT = 128;     // sequences
+constexpr uint32_t BC_PART = 65536;   // most units that a wave sums in float32 (2^23 sequences)
+inline uint32_t bc_planes(uint32_t q) { return q <= BC_PLANES_Q ? 3 : 5; }
+inline size_t bc_lds_bytes(uint32_t q, uint32_t tile, uint32_t stage) {
+    const uint32_t sites = 2 * (tile / q + 2);
+    return 2ull * ((sites * bc_planes(q) * stage + 63) / 64) * 1024;
 }
-
-// Staging of residue bytes: STAGE k-steps (32 sequences each, so
-// SB = 32 * STAGE bytes per site) of the sites a block's 128 rows and 128
-// columns touch (at most 128/q + 2 each), double-buffered.  One LDS DMA
-// instruction moves 16 bytes per lane, i.e. SPI = 1024 / SB sites.  Longer
-// stages wait less often on their copies (16 k-steps: 10.9 ms, 8: 11.1,
-// 4: 11.5, 2: 12.4 at 2^20 sequences, L=232 q=21); the host takes the
-// longest whose double buffer fits 40 KiB, so that four waves share a CU.
-template <uint32_t STAGE>
-struct BcStage {
-    static constexpr uint32_t SB = 32 * STAGE;
-    static constexpr uint32_t LPS = SB / 16;   // lanes per site
-    static constexpr uint32_t SPI = 64 / LPS;  // sites per instruction
-    static_assert(SPI >= 1 && SPI * LPS == 64, "stage size");
-};
-inline uint32_t bc_max_sites(uint32_t q) { return 128 / q + 2; }
-inline size_t bc_lds_bytes(uint32_t q, uint32_t stage) {
-    const uint32_t spi = 32 / stage;
-    return 2ull * ((2 * bc_max_sites(q) + spi - 1) / spi) * 1024;
-}
-inline uint32_t bc_stage_for(uint32_t q) {
-    for (uint32_t st : {16u, 8u})
-        if (bc_lds_bytes(q, st) <= 40960) return st;
-    return 4;
+inline uint32_t bc_stage_for(uint32_t q, uint32_t tile) {
+    return bc_lds_bytes(q, tile, 5) <= 40960 ? 5 : 3;
 }
 typedef __attribute__((address_space(3))) void bc_lds_void;
 
@@ -101,179 +88,222 @@ typedef __attribute__((address_space(3))) void bc_lds_void;
 // included, has completed.
 __device__ __forceinline__ void wait_vmem_bc() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-template <uint32_t STAGE>
-__global__ __launch_bounds__(64) void k_bicounts_mfma128(const uint8_t* __restrict__ seq,
-                                                         uint32_t ldseq, uint32_t nseq,
-                                                         uint32_t L, uint32_t q, uint32_t nblk,
-                                                         uint32_t ksplit,
-                                                         uint32_t* __restrict__ counts) {
+// The work is `total` units: the blocks (rb, cb), rb <= cb, of T = 32 * NT rows and
+// columns, nunits units each, in one sequence that the waves of the grid divide
+// evenly, so that all SIMDs end together however many blocks there are.  A
+// wave that holds the whole of a block stores its counts; the parts of a shared
+// block are added with integer atomics (exact in any order; the table must be
+// zeroed first).  NT = 4 keeps 256 sums per lane in AGPRs, one wave to a SIMD;
+// NT = 2 is for problems too small for that (rule at the launch).
+//
+// Bound by the matrix instructions (16 products of a k-step; with the operands
+// held fixed, the products alone take 1.36 ms of the 1.52 ms at 2^18 sequences,
+// L=232 q=21), as long as the one wave a SIMD holds issues the building of the
+// operands between the products, and reads little of LDS: a k-step's 8 operands
+// take 20 eight-byte reads of 2.6 cycles a CU and 88 other instructions.  Measured
+// (us; 8-bit one-hot products built from bytes, 4-bit ones from nibbles, and
+// this form with a fixed number of parts per block and with even shares):
+//   L    q   sequences   8-bit  nibbles  planes  even shares
+//   232  21  1000003     10653     7020    5595         5533
+//   232  21  262144       3103     2063    1661         1525
+//   232  21  16384         459      400     378          207
+//   150  12  100001        434      377     367          202
+//   93   4   262144        163       84      70           70
+//   99   4   16384          70       26      25           25
+template <int NT, int PL, int STAGE>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
+    const uint8_t* __restrict__ pk, uint32_t nunits, uint32_t L, uint32_t q, uint32_t nblk,
+    uint64_t total, uint32_t* __restrict__ counts) {
     extern __shared__ __attribute__((aligned(16))) uint8_t bc_lds[];
-    constexpr uint32_t BC_STAGE = STAGE, BC_SB = BcStage<STAGE>::SB,
-                       BC_LPS = BcStage<STAGE>::LPS, BC_SPI = BcStage<STAGE>::SPI;
-    uint32_t t = blockIdx.x / ksplit;
-    const uint32_t part = blockIdx.x - t * ksplit;
-    uint32_t rb = 0;
-    while (t >= nblk - rb) {
-        t -= nblk - rb;
-        rb++;
-    }
-    const uint32_t cb = rb + t;
+    constexpr uint32_t T = 32 * NT;
+    constexpr uint32_t KB = 16 * PL;          // bytes of a site's unit
+    constexpr uint32_t LPS = PL * STAGE;      // 16-byte pieces of a site's stage
+    constexpr uint32_t SB = 16 * LPS;
+    static_assert(LPS % 2 == 1, "sites in different banks");
     const uint32_t l = threadIdx.x;
     const uint32_t lr = l & 31, g = l >> 5;
     const uint32_t Lq = L * q;
-    // sequence range of this part, in steps of 32
-    const uint32_t nsteps = (nseq + 31) / 32;
-    const uint32_t s0 = (uint32_t)(((uint64_t)nsteps * part) / ksplit);
-    const uint32_t s1 = (uint32_t)(((uint64_t)nsteps * (part + 1)) / ksplit);
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(seq), (short)0,
-                                          (int)(ldseq * L), 0x00020000);
-
-    // the sites of this block's rows (A) and columns (B), staged as
-    // [A sites..., B sites...] x BC_SB bytes per buffer
-    const uint32_t rA0 = rb * 128, rA1 = (rA0 + 127 < Lq) ? rA0 + 127 : Lq - 1;
-    const uint32_t cB0 = cb * 128, cB1 = (cB0 + 127 < Lq) ? cB0 + 127 : Lq - 1;
-    const uint32_t siA0 = rA0 / q, nsA = rA1 / q - siA0 + 1;
-    const uint32_t siB0 = cB0 / q, nsB = cB1 / q - siB0 + 1;
-    const uint32_t ninst = (nsA + nsB + BC_SPI - 1) / BC_SPI;
-    const uint32_t bufbytes = ninst * 1024;
-
-    uint32_t ldsA[4], a4A[4], naA[4], siteA[4], ldsB[4], a4B[4], naB[4], siteB[4];
-#pragma unroll
-    for (int x = 0; x < 4; x++) {
-        const uint32_t r = rA0 + x * 32 + lr;
-        const uint32_t si = r < Lq ? r / q : siA0;
-        siteA[x] = si;
-        a4A[x] = r < Lq ? (r - si * q) * 0x01010101u : 0x7f7f7f7fu;
-        naA[x] = ~a4A[x];
-        ldsA[x] = (si - siA0) * BC_SB + 16 * g;
-        const uint32_t c = cB0 + x * 32 + lr;
-        const uint32_t sj = c < Lq ? c / q : siB0;
-        siteB[x] = sj;
-        a4B[x] = c < Lq ? (c - sj * q) * 0x01010101u : 0x7f7f7f7fu;
-        naB[x] = ~a4B[x];
-        ldsB[x] = (nsA + sj - siB0) * BC_SB + 16 * g;
-    }
-    v16i acc[4][4];
-#pragma unroll
-    for (int x = 0; x < 4; x++)
-#pragma unroll
-        for (int y = 0; y < 4; y++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[x][y][e] = 0;
-
-    // LDS DMA of one stage: instruction k moves sites BC_SPI*k onward (lane
-    // l: site BC_SPI*k + l/BC_LPS, 16-byte piece l%BC_LPS of the stage's
-    // 32*BC_STAGE sequences);
-    // slots past the block's sites load a valid site that nothing reads.
-    // The last stage of a range can reach past the last step (and, for the
-    // last site, past the buffer): such pieces are never read, and their
-    // source offsets are clamped into the buffer.
-    const uint32_t last16 = ldseq * L - 16;
-    auto stage = [&](uint32_t buf, uint32_t step) {
-        const uint32_t n0 = step * 32;
-        for (uint32_t k = 0; k < ninst; k++) {
-            const uint32_t ts = BC_SPI * k + l / BC_LPS;
-            const uint32_t site = ts < nsA ? siA0 + ts : (ts < nsA + nsB ? siB0 + (ts - nsA) : siA0);
-            const uint32_t off = site * ldseq + n0 + 16 * (l % BC_LPS);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rs, (bc_lds_void*)(bc_lds + buf * bufbytes + k * 1024), 16,
-                off < last16 ? off : last16, 0, 0, 0);
+    const uint32_t ldp = nunits * KB;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(pk), (short)0, (int)(ldp * L), 0x00020000);
+    const uint64_t end = total * (blockIdx.x + 1) / gridDim.x;
+    for (uint64_t cur = total * blockIdx.x / gridDim.x; cur < end;) {
+        // units [u0, u1) of block t
+        uint32_t t = (uint32_t)(cur / nunits);
+        const uint32_t u0 = (uint32_t)(cur - (uint64_t)t * nunits);
+        uint32_t u1 = u0 + BC_PART < nunits ? u0 + BC_PART : nunits;
+        if (end - cur < u1 - u0) u1 = u0 + (uint32_t)(end - cur);
+        cur += u1 - u0;
+        uint32_t rb = 0;
+        while (t >= nblk - rb) {
+            t -= nblk - rb;
+            rb++;
         }
-    };
-    auto operands = [&](const uint8_t* sbase, uint32_t ks, v4i (&A)[4], v4i (&B)[4]) {
-        v4i ra[4], rbv[4];
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            ra[x] = *reinterpret_cast<const v4i*>(sbase + ldsA[x] + 32 * ks);
-            rbv[x] = *reinterpret_cast<const v4i*>(sbase + ldsB[x] + 32 * ks);
+        const uint32_t cb = rb + t;
+
+        // the sites of this block's rows (A) and columns (B), staged as
+        // [A sites..., B sites...] x SB bytes per buffer
+        const uint32_t rA0 = rb * T, rA1 = (rA0 + T - 1 < Lq) ? rA0 + T - 1 : Lq - 1;
+        const uint32_t cB0 = cb * T, cB1 = (cB0 + T - 1 < Lq) ? cB0 + T - 1 : Lq - 1;
+        const uint32_t siA0 = rA0 / q, nsA = rA1 / q - siA0 + 1;
+        const uint32_t siB0 = cB0 / q, nsB = cB1 / q - siB0 + 1;
+        const uint32_t ninst = ((nsA + nsB) * LPS + 63) / 64;
+        const uint32_t bufbytes = ninst * 1024;
+
+        // per operand: LDS address of this lane's words, and the letter's bits as masks
+        // (rows past L*q count the first row's site again and are not stored)
+        uint32_t at[2 * NT], let[2 * NT][PL];
+        auto operand = [&](int w, uint32_t r, uint32_t first, uint32_t slot0) {
+            const uint32_t si = r < Lq ? r / q : first;
+            const uint32_t a = r < Lq ? r - si * q : 0u;
+            at[w] = (slot0 + si - first) * SB + g * 8;
+    #pragma unroll
+            for (int p = 0; p < PL; p++) let[w][p] = 0u - ((a >> p) & 1u);
+        };
+    #pragma unroll
+        for (int x = 0; x < NT; x++) {
+            operand(x, rA0 + x * 32 + lr, siA0, 0);
+            operand(NT + x, cB0 + x * 32 + lr, siB0, nsA);
         }
-#pragma unroll
-        for (int x = 0; x < 4; x++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                A[x][e] = (int)(match_hi((uint32_t)ra[x][e], naA[x]) & 0x80808080u);
-                B[x][e] = (int)((match_hi((uint32_t)rbv[x][e], naB[x]) >> 7) & 0x01010101u);
+        v16f acc[NT][NT];
+    #pragma unroll
+        for (int x = 0; x < NT; x++)
+    #pragma unroll
+            for (int y = 0; y < NT; y++)
+    #pragma unroll
+                for (int e = 0; e < 16; e++) acc[x][y][e] = 0.f;
+
+        // LDS DMA of one stage: piece P is piece P % LPS of site P / LPS; pieces past
+        // the block's sites load a valid site that nothing reads.  The last stage of a
+        // range can reach past the last unit (and, for the last site, past the
+        // buffer): such pieces are never counted, and their source offsets are clamped
+        // into the buffer.
+        const uint32_t last16 = ldp * L - 16;
+        auto stage = [&](uint32_t buf, uint32_t unit) {
+            for (uint32_t k = 0; k < ninst; k++) {
+                const uint32_t ts = (64 * k + l) / LPS, piece = (64 * k + l) - ts * LPS;
+                const uint32_t site =
+                    ts < nsA ? siA0 + ts : (ts < nsA + nsB ? siB0 + (ts - nsA) : siA0);
+                const uint32_t off = site * ldp + unit * KB + 16 * piece;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rs, (bc_lds_void*)(bc_lds + buf * bufbytes + k * 1024), 16,
+                    off < last16 ? off : last16, 0, 0, 0);
             }
-    };
-    auto products = [&](const v4i (&A)[4], const v4i (&B)[4]) {
-#pragma unroll
-        for (int x = 0; x < 4; x++)
-#pragma unroll
-            for (int y = 0; y < 4; y++)
-                acc[x][y] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[x], B[y], acc[x][y], 0, 0, 0);
-    };
-    // full steps (all 32 sequences < nseq), staged BC_STAGE steps at a time
-    // one stage ahead; the ragged last step, if any, goes byte by byte
-    const uint32_t full_end = nseq / 32;
-    const uint32_t e1 = s1 < full_end ? s1 : full_end;
-    if (s0 < e1) {
-        stage(0, s0);
-        uint32_t buf = 0;
-        for (uint32_t st0 = s0; st0 < e1; st0 += BC_STAGE) {
-            wait_vmem_bc();
-            __syncthreads();   // this stage's bytes are in LDS
-            if (st0 + BC_STAGE < e1) stage(buf ^ 1, st0 + BC_STAGE);
-            const uint8_t* sbase = bc_lds + buf * bufbytes;
-            // one step at a time (a guard per step also keeps the compiler
-            // from hoisting all the stage's LDS reads, which would spill)
-#pragma unroll
-            for (uint32_t ks = 0; ks < BC_STAGE; ks++) {
-                if (st0 + ks < e1) {
-                    v4i A[4], B[4];
-                    operands(sbase, ks, A, B);
-                    products(A, B);
+        };
+        // operands: NT of rows, then NT of columns
+        struct Raw {
+            uint2 f[2 * NT][PL];
+        };
+        struct Ops {
+            v4i f[2 * NT];
+        };
+        auto read = [&](const uint8_t* unit, int w, Raw& r) __attribute__((always_inline)) {
+    #pragma unroll
+            for (int p = 0; p < PL; p++)
+                r.f[w][p] = *reinterpret_cast<const uint2*>(unit + at[w] + 16 * p);
+        };
+        // operand w of k-step h of the unit in r.  Bits 4n + e of the word of matches go to
+        // nibble n of operand word e.  As e2m1, nibbles 1, 2 and 4 are 0.5, 1 and 2: rows
+        // hold word e at (0.5, 1, 2, 2) and columns at (2, 1, 0.5, 0.5), so that each
+        // product is 1 and most words need no shift.
+        auto match = [&](const Raw& r, int w, int h, Ops& o) __attribute__((always_inline)) {
+            auto word = [&](int p) { return h ? r.f[w][p].y : r.f[w][p].x; };
+            uint32_t m = ~(word(0) ^ let[w][0]);
+    #pragma unroll
+            for (int p = 1; p < PL; p++)   // m & ~(word ^ letter)
+                m = (uint32_t)__builtin_amdgcn_bitop3_b32((int)m, (int)word(p), (int)let[w][p], 0x90);
+            if (w < NT)
+                o.f[w] = v4i{(int)(m & 0x11111111u), (int)(m & 0x22222222u), (int)(m & 0x44444444u),
+                             (int)((m >> 1) & 0x44444444u)};
+            else
+                o.f[w] = v4i{(int)((m << 2) & 0x44444444u), (int)(m & 0x22222222u),
+                             (int)((m >> 2) & 0x11111111u), (int)((m >> 3) & 0x11111111u)};
+            asm volatile("" : "+v"(o.f[w]));   // built here, not at its use
+        };
+        // the products of o, and between them the building of the operands `on` of the
+        // next k-step (step h of the unit in r); READ: the registers of r take the next
+        // unit's words as they come free.  Scheduling barriers and an empty asm at each
+        // operand keep this order: left to itself, or to scheduling groups, the compiler
+        // issues all products and then all the building.
+        auto step = [&](const Ops& o, Ops& on, Raw& r, int h, bool next,
+                        const uint8_t* unit) __attribute__((always_inline)) {
+    #pragma unroll
+            for (int i = 0; i < NT * NT; i++) {
+                const int x = i / NT, y = i % NT;
+                const v4i f = o.f[x], c = o.f[NT + y];
+                acc[x][y] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                    __builtin_shufflevector(f, f, 0, 1, 2, 3, -1, -1, -1, -1),
+                    __builtin_shufflevector(c, c, 0, 1, 2, 3, -1, -1, -1, -1), acc[x][y], 4, 4, 0,
+                    127, 0, 127);
+                if (NT == 2 || i % 2) {
+                    const int w = NT == 2 ? i : i / 2;
+                    match(r, w, h, on);
+                    if (next) read(unit, w, r);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        {
+            // entering a stage: its bytes have landed, and the reads of the stage before
+            // have completed, so its buffer takes the stage after
+            uint32_t buf = 1;
+            const uint8_t* sbase = bc_lds;
+            auto enter = [&](uint32_t u) __attribute__((always_inline)) {
+                wait_vmem_bc();
+                __syncthreads();
+                buf ^= 1;
+                sbase = bc_lds + buf * bufbytes;
+                if (u + STAGE < u1) stage(buf ^ 1, u + STAGE);
+            };
+            stage(0, u0);
+            enter(u0);
+            Raw r;
+            Ops o0, o1;
+    #pragma unroll
+            for (int w = 0; w < 2 * NT; w++) read(sbase, w, r);
+    #pragma unroll
+            for (int w = 0; w < 2 * NT; w++) match(r, w, 0, o0);
+            // the operands built from the unit past the end (bytes of the last stage's
+            // buffers) are not multiplied
+            uint32_t k = 0;   // unit of the stage
+            for (uint32_t u = u0; u < u1; u++) {
+                if (++k == STAGE) {
+                    k = 0;
+                    if (u + 1 < u1) enter(u + 1);
+                }
+                step(o0, o1, r, 1, true, sbase + k * KB);
+                step(o1, o0, r, 0, false, sbase);
+            }
+        }
+
+        const uint32_t qq = q * q;
+        // r / q as a product: r < 2^15 and r * q < 2^20, so 2^20 / q rounded up is exact
+        const uint32_t inv = ((1u << 20) + q - 1) / q;
+    #pragma unroll
+        for (int x = 0; x < NT; x++) {
+    #pragma unroll
+            for (int y = 0; y < NT; y++) {
+                const uint32_t c = cb * T + y * 32 + lr;
+                if (c >= Lq) continue;
+                const uint32_t jsite = (c * inv) >> 20, b = c - jsite * q;
+    #pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const uint32_t r = rb * T + x * 32 + 8 * (e / 4) + 4 * g + (e % 4);
+                    if (r >= Lq) continue;
+                    const uint32_t isite = (r * inv) >> 20, a = r - isite * q;
+                    if (isite < jsite) {
+                        const uint32_t cnt = (uint32_t)acc[x][y][e];
+                        uint32_t* dst = counts + (size_t)pair_index(isite, jsite, L) * qq + a * q + b;
+                        if (u1 - u0 == nunits)
+                            *dst = cnt;
+                        else
+                            atomicAdd(dst, cnt);
+                    }
                 }
             }
-            __syncthreads();   // reads of this buffer done before it is refilled
-            buf ^= 1;
         }
-    }
-    if (s1 > full_end && full_end >= s0) {
-        // ragged tail: the last, partial step of this part (bytes past nseq
-        // count for nothing)
-        const uint32_t n = full_end * 32 + 16 * g;
-        v4i A[4], B[4];
-#pragma unroll
-        for (int x = 0; x < 4; x++) {
-            v4i ra = onehot16(seq, ldseq, siteA[x], a4A[x], a4A[x] != 0x7f7f7f7fu, n, nseq);
-            v4i rbv = onehot16(seq, ldseq, siteB[x], a4B[x], a4B[x] != 0x7f7f7f7fu, n, nseq);
-            // onehot16 gives 0/1 bytes; rows take -128
-#pragma unroll
-            for (int e = 0; e < 4; e++) ra[e] = (int)((uint32_t)ra[e] << 7);
-            A[x] = ra;
-            B[x] = rbv;
-        }
-#pragma unroll
-        for (int x = 0; x < 4; x++)
-#pragma unroll
-            for (int y = 0; y < 4; y++)
-                acc[x][y] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[x], B[y], acc[x][y], 0, 0, 0);
-    }
-
-    const uint32_t qq = q * q;
-#pragma unroll
-    for (int x = 0; x < 4; x++) {
-#pragma unroll
-        for (int y = 0; y < 4; y++) {
-            const uint32_t c = cb * 128 + y * 32 + lr;
-            if (c >= Lq) continue;
-            const uint32_t jsite = c / q, b = c - jsite * q;
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const uint32_t r = rb * 128 + x * 32 + 8 * (e / 4) + 4 * g + (e % 4);
-                if (r >= Lq) continue;
-                const uint32_t isite = r / q, a = r - isite * q;
-                if (isite < jsite) {
-                    const uint32_t cnt = (0u - (uint32_t)acc[x][y][e]) >> 7;
-                    uint32_t* dst = counts + (size_t)pair_index(isite, jsite, L) * qq + a * q + b;
-                    if (ksplit == 1)
-                        *dst = cnt;
-                    else
-                        atomicAdd(dst, cnt);
-                }
-            }
-        }
+        __syncthreads();   // the last stage has been read
     }
 }
 

@@ -105,6 +105,8 @@ struct mi3_ctx {
     // the reason in scratch_err, if its address could not be resolved)
     char* scratch = nullptr;
     std::string scratch_err;
+    uint8_t* packed = nullptr;                // residues packed for the bicounts
+    size_t packed_cap = 0;
     uint8_t* seq1 = nullptr;                  // one sequence (fill_seqs)
     // host staging
     std::vector<Pinned> pins;
@@ -239,11 +241,9 @@ int pin_get(mi3_ctx* c, size_t bytes) {
     return (int)c->pins.size() - 1;
 }
 
-// Parts of the sequence range for the bicount kernel: about four waves per
-// SIMD (one wave fits per SIMD at a time) share the work evenly, keeping at
-// least 64 k-steps of 32 sequences per wave; each wave's int32 accumulators
-// reach -128 per co-occurrence, so a part stays below 2^24 sequences
-// (|acc| < 2^31).
+// Parts of the sequence range of a 128 x 128 block of the bicount kernel: enough
+// that there are about four waves for each SIMD (one fits at a time), of at
+// least 2048 sequences each, and below 2^24 (a wave sums in float32).
 uint32_t bicount_split(const mi3_ctx* c, uint32_t nseq) {
     const uint32_t Lq = c->L * c->q;
     const uint32_t nblk = (Lq + 127) / 128;
@@ -404,6 +404,7 @@ int mi3_destroy(mi3_ctx* c) {
     hipFree(c->probe_out);
     hipFree(c->wbad);
     hipFree(c->wm_units);
+    hipFree(c->packed);
     hipFree(c->seq1);
     if (c->t0) hipEventDestroy(c->t0);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -815,16 +816,60 @@ int mi3_calc_bicounts(mi3_ctx* c, const char* seqbuf, uint32_t nseq) {
     const uint32_t nbw = nblk * (nblk + 1) / 2;
     const uint32_t ksplit = bicount_split(c, nseq);
     Scope s(c, "calcBicounts", (size_t)nseq * c->L);
-    if (ksplit > 1) {
+    // residues packed to bit planes (16 bytes a plane per 128 sequences of a site);
+    // the workspace is kept and grows to the largest call's size
+    const uint32_t planes = bc_planes(c->q), nunits = (nseq + BC_UNIT - 1) / BC_UNIT;
+    const size_t pk_bytes = (size_t)c->L * nunits * 16 * planes;
+    if (ksplit > 1 || nunits == 0 || nunits > BC_PART) {   // no wave stores a whole block
         int frc = fill_u32_dev(c, cb->d, 0u, (uint64_t)c->nP * c->q * c->q);
         if (frc) return frc;
     }
-    const uint32_t stage = bc_stage_for(c->q);
-    auto kern = stage == 16 ? k_bicounts_mfma128<16> : stage == 8 ? k_bicounts_mfma128<8>
-                                                                   : k_bicounts_mfma128<4>;
-    hipLaunchKernelGGL(kern, dim3(nbw * ksplit), dim3(64), bc_lds_bytes(c->q, stage), c->stream,
-                       (const uint8_t*)sb->d, (uint32_t)ld, nseq, c->L, c->q, nblk, ksplit,
-                       (uint32_t*)cb->d);
+    if (c->packed_cap < pk_bytes) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        hipFree(c->packed);
+        c->packed = nullptr;
+        c->packed_cap = 0;
+        HIPCHK(c, hipMalloc(&c->packed, pk_bytes));
+        c->packed_cap = pk_bytes;
+    }
+    if (nunits) {
+        const dim3 grid((nunits * 2 + 255) / 256, c->L);
+        if (planes == 3)
+            hipLaunchKernelGGL(k_pack_residues<3>, grid, dim3(256), 0, c->stream,
+                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, c->packed);
+        else
+            hipLaunchKernelGGL(k_pack_residues<5>, grid, dim3(256), 0, c->stream,
+                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, c->packed);
+    }
+    // 128 x 128 blocks where those, times the parts, fill the card's SIMDs with a wave
+    // each; below, 64 x 64 blocks, two waves to a SIMD.  The waves that the card holds
+    // divide the work evenly, except where a block has one part: there a wave
+    // takes a block, and stores its counts without atomics (50 kB of them per
+    // block: 5 parts per block instead of even shares took 378 us instead of 207
+    // at 16384 sequences, L=232 q=21).
+    const bool small = (uint64_t)nbw * ksplit < 4ull * c->ncu;
+    const uint32_t tile = small ? 64 : 128;
+    const uint32_t nb = (Lq + tile - 1) / tile;
+    const uint32_t ntiles = nb * (nb + 1) / 2, slots = (small ? 8 : 4) * c->ncu;
+    const dim3 grid(ksplit == 1 || ntiles * ksplit < slots ? ntiles * ksplit : slots);
+    const uint32_t stage = bc_stage_for(c->q, tile);
+    const size_t lds = bc_lds_bytes(c->q, tile, stage);
+#define MI3_BC(NT, PL, ST)                                                                     \
+    hipLaunchKernelGGL((k_bicounts_fp4<NT, PL, ST>), grid, dim3(64), lds, c->stream,            \
+                       (const uint8_t*)c->packed, nunits, c->L, c->q, nb,                       \
+                       (uint64_t)ntiles * nunits,                                              \
+                       (uint32_t*)cb->d)
+    if (planes == 5) {
+        if (small) MI3_BC(2, 5, 5);
+        else MI3_BC(4, 5, 5);
+    } else if (stage == 5) {
+        if (small) MI3_BC(2, 3, 5);
+        else MI3_BC(4, 3, 5);
+    } else {
+        if (small) MI3_BC(2, 3, 3);
+        else MI3_BC(4, 3, 3);
+    }
+#undef MI3_BC
     HIPCHK(c, hipGetLastError());
     cb->version++;
     return MI3_OK;
