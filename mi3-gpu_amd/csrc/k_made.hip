@@ -437,90 +437,127 @@ __global__ void k_relu_grad(uint64_t n, const float* __restrict__ dh,
 // rows of those units on v_mfma_f32_16x16x32_bf16, the k-steps dealt to the
 // 4 waves (wave 0 starts from the bias) and the partials summed in a fixed
 // order, then bf16(relu(.)) into LDS; (C) site j's q logits the same way
-// (two column tiles) from the layer-2 units, W3b rows q*j..q*j+q-1 and b3;
-// (D) 16 lanes per walker: softmax, draw or read, nll, then wave 1 draws the
-// next site's uniforms; (E) the float32 layer-1 sums of units of degree
-// > j add W1t's row of the site's letter (the sums are formed in site order,
-// as the teacher-forced embedding forms them).
+// (one or two column tiles) from the layer-2 units, W3b rows q*j..q*j+q-1 and
+// b3; (D) 16 lanes per walker: softmax, draw or read; (E) the float32 layer-1
+// sums of units of degree > j add W1t's row of the site's letter (the sums
+// are formed in site order, as the teacher-forced embedding forms them).  The
+// uniforms of 16 sites are drawn together, one per thread.
 //
-// The B operands and biases of (B) and (C) for site j+1 are loaded into
-// registers right after the products of site j use them; when teacher
-// forcing, so are the next site's letters.  Requires H % 32 == 0,
-// H <= 512, q <= 25.
+// Bound by the chain of a site's phases (five barriers, two LDS exchanges of
+// partial products, the gather of W1t rows once the letters are known) and,
+// with many tiles, by instruction issue and the vector L1.  So a tile takes 40 KiB
+// of LDS and 128 registers per lane, four tiles to a CU; the softmax exchanges
+// values within its 16 lanes by data-parallel primitives and sums the partials
+// itself; loads have no branches and one 32-bit offset per lane.  The
+// operands of (B) for site j+1 are loaded after those of site j are used, those of
+// (C) after the gathers of (E); when teacher forcing, so are the next site's
+// letters.  Measured (us; three tiles to a CU, logits through LDS, shuffles, one
+// wave drawing, branches around loads; and this form), draws, L=232 q=21 H=512:
+// 65536 walkers 5532 and 4270, 4096 walkers (one tile per CU) 846 and 576; L=96
+// q=4 H=256, 32768 walkers 924 and 434.
+// Requires H % 32 == 0, H <= 512, q <= 25.
 constexpr int MF_T = 16, MF_WAVES = 4, MF_THREADS = 64 * MF_WAVES, MF_HMAX = 512;
-constexpr int MF_HU = MF_HMAX / MF_THREADS;     // layer-1 units per thread
 constexpr int MF_QMAX = 25;
-constexpr int MF_HP = MF_HMAX + 8;              // padded LDS row (bf16) of a walker's units
-constexpr int MF_KS = MF_HMAX / 32 / MF_WAVES;  // k-steps of 32 per wave
-constexpr int MF_NC = 32;                       // logit columns (two tiles of 16)
+constexpr int MF_NC = MF_QMAX;                  // columns of the partial products (odd)
 static_assert(MF_THREADS == 16 * MF_T, "16 lanes per walker in the softmax");
 
+// KS: k-steps of 32 units per wave; rows are padded by 8 units
+template <int KS>
 struct MadeFusedLds {
-    bf16 h1[MF_T][MF_HP];                  // bf16(relu(layer 1)), final units only
-    bf16 h2[MF_T][MF_HP];                  // bf16(relu(layer 2)), final units only
-    float part[MF_WAVES][MF_T][MF_NC + 1]; // per-wave partial products
-    float z[MF_T][MF_NC + 1];              // the site's logits
-    float u[2][MF_T];                      // uniforms of this / the next site
-    uint32_t s[MF_T];                      // the site's letters
+    bf16 h1[MF_T][32 * MF_WAVES * KS + 8]; // bf16(relu(layer 1)), final units only
+    bf16 h2[MF_T][32 * MF_WAVES * KS + 8]; // bf16(relu(layer 2)), final units only
+    float part[MF_WAVES][MF_T][MF_NC];     // per-wave partial products
+    float u[MF_T][MF_T];                   // uniforms of 16 sites
+    uint32_t s[MF_T];                      // offsets of the letters' rows of W1t
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // B operand of one wave's k-steps for one 16-column tile: this lane's 8
-// k-values of column lane%16 (zero for a negative row or k past H), and for
-// wave 0 the column's bias (the accumulator's start).
+// k-values of column lane%16, and the column's bias (the accumulator's start in
+// wave 0).  Buffer loads: a uniform base per site, one 32-bit offset per lane for
+// all sites, and no branches; what lies past the rows' end reads as zero.
+// Columns that nobody reads and k-steps past H, which are not multiplied, hold
+// whatever is there.
+template <int KS>
 struct MadeB {
-    bf16x8 b[MF_KS];
+    bf16x8 b[KS];
     float bias;
 };
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void made_load_b(MadeB& r, const bf16* __restrict__ W,
-                                            const float* __restrict__ bias, uint32_t H, int row,
-                                            int lg, int wave) {
-    const bf16x8 zero8 = {};
-#pragma unroll
-    for (int t = 0; t < MF_KS; t++) {
-        const uint32_t k0 = 32 * (wave + MF_WAVES * t);
-        r.b[t] = (row >= 0 && k0 < H)
-            ? *reinterpret_cast<const bf16x8*>(W + (size_t)row * H + k0 + 8 * lg) : zero8;
-    }
-    r.bias = (wave == 0 && row >= 0) ? bias[row] : 0.f;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t made_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
-// part[wave][.][c0 + .] = bias (wave 0) + X[16 x H] . (this wave's k-steps of b)
-__device__ __forceinline__ void made_product(const bf16 (*X)[MF_HP], const MadeB& b, uint32_t H,
-                                             float (*part)[MF_NC + 1], int c0, int lr, int lg,
-                                             int wave) {
-    f32x4 acc;
+// rows of W from `at` bytes, columns' biases from `bat` bytes
+template <int KS>
+__device__ __forceinline__ void made_load_b(MadeB<KS>& r, __amdgpu_buffer_rsrc_t W, uint32_t at,
+                                            __amdgpu_buffer_rsrc_t bias, uint32_t bat) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) acc[e] = b.bias;
+    for (int t = 0; t < KS; t++) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(W, (int)(at + 64 * MF_WAVES * t), 0, 0);
+        r.b[t] = __builtin_bit_cast(bf16x8, v);
+    }
+    r.bias = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(bias, (int)bat, 0, 0));
+}
+
+// part[wave][.][16 c + .] = bias (wave 0) + X[16 x H] . (this wave's k-steps of b[c])
+template <int KS, int NC>
+__device__ __forceinline__ void made_product(const bf16 (*X)[32 * MF_WAVES * KS + 8],
+                                             const MadeB<KS> (&b)[NC], uint32_t H,
+                                             float (*part)[MF_NC], int lr, int lg, int wave) {
+    f32x4 acc[NC];
+    bf16x8 a[KS];
 #pragma unroll
-    for (int t = 0; t < MF_KS; t++) {
-        const uint32_t k0 = 32 * (wave + MF_WAVES * t);
-        if (k0 < H) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&X[lr][k0 + 8 * lg]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b.b[t], acc, 0, 0, 0);
+    for (int t = 0; t < KS; t++)
+        a[t] = *reinterpret_cast<const bf16x8*>(&X[lr][32 * (wave + MF_WAVES * t) + 8 * lg]);
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[c][e] = wave == 0 ? b[c].bias : 0.f;
+#pragma unroll
+    for (int t = 0; t < KS; t++) {
+        if (t < KS - 1 || 32u * (wave + MF_WAVES * t) < H) {
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[c].b[t], acc[c], 0, 0, 0);
         }
     }
     // D layout: value e of lane l is row 4*(l/16) + e, column l%16
 #pragma unroll
-    for (int e = 0; e < 4; e++) part[4 * lg + e][c0 + lr] = acc[e];
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (16 * c + lr < MF_NC) part[4 * lg + e][16 * c + lr] = acc[c][e];
 }
 
-__device__ __forceinline__ float made_part_sum(const float (*part)[MF_T][MF_NC + 1], uint32_t r,
+__device__ __forceinline__ float made_part_sum(const float (*part)[MF_T][MF_NC], uint32_t r,
                                                uint32_t c) {
     return ((part[0][r][c] + part[1][r][c]) + part[2][r][c]) + part[3][r][c];
 }
 
-__global__ __launch_bounds__(MF_THREADS) void k_made_fused(
+// Value of another lane of the row of 16 by data-parallel primitives: rotated by
+// n lanes, shifted up by n lanes (zero where none is), or lane n's.
+constexpr int DPP_ROW_SHR = 0x110, DPP_ROW_ROR = 0x120, DPP_ROW_BCAST = 0x150;
+template <int CTRL>
+__device__ __forceinline__ float row_dpp(float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
+// KS = ceil(H / 128), NC = ceil(q / 16): smaller networks take less LDS and fewer
+// registers, so more tiles share a CU.
+template <int KS, int NC>
+__global__ __launch_bounds__(MF_THREADS, KS > 2 ? 4 : 5) void k_made_fused(
     uint32_t L, uint32_t q, uint32_t H, uint32_t B, const float* __restrict__ W1t,
     const float* __restrict__ b1, const bf16* __restrict__ W2b, const float* __restrict__ b2,
     const bf16* __restrict__ W3b, const float* __restrict__ b3, uint32_t k0, uint32_t k1,
     uint32_t counter, uint32_t walker_base, uint8_t* __restrict__ seq, uint32_t ld,
     float* __restrict__ nll, int draw) {
-    __shared__ MadeFusedLds sm;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int lr = lane & 15, lg = lane >> 4;
+    constexpr int HU = (KS + 1) / 2;   // layer-1 units per thread
+    __shared__ MadeFusedLds<KS> sm;
+    int tid = threadIdx.x, lr = tid & 15, lg = (tid >> 4) & 3;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t tile0 = blockIdx.x * MF_T;
     const uint32_t Lm1 = L - 1;
@@ -528,40 +565,34 @@ __global__ __launch_bounds__(MF_THREADS) void k_made_fused(
     auto n_units = [&](uint32_t jj) -> uint32_t {
         return (jj >= 1 && jj < L && jj - 1 < H) ? (H - (jj - 1) + Lm1 - 1) / Lm1 : 0u;
     };
-    uint32_t deg[MF_HU];
-    float h1r[MF_HU][MF_T];
+    uint32_t deg[HU];
+    float h1r[HU][MF_T];
 #pragma unroll
-    for (int u = 0; u < MF_HU; u++) {
+    for (int u = 0; u < HU; u++) {
         const uint32_t k = tid + MF_THREADS * u;
         deg[u] = k < H ? 1 + k % Lm1 : 0xffffffffu;
         const float v = k < H ? b1[k] : 0.f;
 #pragma unroll
         for (int w = 0; w < MF_T; w++) h1r[u][w] = v;
     }
-    for (uint32_t e = tid; e < MF_T * MF_HP; e += MF_THREADS) {
+    for (uint32_t e = tid; e < sizeof(sm.h1) / sizeof(bf16); e += MF_THREADS) {
         (&sm.h1[0][0])[e] = (bf16)0.f;
         (&sm.h2[0][0])[e] = (bf16)0.f;
     }
-    MadeB w2r, w3r[2];
-    auto load_w2 = [&](uint32_t jj) {
-        const uint32_t nU = n_units(jj);
-        const int row = (nU <= MF_T && (uint32_t)lr < nU) ? (int)((jj - 1) + lr * Lm1) : -1;
-        made_load_b(w2r, W2b, b2, H, row, lg, wave);
+    MadeB<KS> w2r[1], w3r[NC];
+    const __amdgpu_buffer_rsrc_t w2 = made_rsrc(W2b, H * H * 2), bias2 = made_rsrc(b2, H * 4);
+    // operands of the 16 layer-2 units jj - 1 + (c0 + lane % 16) (L - 1)
+    auto load_w2 = [&](uint32_t jj, uint32_t c0) {
+        const uint32_t row = (jj > 0 ? jj - 1 : 0) + (c0 + lr) * Lm1;
+        made_load_b(w2r[0], w2, row * H * 2 + 2 * (32 * wave + 8 * lg), bias2, row * 4);
     };
     auto load_w3 = [&](uint32_t jj) {
+        const size_t r0 = (size_t)q * (jj < L ? jj : 0u);
+        const __amdgpu_buffer_rsrc_t w3 = made_rsrc(W3b + r0 * H, q * H * 2);
+        const __amdgpu_buffer_rsrc_t bias3 = made_rsrc(b3 + r0, q * 4);
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const uint32_t c = 16 * t + lr;
-            made_load_b(w3r[t], W3b, b3, H, (jj < L && c < q) ? (int)(q * jj + c) : -1, lg, wave);
-        }
-    };
-    // uniforms of site jj for the tile's walkers (wave 1, lanes < 16)
-    auto draw_u = [&](uint32_t jj) {
-        if (draw && wave == 1 && lane < MF_T && jj < L) {
-            const uint4 r = philox4x32_10(make_uint4(jj, walker_base + tile0 + lane, counter,
-                                                     TAG_MADE), k0, k1);
-            sm.u[jj & 1][lane] = (float)(r.x >> 8) * 0x1.0p-24f;
-        }
+        for (int t = 0; t < NC; t++)
+            made_load_b(w3r[t], w3, (16 * t + lr) * H * 2 + 2 * (32 * wave + 8 * lg), bias3, (16 * t + lr) * 4);
     };
     // teacher forcing: every lane of walker w's group holds its letter at the
     // next site
@@ -570,16 +601,27 @@ __global__ __launch_bounds__(MF_THREADS) void k_made_fused(
         const uint32_t b = tile0 + ((uint32_t)tid >> 4);
         s_next = (!draw && b < B && jj < L) ? seq[(size_t)jj * ld + b] : 0u;
     };
-    load_w2(0);
+    load_w2(0, 0);
     load_w3(0);
     load_s(0);
-    draw_u(0);
     float nacc = 0.f;    // nll of walker tile0 + tid / 16 (every lane of its group)
 
     for (uint32_t j = 0; j < L; j++) {
+        // what depends on the lane is formed anew at each site: kept over the sites, it
+        // takes the registers of a fourth tile on the CU
+        asm volatile("" : "+v"(tid));
+        lr = tid & 15;
+        lg = (tid >> 4) & 3;
+        // uniforms of sites j .. j + MF_T - 1
+        if (draw && j % MF_T == 0) {
+            const uint4 r = philox4x32_10(
+                make_uint4(j + ((uint32_t)tid >> 4), walker_base + tile0 + (tid & 15), counter,
+                           TAG_MADE), k0, k1);
+            sm.u[tid >> 4][tid & 15] = (float)(r.x >> 8) * 0x1.0p-24f;
+        }
         // (A) layer-1 units of degree j are final
 #pragma unroll
-        for (int u = 0; u < MF_HU; u++) {
+        for (int u = 0; u < HU; u++) {
             if (deg[u] == j) {
                 const uint32_t k = tid + MF_THREADS * u;
 #pragma unroll
@@ -590,11 +632,8 @@ __global__ __launch_bounds__(MF_THREADS) void k_made_fused(
         // (B) layer-2 units of degree j, 16 at a time
         const uint32_t nU = n_units(j);
         for (uint32_t c0 = 0; c0 < nU; c0 += MF_T) {
-            if (nU > MF_T) {   // more than one column tile: operands loaded here
-                const uint32_t c = c0 + lr;
-                made_load_b(w2r, W2b, b2, H, c < nU ? (int)((j - 1) + c * Lm1) : -1, lg, wave);
-            }
-            made_product(sm.h1, w2r, H, sm.part[wave], 0, lr, lg, wave);
+            if (c0 > 0) load_w2(j, c0);   // the first 16 are there
+            made_product(sm.h1, w2r, H, sm.part[wave], lr, lg, wave);
             __syncthreads();
             {
                 const uint32_t r = tid / MF_T, c = tid % MF_T;   // 256 = 16 x 16 entries
@@ -604,46 +643,38 @@ __global__ __launch_bounds__(MF_THREADS) void k_made_fused(
             }
             __syncthreads();
         }
-        load_w2(j + 1);
         // (C) logits of site j (columns a < q), b3 included
-        made_product(sm.h2, w3r[0], H, sm.part[wave], 0, lr, lg, wave);
-        made_product(sm.h2, w3r[1], H, sm.part[wave], 16, lr, lg, wave);
-        load_w3(j + 1);
+        made_product(sm.h2, w3r, H, sm.part[wave], lr, lg, wave);
         __syncthreads();
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t e = tid + MF_THREADS * h, r = e / MF_NC, c = e % MF_NC;
-            if (c < q) sm.z[r][c] = made_part_sum(sm.part, r, c);
-        }
-        __syncthreads();
+        load_w2(j + 1, 0);
         // (D) softmax and the letter: 16 lanes per walker (walker tid / 16;
         // lane l holds letters l and l + 16), max, sum and the inverse-CDF
         // search by 16-lane shuffles and one ballot; wave 1 then draws the
         // next site's uniforms
+        float zs, mxs, ses;   // this lane's logit if the letter is s % 16, max, sum
+        uint32_t ls;
         {
             const uint32_t w = (uint32_t)tid >> 4, l = (uint32_t)tid & 15;
-            const float z1 = (l < q) ? sm.z[w][l] : -INFINITY;
-            const float z2 = (l + 16 < q) ? sm.z[w][l + 16] : -INFINITY;
+            const float z1 = (l < q) ? made_part_sum(sm.part, w, l) : -INFINITY;
+            const float z2 = (NC > 1 && l + 16 < q) ? made_part_sum(sm.part, w, l + 16) : -INFINITY;
             float mx = fmaxf(z1, z2);
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 16));
+            mx = fmaxf(mx, row_dpp<DPP_ROW_ROR + 8>(mx));
+            mx = fmaxf(mx, row_dpp<DPP_ROW_ROR + 4>(mx));
+            mx = fmaxf(mx, row_dpp<DPP_ROW_ROR + 2>(mx));
+            mx = fmaxf(mx, row_dpp<DPP_ROW_ROR + 1>(mx));
             float c1 = (l < q) ? __expf(z1 - mx) : 0.f;
             float c2 = (l + 16 < q) ? __expf(z2 - mx) : 0.f;
             // inclusive prefix sums over the group (letters in order)
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                const float t1 = __shfl_up(c1, o, 16), t2 = __shfl_up(c2, o, 16);
-                if (l >= (uint32_t)o) {
-                    c1 += t1;
-                    c2 += t2;
-                }
-            }
-            const float tot1 = __shfl(c1, 15, 16);
-            const float se = tot1 + __shfl(c2, 15, 16);
+            c1 += row_dpp<DPP_ROW_SHR + 1>(c1), c2 += row_dpp<DPP_ROW_SHR + 1>(c2);
+            c1 += row_dpp<DPP_ROW_SHR + 2>(c1), c2 += row_dpp<DPP_ROW_SHR + 2>(c2);
+            c1 += row_dpp<DPP_ROW_SHR + 4>(c1), c2 += row_dpp<DPP_ROW_SHR + 4>(c2);
+            c1 += row_dpp<DPP_ROW_SHR + 8>(c1), c2 += row_dpp<DPP_ROW_SHR + 8>(c2);
+            const float tot1 = row_dpp<DPP_ROW_BCAST + 15>(c1);
+            const float se = tot1 + row_dpp<DPP_ROW_BCAST + 15>(c2);
             uint32_t s;
             if (draw) {
                 // first letter a (a + 1 < q) whose cumulative mass exceeds u
-                const float uu = sm.u[j & 1][w] * se;
+                const float uu = sm.u[j % MF_T][w] * se;
                 const uint64_t m1 = __ballot((l + 1 < q) && uu < c1);
                 const uint64_t m2 = __ballot((l + 17 < q) && uu < tot1 + c2);
                 const uint32_t sh = (uint32_t)tid & 48u;
@@ -655,29 +686,33 @@ __global__ __launch_bounds__(MF_THREADS) void k_made_fused(
             } else {
                 s = s_next < q ? s_next : q - 1;
             }
-            nacc += mx + __logf(se) - sm.z[w][s];
-            if (l == 0) sm.s[w] = s;
+            if (l == 0) sm.s[w] = s * H * 4;   // bytes of its row of W1t
+            zs = s < 16 ? z1 : z2;
+            ls = s & 15;
+            mxs = mx;
+            ses = se;
         }
-        draw_u(j + 1);
         load_s(j + 1);
         __syncthreads();
-        // (E) sums of the layer-1 units that see site j
-        if (j + 1 < L) {
-            uint32_t sw[MF_T];
+        // (E) sums of the layer-1 units that see site j.  Waves that hold none read
+        // nothing (an empty buffer, zeros); sums that are final already may change.
+        float v[HU][MF_T];
 #pragma unroll
-            for (int w = 0; w < MF_T; w++) sw[w] = sm.s[w];
+        for (int u = 0; u < HU; u++) {
+            const bool sees = __any(deg[u] != 0xffffffffu && deg[u] > j);
+            const __amdgpu_buffer_rsrc_t w1 =
+                made_rsrc(W1t + (size_t)(q * j) * H, sees ? q * H * 4 : 0u);
 #pragma unroll
-            for (int u = 0; u < MF_HU; u++) {
-                if (deg[u] != 0xffffffffu && deg[u] > j) {
-                    const uint32_t k = tid + MF_THREADS * u;
-                    float v[MF_T];
-#pragma unroll
-                    for (int w = 0; w < MF_T; w++) v[w] = W1t[(size_t)(q * j + sw[w]) * H + k];
-#pragma unroll
-                    for (int w = 0; w < MF_T; w++) h1r[u][w] += v[w];
-                }
-            }
+            for (int w = 0; w < MF_T; w++)
+                v[u][w] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    w1, (int)(sm.s[w] + 4 * (tid + MF_THREADS * u)), 0, 0));
         }
+        nacc += mxs + __logf(ses) - __shfl(zs, (int)ls, 16);
+#pragma unroll
+        for (int u = 0; u < HU; u++)
+#pragma unroll
+            for (int w = 0; w < MF_T; w++) h1r[u][w] += v[u][w];
+        load_w3(j + 1);
     }
     if ((tid & 15) == 0 && tile0 + (tid >> 4) < B) nll[tile0 + (tid >> 4)] = nacc;
 }

@@ -139,7 +139,12 @@ int mi3_made_fused(void* stream, uint32_t L, uint32_t q, uint32_t H, uint32_t B,
     if (q > (uint32_t)MF_QMAX || H == 0 || H % 32 || H > (uint32_t)MF_HMAX)
         return mfail(MI3_EUNSUP, "made_fused: needs q <= 25 and H a multiple of 32 up to 512");
     if (B == 0) return MI3_OK;
-    hipLaunchKernelGGL(k_made_fused, dim3((B + MF_T - 1) / MF_T), dim3(MF_THREADS), 0, S(stream),
+    const uint32_t ks = (H + 127) / 128;
+    auto kern = q > 16 ? (ks == 1 ? k_made_fused<1, 2> : ks == 2 ? k_made_fused<2, 2>
+                          : ks == 3 ? k_made_fused<3, 2> : k_made_fused<4, 2>)
+                       : (ks == 1 ? k_made_fused<1, 1> : ks == 2 ? k_made_fused<2, 1>
+                          : ks == 3 ? k_made_fused<3, 1> : k_made_fused<4, 1>);
+    hipLaunchKernelGGL(kern, dim3((B + MF_T - 1) / MF_T), dim3(MF_THREADS), 0, S(stream),
                        L, q, H, B, W1t, b1, static_cast<const bf16*>(W2b), b2,
                        static_cast<const bf16*>(W3b), b3, (uint32_t)seed, (uint32_t)(seed >> 32),
                        counter, walker_base, seq, ld, nll, draw);

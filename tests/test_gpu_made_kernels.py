@@ -87,3 +87,41 @@ def test_column_sums(gpu_ok, rows, cols):
     d.sync()
     np.testing.assert_allclose(d.read('o'), x.astype('f8').sum(axis=0), rtol=0, atol=2e-6 * rows)
     d.close()
+
+
+# (L, q, H, B): each number of k-steps per wave (H to 128, 256, 384, 512) full and
+# ragged, one and two column tiles of letters, more than 16 units of a degree and
+# fewer units than degrees, walkers that end inside a tile
+@pytest.mark.parametrize("L,q,H,B", [(2, 4, 32, 1), (8, 17, 128, 33), (40, 25, 160, 64), (24, 2, 256, 16),
+                                     (56, 21, 288, 100), (16, 10, 384, 1000), (600, 4, 416, 20),
+                                     (4, 16, 512, 17), (24, 21, 480, 50)])
+def test_fused_draws(gpu_ok, L, q, H, B):
+    from mi3gpu.made import MADE
+    from oracle import made_oracle as mo
+    from oracle.philox import philox4x32_10
+    from test_gpu_made import _params, _perturb
+    from mi3gpu._lib import lib
+    m = MADE(L, q, H, max_batch=16, seed=4)
+    _perturb(m, np.random.default_rng(8), {'W1t': 0.1, 'b1': 0.1, 'W2': 0.1, 'b2': 0.1, 'W3': 0.1, 'b3': 0.5})
+    ld = (B + 15) // 16 * 16
+    m.mem.alloc('out', (L, ld), 'u1')
+    m.mem.alloc('drawn', (B,), 'f4')
+    m.mem.alloc('read', (B,), 'f4')
+    for nll, draw in (('drawn', 1), ('read', 0)):
+        assert lib().mi3_made_fused(m.mem.stream, L, q, H, B, *[m.mem[k] for k in ('W1t', 'b1', 'W2b', 'b2', 'W3b', 'b3')],
+                                    5 + (7 << 32), 9, 3, m.mem['out'], ld, m.mem[nll], draw) == 0
+    s = m.get('out').T[:B]
+    np.testing.assert_array_equal(m.get('drawn'), m.get('read'))
+    # a unit that rounds to the other bfloat16 neighbour (2^-8 of a value of at most
+    # 2) moves a logit by up to 2e-3; two of them are allowed for
+    f = mo.forward(s, *_params(m), q, bf=True)
+    np.testing.assert_allclose(m.get('read'), f['nll'], rtol=1e-4, atol=5e-3)
+    z = f['logits'].reshape(B, L, q)
+    cdf = np.cumsum(np.exp(z - f['lse'][..., None]), axis=2)
+    j, b = np.meshgrid(np.arange(L, dtype=np.uint32), 3 + np.arange(B, dtype=np.uint32))
+    one = np.ones_like(j)
+    u = (philox4x32_10(j, b, 9 * one, 0x4D414445 * one, 5, 7)[0] >> 8) * 2.0 ** -24
+    want = np.minimum((cdf <= u[..., None]).sum(axis=2), q - 1)
+    clear = np.abs(cdf - u[..., None]).min(axis=2) > 5e-3
+    assert clear.mean() > 0.5 and np.array_equal(want[clear], s[clear])
+    m.close()
