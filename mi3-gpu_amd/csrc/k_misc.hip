@@ -32,6 +32,64 @@ __global__ void k_unpack_chunked(const float* __restrict__ J, float* __restrict_
     Ju[idx] = v;
 }
 
+// Folded model for energies: k neighbouring sites as one of q^k letters, so that
+// one gather adds k*k couplings (rule at fold_sites).  Couplings of the folded
+// sites i < m in the chunked layout above, and zeros for the partners m <= i, which
+// the energies do not count; what lies within a folded site is added to its
+// couplings with the next one (the last site's to those with the one before).
+// Sites past L have no couplings.
+__global__ void k_fold_chunked(const float* __restrict__ J, float* __restrict__ Ju, uint32_t L,
+                               uint32_t q, uint32_t k, uint32_t Q, uint32_t nfold, uint32_t nchunk,
+                               uint32_t chf, uint32_t total) {
+    const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= total) return;
+    const uint32_t unit = idx / chf, within = idx - unit * chf;
+    const uint32_t i = unit / nchunk, c = unit - i * nchunk;
+    const uint32_t m = c * CH + (within & 31), ab = within >> 5;
+    float v = 0.f;
+    if (ab < Q * Q && m < nfold && m > i) {
+        const uint32_t a = ab / Q, b = ab - a * Q;
+        auto letter = [&](uint32_t x, uint32_t t) {   // of site t of a folded one
+            for (uint32_t u = t + 1; u < k; u++) x /= q;
+            return x % q;
+        };
+        auto coupling = [&](uint32_t x, uint32_t y, uint32_t sx, uint32_t sy) {
+            return y < L ? J[(size_t)pair_index(x, y, L) * q * q + sx * q + sy] : 0.f;
+        };
+        for (uint32_t t = 0; t < k; t++)
+            for (uint32_t u = 0; u < k; u++)
+                v += coupling(i * k + t, m * k + u, letter(a, t), letter(b, u));
+        if (m == i + 1)
+            for (uint32_t t = 0; t < k; t++)
+                for (uint32_t u = t + 1; u < k; u++) {
+                    v += coupling(i * k + t, i * k + u, letter(a, t), letter(a, u));
+                    if (m == nfold - 1)
+                        v += coupling(m * k + t, m * k + u, letter(b, t), letter(b, u));
+                }
+    }
+    Ju[idx] = v;
+}
+
+// Sequences of the folded model: 16 of a folded site per thread, site-major rows of
+// ldp bytes (ld and ldp are multiples of 16).  Residues are cut to 3 bits, so that none reaches its neighbour's
+// byte.
+__global__ __launch_bounds__(256) void k_fold_residues(const uint8_t* __restrict__ seq, uint32_t ld,
+                                                       uint32_t L, uint32_t q, uint32_t k,
+                                                       uint8_t* __restrict__ out, uint32_t ldp) {
+    const uint32_t n = (blockIdx.x * 256 + threadIdx.x) * 16, I = blockIdx.y;
+    if (n >= ldp) return;
+    uint32_t x = 0, y = 0, z = 0, w = 0;
+    for (uint32_t t = 0; t < k; t++) {
+        uint4 s = make_uint4(0, 0, 0, 0);
+        if (I * k + t < L && n < ld) s = *reinterpret_cast<const uint4*>(seq + (size_t)(I * k + t) * ld + n);
+        x = x * q + (s.x & 0x07070707u);
+        y = y * q + (s.y & 0x07070707u);
+        z = z * q + (s.z & 0x07070707u);
+        w = w * q + (s.w & 0x07070707u);
+    }
+    *reinterpret_cast<uint4*>(out + (size_t)I * ldp + n) = make_uint4(x, y, z, w);
+}
+
 // Plain streaming kernels over n 16-byte words (grid-stride, eight
 // nontemporal loads in flight per thread): the references for the HBM
 // bandwidth a kernel reaches.  The read kernel stores the xor of the data

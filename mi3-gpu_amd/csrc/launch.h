@@ -88,6 +88,22 @@ inline uint32_t direct_walkers(uint32_t q, uint32_t ncu) { return (q <= 8 ? 12 :
 // 14 / 17 against 18 / 48, 8192 27 / 32 against 19 / 48).
 inline uint32_t direct_sequences(uint32_t q, uint32_t ncu) { return (q <= 8 ? 16 : 8) * ncu; }
 
+// Sites that the energies of many sequences take together as one of q^k letters
+// (1: none): a gather then adds k*k couplings, and the energies are bound by their
+// gathers and what each takes to address.  Reduced alphabets only: the folded one has
+// to stay within MAX_Q letters, and for q = 2 three sites (8 letters, whole rows
+// staged) take as long as four at half the cost of their table.  The table is formed
+// anew when the couplings change (15 us at L=93 q=4 against 8 without folding), so
+// few sequences and short chains are left as they are.  us, before / folded, table
+// included: L=93 q=4, 2^18 sequences 283 / 192, 2^17 154 / 104, 2^16 104 / 100, 2^14
+// 68 / 78; L=232 q=4, 2^18 1381 / 578, 2^16 489 / 297; L=93 q=2, 2^18 273 / 89; L=93
+// q=5, 2^18 296 / 235; L=17 q=4, 2^18 44 / 41.  The error against 64 bits is about
+// half (fewer additions).
+inline uint32_t fold_width(uint32_t q) { return q == 2 ? 3 : q <= 5 ? 2 : 1; }
+inline uint32_t fold_sites(uint32_t q, uint32_t L, uint32_t nseq, uint32_t ncu) {
+    return L >= 32 && nseq > 256 * ncu ? fold_width(q) : 1;
+}
+
 // Walkers (or sequences) per work-group of the chunk-staged kernels, `most` or
 // less: half as many take 0.7-0.97 of the time, on twice the CUs, so tiles are
 // halved only while they occupy at most a quarter of the card.

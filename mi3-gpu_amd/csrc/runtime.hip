@@ -90,6 +90,7 @@ struct mi3_ctx {
     uint32_t ncu = 256;  // compute units of the device
     // derived device data
     std::map<std::string, Chunked> chunked;  // chunked layouts keyed by source buffer
+    std::map<std::string, Chunked> folded;   // those of the folded models
     double* red = nullptr;                    // reduction partials
     float* red_out = nullptr;                 // 2 floats: internal reduction result
     uint64_t* wq = nullptr;                   // fixed-point weights
@@ -224,6 +225,43 @@ int chunked_of(mi3_ctx* c, const char* name, float** out) {
         ch.version = b->version;
     }
     *out = ch.d;
+    return MI3_OK;
+}
+
+// The folded model's couplings (k_fold_chunked; its size depends on L and q
+// alone), rebuilt when stale.
+int folded_of(mi3_ctx* c, const char* name, float** out) {
+    Buf* b;
+    int rc = need(c, name, (size_t)c->nP * c->q * c->q * sizeof(float), &b);
+    if (rc) return rc;
+    Chunked& ch = c->folded[name];
+    const uint32_t k = fold_width(c->q), nfold = (c->L + k - 1) / k;
+    uint32_t Q = c->q;
+    for (uint32_t t = 1; t < k; t++) Q *= c->q;
+    const uint32_t chf = chunk_floats(Q), nchunk = (nfold + 31) / 32;
+    const uint32_t total = nfold * nchunk * chf;
+    if (!ch.d) HIPCHK(c, hipMalloc(&ch.d, total * sizeof(float)));
+    if (ch.version != b->version) {
+        Scope s(c, "fold_couplings", total * 4ull);
+        hipLaunchKernelGGL(k_fold_chunked, dim3(grid1(total)), dim3(256), 0, c->stream,
+                           (const float*)b->d, ch.d, c->L, c->q, k, Q, nfold, nchunk, chf, total);
+        HIPCHK(c, hipGetLastError());
+        ch.version = b->version;
+    }
+    *out = ch.d;
+    return MI3_OK;
+}
+
+// Workspace for packed residues, used in stream order; it is kept and grows to the
+// largest call's size.
+int packed_of(mi3_ctx* c, size_t bytes) {
+    if (c->packed_cap >= bytes) return MI3_OK;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    hipFree(c->packed);
+    c->packed = nullptr;
+    c->packed_cap = 0;
+    HIPCHK(c, hipMalloc(&c->packed, bytes));
+    c->packed_cap = bytes;
     return MI3_OK;
 }
 
@@ -389,6 +427,7 @@ int mi3_destroy(mi3_ctx* c) {
     if (c->stream) hipStreamSynchronize(c->stream);
     for (auto& kv : c->bufs) hipFree(kv.second.d);
     for (auto& kv : c->chunked) hipFree(kv.second.d);
+    for (auto& kv : c->folded) hipFree(kv.second.d);
     for (auto& p : c->pins) hipHostFree(p.h);
     for (auto& t : c->tickets)
         if (t.ev) hipEventDestroy(t.ev);
@@ -780,20 +819,33 @@ int mi3_calc_energies(mi3_ctx* c, const char* seqbuf, const char* Jbuf, const ch
     if (nseq > ld) return fail(c, MI3_EINVAL, "nseq exceeds the sequence buffer");
     rc = need(c, Ebuf, (size_t)nseq * 4, &eb);
     if (rc) return rc;
-    float* Ju;
-    rc = chunked_of(c, Jbuf, &Ju);
-    if (rc) return rc;
     EnergyArgs a;
-    a.Ju = Ju;
     a.seq = (const uint8_t*)sb->d;
     a.E = (float*)eb->d;
     a.ld = (uint32_t)ld;
     a.nseq = nseq;
     a.L = c->L;
     a.q = c->q;
-    a.nchunk = c->nchunk;
     a.ncu = c->ncu;
+    const uint32_t k = ld % 16 ? 1 : fold_sites(c->q, c->L, nseq, c->ncu);
+    if (k > 1) {
+        a.L = (c->L + k - 1) / k;
+        for (uint32_t t = 1; t < k; t++) a.q *= c->q;
+        a.ld = (nseq + 31) / 32 * 32;
+        rc = packed_of(c, (size_t)a.L * a.ld);
+        if (rc) return rc;
+    }
+    a.nchunk = (a.L + 31) / 32;
+    float* Ju;
+    rc = k > 1 ? folded_of(c, Jbuf, &Ju) : chunked_of(c, Jbuf, &Ju);
+    if (rc) return rc;
+    a.Ju = Ju;
     Scope s(c, "getEnergies", (size_t)nseq * (c->L + 4));
+    if (k > 1) {
+        hipLaunchKernelGGL(k_fold_residues, dim3((a.ld / 16 + 255) / 256, a.L), dim3(256), 0, c->stream,
+                           a.seq, (uint32_t)ld, c->L, c->q, k, c->packed, a.ld);
+        a.seq = c->packed;
+    }
     HIPCHK(c, launch_energies(a, c->stream));
     eb->version++;
     return MI3_OK;
@@ -816,22 +868,15 @@ int mi3_calc_bicounts(mi3_ctx* c, const char* seqbuf, uint32_t nseq) {
     const uint32_t nbw = nblk * (nblk + 1) / 2;
     const uint32_t ksplit = bicount_split(c, nseq);
     Scope s(c, "calcBicounts", (size_t)nseq * c->L);
-    // residues packed to bit planes (16 bytes a plane per 128 sequences of a site);
-    // the workspace is kept and grows to the largest call's size
+    // residues packed to bit planes (16 bytes a plane per 128 sequences of a site)
     const uint32_t planes = bc_planes(c->q), nunits = (nseq + BC_UNIT - 1) / BC_UNIT;
     const size_t pk_bytes = (size_t)c->L * nunits * 16 * planes;
     if (ksplit > 1 || nunits == 0 || nunits > BC_PART) {   // no wave stores a whole block
         int frc = fill_u32_dev(c, cb->d, 0u, (uint64_t)c->nP * c->q * c->q);
         if (frc) return frc;
     }
-    if (c->packed_cap < pk_bytes) {
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        hipFree(c->packed);
-        c->packed = nullptr;
-        c->packed_cap = 0;
-        HIPCHK(c, hipMalloc(&c->packed, pk_bytes));
-        c->packed_cap = pk_bytes;
-    }
+    rc = packed_of(c, pk_bytes);
+    if (rc) return rc;
     if (nunits) {
         const dim3 grid((nunits * 2 + 255) / 256, c->L);
         if (planes == 3)

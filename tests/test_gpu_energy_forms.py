@@ -30,3 +30,29 @@ def test_energy_forms(gpu_ok, tmp_path, L, q, n):
     # float32 sums of L(L-1)/2 terms: 1e-5 of the sum of magnitudes, as for the other sizes
     err = np.abs(E - cboracle.energies(s, J)) / cboracle.energies(s, np.abs(J))
     assert E.shape == (n,) and err.max() < 1e-5
+
+
+# (L, q, sequences): folded sites that end with the chain and past it, one and two
+# chunks of them, counts on both sides of the rule
+@pytest.mark.parametrize("L,q,n", [(32, 2, 65537), (97, 2, 66000), (98, 2, 65552), (33, 3, 65537), (64, 4, 65536),
+                                   (65, 4, 65537), (130, 4, 65553), (32, 5, 70001), (67, 5, 65537)])
+def test_energies_folded(gpu_ok, tmp_path, L, q, n):
+    """Also after the couplings change, and (folded: the other forms turn an infinite
+    coupling into NaN) with forbidden pairs of letters, whose energies alone are
+    infinite."""
+    s = seqs_rand(n, L, q, 4)
+    g = make_gpu(tmp_path, L, q, 512, wgsize=512)
+    g.initLargeBufs(n)
+    g.setBuf('seq large', s)
+    for seed in (3, 4):
+        J = model(L, q, seed)
+        want, mag = cboracle.energies(s, J), cboracle.energies(s, np.abs(J))
+        forbid = seed == 4 and n > 65536
+        if forbid:   # sites 0 and 1, letters 1 and 0; the last two sites, 0 and 1
+            J[0, q] = J[-1, 1] = np.inf
+        g.setBuf('J', J)
+        g.calcEnergies('large')
+        E = g.getBuf('E large').read()
+        no = (((s[:, 0] == 1) & (s[:, 1] == 0)) | ((s[:, -2] == 0) & (s[:, -1] == 1))) & forbid
+        assert np.array_equal(np.isposinf(E), no)
+        assert (np.abs(E - want) / mag)[~no].max() < 1e-5
