@@ -454,6 +454,54 @@ __global__ void k_fixed_to_float(const unsigned long long* __restrict__ acc,
     out[idx] = (float)((double)acc[idx] * back);
 }
 
+// Pass 3 where sites were folded (k_fold_residues: nfold sites of Q = q^k letters):
+// a bin is the sum of the folded bins that hold its letters, exact in any order, of the
+// pair of its folded sites; for two sites of one folded site, of the pair that that
+// makes with the next (the last: with the one before), over all of the other's letters.
+// Bound by the latency of its loads, all in flight at once (in loops over q and k
+// given at run time: 44 us instead of 6 on average).
+template <int q, int k>
+__global__ __launch_bounds__(256) void k_unfold_to_float(const unsigned long long* __restrict__ acc,
+                                                         float* __restrict__ out, uint32_t L,
+                                                         uint32_t nfold,
+                                                         const float* __restrict__ wsum,
+                                                         const uint32_t* __restrict__ bad) {
+    constexpr uint32_t qq = q * q, Qr = k == 2 ? q : qq, Q = Qr * q;   // Qr: letters but one
+    // block: the bins of a row i with some of its partners
+    const uint32_t i = blockIdx.y, idx = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t m = i + 1 + idx / qq;
+    if (m >= L) return;
+    const uint32_t ab = idx % qq, a = ab / q, b = ab % q;
+    const uint32_t I = i / k, M = m / k, ti = i % k, tm = m % k;
+    // the folded letter of which site t has letter s and the others rest
+    auto folded = [](uint32_t t, uint32_t s, uint32_t rest) -> uint32_t {
+        if (k == 2) return t == 0 ? s * q + rest : rest * q + s;
+        const uint32_t hi = rest / q, lo = rest % q;
+        return t == 0 ? s * qq + rest : t == 1 ? hi * qq + s * q + lo : rest * q + s;
+    };
+    unsigned long long sum = 0;
+    const uint32_t lo = I != M ? I : (I + 1 < nfold ? I : I - 1), hi = I != M ? M : lo + 1;
+    const unsigned long long* bins = acc + (size_t)pair_index(lo, hi, nfold) * Q * Q;
+    if (I != M) {
+#pragma unroll
+        for (uint32_t x = 0; x < Qr; x++)
+#pragma unroll
+            for (uint32_t y = 0; y < Qr; y++) sum += bins[folded(ti, a, x) * Q + folded(tm, b, y)];
+    } else {
+        // the site of the folded one that is neither (k = 3) has letter r
+#pragma unroll
+        for (uint32_t r = 0; r < (k == 2 ? 1 : q); r++) {
+            const uint32_t A = k == 2 ? a * q + b
+                               : ti == 1 ? r * qq + a * q + b
+                               : tm == 1 ? a * qq + b * q + r : a * qq + r * q + b;
+#pragma unroll
+            for (uint32_t B = 0; B < Q; B++) sum += bins[lo == I ? A * Q + B : B * Q + A];
+        }
+    }
+    const double back = bad[0] ? NAN : (double)wsum[0] * (1.0 / 4611686018427387904.0);
+    out[(size_t)pair_index(i, m, L) * qq + ab] = (float)((double)sum * back);
+}
+
 // The other regularisers of the coupling step (mcmc.cl:904-1243), one wave
 // per q x q pair block; all read the block Jt = J + dJ and the model
 // bimarginals f of the block and subtract a step from dJ:

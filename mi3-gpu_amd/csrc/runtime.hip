@@ -96,6 +96,7 @@ struct mi3_ctx {
     uint64_t* wq = nullptr;                   // fixed-point weights
     size_t wq_cap = 0;
     unsigned long long* wacc = nullptr;       // fixed-point weighted-marginal bins
+    uint64_t wacc_cap = 0;
     unsigned long long* probe_out = nullptr;  // sink of mi3_wm_atomic_probe
     uint32_t* wbad = nullptr;
     uint32_t* wm_units = nullptr;
@@ -963,8 +964,45 @@ int mi3_weighted_marg(mi3_ctx* c, const char* seqbuf, const char* wbuf, uint32_t
         HIPCHK(c, hipMalloc(&c->wq, (size_t)nseq * sizeof(uint64_t) + 256));
         c->wq_cap = nseq;
     }
-    if (!c->wacc) HIPCHK(c, hipMalloc(&c->wacc, nbins * sizeof(unsigned long long)));
-    size_t lds = qq * WM_COLS * sizeof(unsigned long long);
+    // the model that is counted: this one, or its folded one (fold_sites), whose bins
+    // are added up to this one's afterwards.  That costs by its bins, so it takes 2^20
+    // additions for each of a pair's (us, without / with: L=93 q=4, 2^18 sequences 306 /
+    // 132, 66048 96 / 75; q=5 307 / 197 and, left as it is, 94 / 126; q=2 306 / 69;
+    // L=232 q=4, 2^17 sequences 730 / 293; L=33 q=4, 66048, left as it is, 46 / 68)
+    uint32_t k = fold_sites(c->q, c->L, nseq, c->ncu);
+    uint64_t Q = 1;
+    for (uint32_t t = 0; t < k; t++) Q *= c->q;
+    if ((uint64_t)c->nP * nseq < (Q * Q << 20)) k = 1;
+    uint32_t L = c->L, q = c->q, wld = (uint32_t)ld, n_units = c->n_units, split = c->wm_split;
+    const uint8_t* seq = (const uint8_t*)sb->d;
+    if (k > 1) {
+        L = (c->L + k - 1) / k;
+        q = (uint32_t)Q;
+        wld = (nseq + 31) / 32 * 32;
+        rc = packed_of(c, (size_t)L * wld);
+        if (rc) return rc;
+        seq = c->packed;
+    }
+    const uint64_t nacc = (uint64_t)(L * (L - 1) / 2) * q * q;
+    size_t lds = (size_t)q * q * WM_COLS * sizeof(unsigned long long);
+    if (k > 1) {
+        // fewer units, their sequences split: a part's adds take about 5 cycles a
+        // sequence and its histograms' flush (global atomics, all parts together) 0.35 per
+        // bin, so the sum is least at sqrt(14 nseq / (units bins)); at most a work-group
+        // per CU
+        n_units = (L * (L - 1) / 2 + WM_COLS - 1) / WM_COLS;
+        split = (uint32_t)std::sqrt(14.0 * nseq / ((double)n_units * q * q));
+        if (split > c->ncu / n_units) split = c->ncu / n_units;
+        if (split < 1) split = 1;
+    }
+    if (c->wacc_cap < nacc) {
+        if (c->wacc) HIPCHK(c, hipStreamSynchronize(c->stream));
+        hipFree(c->wacc);
+        c->wacc = nullptr;
+        c->wacc_cap = 0;
+        HIPCHK(c, hipMalloc(&c->wacc, nacc * sizeof(unsigned long long)));
+        c->wacc_cap = nacc;
+    }
     HIPCHK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(k_weighted_marg),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     Scope s(c, "weightedMarg", (size_t)nseq * (c->L + 8));
@@ -977,15 +1015,26 @@ int mi3_weighted_marg(mi3_ctx* c, const char* seqbuf, const char* wbuf, uint32_t
                        nb, 1, c->red_out);
     hipLaunchKernelGGL(k_weights_fixed, dim3(grid1(nseq ? nseq : 1)), dim3(256), 0, c->stream,
                        (const float*)wb->d, nseq, (const float*)c->red_out, c->wq, c->wbad);
-    hipLaunchKernelGGL(k_fill_u32, dim3(grid1(2 * nbins)), dim3(256), 0, c->stream,
-                       (uint32_t*)c->wacc, 0u, 2 * nbins);
-    hipLaunchKernelGGL(k_weighted_marg, dim3(c->n_units * c->wm_split), dim3(WM_THREADS), lds,
-                       c->stream, (const uint8_t*)sb->d, (uint32_t)ld, nseq,
-                       (const uint64_t*)c->wq, c->L, c->q, (const uint32_t*)c->wm_units,
-                       c->wm_split, c->wacc, 0u);
-    hipLaunchKernelGGL(k_fixed_to_float, dim3(grid1(nbins)), dim3(256), 0, c->stream,
-                       (const unsigned long long*)c->wacc, (float*)bb->d, nbins,
-                       (const float*)c->red_out, (const uint32_t*)c->wbad);
+    if (k > 1)
+        hipLaunchKernelGGL(k_fold_residues, dim3((wld / 16 + 255) / 256, L), dim3(256), 0, c->stream,
+                           (const uint8_t*)sb->d, (uint32_t)ld, c->L, c->q, k, c->packed, wld);
+    hipLaunchKernelGGL(k_fill_u32, dim3(grid1(2 * nacc)), dim3(256), 0, c->stream,
+                       (uint32_t*)c->wacc, 0u, 2 * nacc);
+    hipLaunchKernelGGL(k_weighted_marg, dim3(n_units * split), dim3(WM_THREADS), lds, c->stream, seq,
+                       wld, nseq, (const uint64_t*)c->wq, L, q, (const uint32_t*)c->wm_units, split,
+                       c->wacc, 0u);
+    if (k > 1) {
+        auto unfold = c->q == 2 ? k_unfold_to_float<2, 3> : c->q == 3 ? k_unfold_to_float<3, 2>
+                      : c->q == 4 ? k_unfold_to_float<4, 2> : k_unfold_to_float<5, 2>;
+        hipLaunchKernelGGL(unfold, dim3(grid1((uint64_t)(c->L - 1) * c->q * c->q), c->L - 1),
+                           dim3(256), 0, c->stream, (const unsigned long long*)c->wacc,
+                           (float*)bb->d, c->L, L, (const float*)c->red_out,
+                           (const uint32_t*)c->wbad);
+    }
+    else
+        hipLaunchKernelGGL(k_fixed_to_float, dim3(grid1(nbins)), dim3(256), 0, c->stream,
+                           (const unsigned long long*)c->wacc, (float*)bb->d, nbins,
+                           (const float*)c->red_out, (const uint32_t*)c->wbad);
     HIPCHK(c, hipGetLastError());
     bb->version++;
     return MI3_OK;
