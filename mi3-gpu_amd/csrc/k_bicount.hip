@@ -18,6 +18,7 @@
 namespace mi3 {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -96,20 +97,21 @@ __device__ __forceinline__ void wait_vmem_bc() { __builtin_amdgcn_s_waitcnt(0x0F
 // zeroed first).  NT = 4 keeps 256 sums per lane in AGPRs, one wave to a SIMD;
 // NT = 2 is for problems too small for that (rule at the launch).
 //
-// Bound by the matrix instructions (16 products of a k-step; with the operands
-// held fixed, the products alone take 1.36 ms of the 1.52 ms at 2^18 sequences,
-// L=232 q=21), as long as the one wave a SIMD holds issues the building of the
-// operands between the products, and reads little of LDS: a k-step's 8 operands
-// take 20 eight-byte reads of 2.6 cycles a CU and 88 other instructions.  Measured
-// (us; 8-bit one-hot products built from bytes, 4-bit ones from nibbles, and
-// this form with a fixed number of parts per block and with even shares):
-//   L    q   sequences   8-bit  nibbles  planes  even shares
-//   232  21  1000003     10653     7020    5595         5533
-//   232  21  262144       3103     2063    1661         1525
-//   232  21  16384         459      400     378          207
-//   150  12  100001        434      377     367          202
-//   93   4   262144        163       84      70           70
-//   99   4   16384          70       26      25           25
+// Bound by the issue of the one wave that a SIMD holds: a matrix instruction takes 37
+// cycles (at 2.4 GHz) alone and one is issued every 59 here.  So the operands of a
+// k-step are built between the products of the one before, evenly and two at a
+// time (their chains of dependent instructions otherwise stall; four at a time, or
+// the reads later, took 3-5% longer); reads are eight bytes wide (2.6 cycles of a CU;
+// 16 bytes 7.6).  Measured (us; 8-bit one-hot products built from bytes, 4-bit ones from
+// nibbles, this form with a fixed number of parts per block, with even shares,
+// and with this order of the building):
+//   L    q   sequences   8-bit  nibbles  planes  even shares  order
+//   232  21  1000003     10653     7020    5595         5533   4825
+//   232  21  262144       3103     2063    1661         1525   1381
+//   232  21  16384         459      400     378          207    199
+//   150  12  100001        434      377     367          202    202
+//   93   4   262144        163       84      70           70     70
+//   99   4   16384          70       26      25           25     25
 template <int NT, int PL, int STAGE>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
@@ -158,20 +160,20 @@ __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
             const uint32_t si = r < Lq ? r / q : first;
             const uint32_t a = r < Lq ? r - si * q : 0u;
             at[w] = (slot0 + si - first) * SB + g * 8;
-    #pragma unroll
+#pragma unroll
             for (int p = 0; p < PL; p++) let[w][p] = 0u - ((a >> p) & 1u);
         };
-    #pragma unroll
+#pragma unroll
         for (int x = 0; x < NT; x++) {
             operand(x, rA0 + x * 32 + lr, siA0, 0);
             operand(NT + x, cB0 + x * 32 + lr, siB0, nsA);
         }
         v16f acc[NT][NT];
-    #pragma unroll
+#pragma unroll
         for (int x = 0; x < NT; x++)
-    #pragma unroll
+#pragma unroll
             for (int y = 0; y < NT; y++)
-    #pragma unroll
+#pragma unroll
                 for (int e = 0; e < 16; e++) acc[x][y][e] = 0.f;
 
         // LDS DMA of one stage: piece P is piece P % LPS of site P / LPS; pieces past
@@ -193,42 +195,47 @@ __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
         };
         // operands: NT of rows, then NT of columns
         struct Raw {
-            uint2 f[2 * NT][PL];
+            u2v f[2 * NT][PL];   // (as a uint2, each iteration waits for the LDS DMA in flight)
         };
         struct Ops {
             v4i f[2 * NT];
         };
         auto read = [&](const uint8_t* unit, int w, Raw& r) __attribute__((always_inline)) {
-    #pragma unroll
+#pragma unroll
             for (int p = 0; p < PL; p++)
-                r.f[w][p] = *reinterpret_cast<const uint2*>(unit + at[w] + 16 * p);
+                r.f[w][p] = *reinterpret_cast<const u2v*>(unit + at[w] + 16 * p);
         };
-        // operand w of k-step h of the unit in r.  Bits 4n + e of the word of matches go to
-        // nibble n of operand word e.  As e2m1, nibbles 1, 2 and 4 are 0.5, 1 and 2: rows
-        // hold word e at (0.5, 1, 2, 2) and columns at (2, 1, 0.5, 0.5), so that each
-        // product is 1 and most words need no shift.
-        auto match = [&](const Raw& r, int w, int h, Ops& o) __attribute__((always_inline)) {
+        // planes [p0, p1) of the matches of operand w at k-step h of the unit in r
+        auto match = [&](const Raw& r, int w, int h, int p0, int p1,
+                         uint32_t& m) __attribute__((always_inline)) {
             auto word = [&](int p) { return h ? r.f[w][p].y : r.f[w][p].x; };
-            uint32_t m = ~(word(0) ^ let[w][0]);
-    #pragma unroll
-            for (int p = 1; p < PL; p++)   // m & ~(word ^ letter)
-                m = (uint32_t)__builtin_amdgcn_bitop3_b32((int)m, (int)word(p), (int)let[w][p], 0x90);
+#pragma unroll
+            for (int p = p0; p < p1; p++)   // m & ~(word ^ letter)
+                m = p == 0 ? ~(word(0) ^ let[w][0])
+                           : (uint32_t)__builtin_amdgcn_bitop3_b32((int)m, (int)word(p),
+                                                                   (int)let[w][p], 0x90);
+        };
+        // the matches as operand w: bits 4n + e go to nibble n of word e.  As e2m1, nibbles 1,
+        // 2 and 4 are 0.5, 1 and 2: rows hold word e at (0.5, 1, 2, 2) and columns at (2, 1,
+        // 0.5, 0.5), so that each product is 1 and most words need no shift.
+        auto spread = [&](uint32_t m, int w, Ops& o) __attribute__((always_inline)) {
             if (w < NT)
                 o.f[w] = v4i{(int)(m & 0x11111111u), (int)(m & 0x22222222u), (int)(m & 0x44444444u),
                              (int)((m >> 1) & 0x44444444u)};
             else
                 o.f[w] = v4i{(int)((m << 2) & 0x44444444u), (int)(m & 0x22222222u),
                              (int)((m >> 2) & 0x11111111u), (int)((m >> 3) & 0x11111111u)};
-            asm volatile("" : "+v"(o.f[w]));   // built here, not at its use
+            asm volatile("" : "+v"(o.f[w]));
         };
         // the products of o, and between them the building of the operands `on` of the
-        // next k-step (step h of the unit in r); READ: the registers of r take the next
+        // next k-step (step h of the unit in r); next: the registers of r take the next
         // unit's words as they come free.  Scheduling barriers and an empty asm at each
         // operand keep this order: left to itself, or to scheduling groups, the compiler
         // issues all products and then all the building.
         auto step = [&](const Ops& o, Ops& on, Raw& r, int h, bool next,
                         const uint8_t* unit) __attribute__((always_inline)) {
-    #pragma unroll
+            uint32_t m[2] = {0, 0};
+#pragma unroll
             for (int i = 0; i < NT * NT; i++) {
                 const int x = i / NT, y = i % NT;
                 const v4i f = o.f[x], c = o.f[NT + y];
@@ -236,10 +243,24 @@ __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
                     __builtin_shufflevector(f, f, 0, 1, 2, 3, -1, -1, -1, -1),
                     __builtin_shufflevector(c, c, 0, 1, 2, 3, -1, -1, -1, -1), acc[x][y], 4, 4, 0,
                     127, 0, 127);
-                if (NT == 2 || i % 2) {
-                    const int w = NT == 2 ? i : i / 2;
-                    match(r, w, h, on);
-                    if (next) read(unit, w, r);
+                if (NT == 2) {
+                    match(r, i, h, 0, PL, m[0]);
+                    if (next) read(unit, i, r);
+                    spread(m[0], i, on);
+                } else {
+                    const int w = i / 4 * 2;   // two operands to four products
+                    if (i % 4 < 2) {
+                        const int p0 = i % 4 ? (PL + 1) / 2 : 0, p1 = i % 4 ? PL : (PL + 1) / 2;
+                        match(r, w, h, p0, p1, m[0]);
+                        match(r, w + 1, h, p0, p1, m[1]);
+                        asm volatile("" : "+v"(m[0]), "+v"(m[1]));   // formed here, not at their use
+                        if (i % 4 && next) {
+                            read(unit, w, r);
+                            read(unit, w + 1, r);
+                        }
+                    } else {
+                        spread(m[i % 2], w + i % 2, on);
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -260,10 +281,14 @@ __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
             enter(u0);
             Raw r;
             Ops o0, o1;
-    #pragma unroll
+#pragma unroll
             for (int w = 0; w < 2 * NT; w++) read(sbase, w, r);
-    #pragma unroll
-            for (int w = 0; w < 2 * NT; w++) match(r, w, 0, o0);
+#pragma unroll
+            for (int w = 0; w < 2 * NT; w++) {
+                uint32_t m = 0;
+                match(r, w, 0, 0, PL, m);
+                spread(m, w, o0);
+            }
             // the operands built from the unit past the end (bytes of the last stage's
             // buffers) are not multiplied
             uint32_t k = 0;   // unit of the stage
@@ -280,14 +305,14 @@ __attribute__((amdgpu_waves_per_eu(1, NT == 4 ? 1 : 2))) void k_bicounts_fp4(
         const uint32_t qq = q * q;
         // r / q as a product: r < 2^15 and r * q < 2^20, so 2^20 / q rounded up is exact
         const uint32_t inv = ((1u << 20) + q - 1) / q;
-    #pragma unroll
+#pragma unroll
         for (int x = 0; x < NT; x++) {
-    #pragma unroll
+#pragma unroll
             for (int y = 0; y < NT; y++) {
                 const uint32_t c = cb * T + y * 32 + lr;
                 if (c >= Lq) continue;
                 const uint32_t jsite = (c * inv) >> 20, b = c - jsite * q;
-    #pragma unroll
+#pragma unroll
                 for (int e = 0; e < 16; e++) {
                     const uint32_t r = rb * T + x * 32 + 8 * (e / 4) + 4 * g + (e % 4);
                     if (r >= Lq) continue;
