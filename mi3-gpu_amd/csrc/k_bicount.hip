@@ -98,7 +98,7 @@ __device__ __forceinline__ void wait_vmem_bc() { __builtin_amdgcn_s_waitcnt(0x0F
 // NT = 2 is for problems too small for that (rule at the launch).
 //
 // Bound by the issue of the one wave that a SIMD holds: a matrix instruction takes 37
-// cycles (at 2.4 GHz) alone and one is issued every 59 here.  So the operands of a
+// cycles (at 2.4 GHz) alone and one is issued every 58 here.  So the operands of a
 // k-step are built between the products of the one before, evenly and two at a
 // time (their chains of dependent instructions otherwise stall; four at a time, or
 // the reads later, took 3-5% longer); reads are eight bytes wide (2.6 cycles of a CU;
@@ -106,9 +106,9 @@ __device__ __forceinline__ void wait_vmem_bc() { __builtin_amdgcn_s_waitcnt(0x0F
 // nibbles, this form with a fixed number of parts per block, with even shares,
 // and with this order of the building):
 //   L    q   sequences   8-bit  nibbles  planes  even shares  order
-//   232  21  1000003     10653     7020    5595         5533   4825
-//   232  21  262144       3103     2063    1661         1525   1381
-//   232  21  16384         459      400     378          207    199
+//   232  21  1000003     10653     7020    5595         5533   4783
+//   232  21  262144       3103     2063    1661         1525   1342
+//   232  21  16384         459      400     378          207    197
 //   150  12  100001        434      377     367          202    202
 //   93   4   262144        163       84      70           70     70
 //   99   4   16384          70       26      25           25     25
