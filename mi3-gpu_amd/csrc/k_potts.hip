@@ -1288,7 +1288,9 @@ __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(4, 
 
 // No staging: one wave per work-group, ROWS neighbouring rows at a time (of one
 // chunk, so that they share its partners), all their gathers of a chunk in
-// flight.  Lanes whose partner does not count read the row all the same.
+// flight.  Lanes whose partner does not count read the row all the same, and
+// select its couplings away (as a 0 factor, an infinite one would make NaN of
+// the energies of sequences that do not hold it, or hold it in a row that counts).
 template <int NC>
 __global__ __launch_bounds__(64) void k_energies_direct(
     const float* __restrict__ Ju, const uint8_t* __restrict__ seq, float* __restrict__ E,
@@ -1304,13 +1306,15 @@ __global__ __launch_bounds__(64) void k_energies_direct(
     for (uint32_t i0 = 0; i0 + 1 < L; i0 += ROWS) {
         const uint32_t kp = i0 >> 5;
         uint32_t base[ROWS][S];
-        float keep[ROWS];
+        // whether a coupling counts: in the first chunk those of partners past the
+        // row, then all; none in rows past the last, which repeat it
+        bool all[ROWS], counts[ROWS];
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            // rows past the last repeat it and count nothing
             const uint32_t i = i0 + r + 1 < L ? i0 + r : L - 2;
             w.row_bases(i, lane, q, j * 4 + i * NC * chb, base[r]);
-            keep[r] = i == i0 + r ? 1.f : 0.f;
+            all[r] = i == i0 + r;
+            counts[r] = all[r] && j > (i & 31);
         }
 #pragma unroll
         for (int k = 0; k < NC; k++) {
@@ -1322,8 +1326,8 @@ __global__ __launch_bounds__(64) void k_energies_direct(
                     rJ, base[r][0] + byte_x128(w.st[0][k >> 2], k & 3), k * chb, 0));
 #pragma unroll
             for (int r = 0; r < ROWS; r++) {
-                const float f = (uint32_t)k != kp || j > ((i0 + r) & 31) ? keep[r] : 0.f;
-                acc[0] = __fmaf_rn(v[r], f, acc[0]);
+                acc[0] += counts[r] ? v[r] : 0.f;
+                counts[r] = all[r];
             }
         }
     }

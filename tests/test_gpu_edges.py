@@ -1,0 +1,28 @@
+"""Sequences and couplings at the edges of what the engine accepts."""
+import numpy as np
+import pytest
+
+from test_gpu_kernels import make_gpu, model, seqs_rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,q,n", [(40, 4, 300), (65, 21, 515), (130, 9, 77)])
+def test_unstaged_energies_of_forbidden_pairs(gpu_ok, tmp_path, L, q, n):
+    """An infinite coupling makes the energies of the sequences that hold it infinite and no others:
+    pairs within a chunk of 32 sites, its last site, across chunks, and the last sites."""
+    J = model(L, q, 3)
+    s = seqs_rand(n, L, q, 4)
+    hold = np.zeros(n, bool)
+    for i, j in ((0, 1), (3, 31), (5, 20), (30, 31), (31, 32), (2, L - 2), (L - 3, L - 1), (L - 2, L - 1)):
+        J[i * (2 * L - i - 1) // 2 + j - i - 1, 1 * q + 2] = np.inf
+        hold |= (s[:, i] == 1) & (s[:, j] == 2)
+    assert hold.any() and not hold.all()
+    g = make_gpu(tmp_path, L, q, 512)
+    g.initLargeBufs(n)
+    g.setBuf('J', J)
+    g.setBuf('seq large', s)
+    g.calcEnergies('large')
+    E = g.getBuf('E large').read()
+    np.testing.assert_array_equal(np.isposinf(E), hold)
+    assert np.isfinite(E[~hold]).all()
