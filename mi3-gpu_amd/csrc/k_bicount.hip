@@ -29,8 +29,8 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 //   PL = 3 (q <= 7), PL = 5 (q <= 25).
 // A residue equals a letter where every plane agrees with the letter's bit: PL
 // instructions for 32 sequences.  Sequences past the end are all ones, which is
-// no residue.  The bits of a word are in the same order at every site, which is
-// all that a sum over sequences needs.
+// no residue, and so is a byte that takes more than PL bits.  The bits of a word
+// are in the same order at every site, which is all that a sum over sequences needs.
 template <int PL>
 __global__ __launch_bounds__(256) void k_pack_residues(const uint8_t* __restrict__ seq,
                                                        uint32_t ldseq, uint32_t nseq,
@@ -54,6 +54,14 @@ __global__ __launch_bounds__(256) void k_pack_residues(const uint8_t* __restrict
 #pragma unroll
         for (uint32_t e = 0; e < 4; e++) w[k >> 1][(k & 1) * 4 + e] = x[e];
     }
+    // bit 0 of a byte: it takes more than PL bits
+    constexpr uint32_t LOW = 0x01010101u * ((1u << PL) - 1);
+    uint32_t no[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            no[h][e] = (((w[h][e] & 0x7f7f7f7fu) + (0x7f7f7f7fu - LOW)) | w[h][e]) >> 7;
     uint2* o = reinterpret_cast<uint2*>(out + ((size_t)site * nunits + (c >> 1)) * (16 * PL) +
                                         (c & 1) * 8);
 #pragma unroll
@@ -62,7 +70,7 @@ __global__ __launch_bounds__(256) void k_pack_residues(const uint8_t* __restrict
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int e = 0; e < 8; e++) m[h] |= ((w[h][e] >> p) & 0x01010101u) << e;
+            for (int e = 0; e < 8; e++) m[h] |= (((w[h][e] >> p) | no[h][e]) & 0x01010101u) << e;
         o[2 * p] = make_uint2(m[0], m[1]);
     }
 }

@@ -2,9 +2,14 @@
 import numpy as np
 import pytest
 
+from mi3gpu._lib import lib, check
 from test_gpu_kernels import make_gpu, model, seqs_rand
 
 pytestmark = pytest.mark.gpu
+
+
+def _write(g, name, a):
+    check(g._ctx, lib().mi3_buf_write(g._ctx, name, a.ctypes.data, a.nbytes, 0))
 
 
 @pytest.mark.parametrize("L,q,n", [(40, 4, 300), (65, 21, 515), (130, 9, 77)])
@@ -18,7 +23,7 @@ def test_unstaged_energies_of_forbidden_pairs(gpu_ok, tmp_path, L, q, n):
         J[i * (2 * L - i - 1) // 2 + j - i - 1, 1 * q + 2] = np.inf
         hold |= (s[:, i] == 1) & (s[:, j] == 2)
     assert hold.any() and not hold.all()
-    g = make_gpu(tmp_path, L, q, 512)
+    g = make_gpu(tmp_path, L, q, 512, wgsize=512)
     g.initLargeBufs(n)
     g.setBuf('J', J)
     g.setBuf('seq large', s)
@@ -26,3 +31,20 @@ def test_unstaged_energies_of_forbidden_pairs(gpu_ok, tmp_path, L, q, n):
     E = g.getBuf('E large').read()
     np.testing.assert_array_equal(np.isposinf(E), hold)
     assert np.isfinite(E[~hold]).all()
+
+
+@pytest.mark.parametrize("L,q,n", [(5, 2, 129), (40, 4, 1000), (7, 7, 640), (9, 8, 640), (6, 25, 300)])
+def test_bicounts_bytes_that_are_no_letter(gpu_ok, tmp_path, L, q, n):
+    rng = np.random.default_rng(q)
+    s = seqs_rand(n, L, q, 5)
+    odd = rng.random(s.shape) < 0.3
+    s[odd] = rng.choice([q, 7, 8, 9, 31, 32, 33, 64, 127], size=odd.sum())
+    g = make_gpu(tmp_path, L, q, 512, wgsize=512)
+    g.initLargeBufs(n)
+    dev = np.zeros((L, g._seq_ld('seq large')), 'u1')
+    dev[:, :n] = s.T
+    _write(g, b'seq large', dev)
+    check(g._ctx, lib().mi3_calc_bicounts(g._ctx, b'seq large', n))
+    X = (s[:, :, None] == np.arange(q)).reshape(n, L * q).astype(np.int64)
+    want = (X.T @ X).reshape(L, q, L, q).transpose(0, 2, 1, 3).reshape(L, L, q * q)
+    np.testing.assert_array_equal(g.getBuf('bicount').read(), want[np.triu_indices(L, 1)])
