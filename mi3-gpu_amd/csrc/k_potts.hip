@@ -303,7 +303,9 @@ __device__ __forceinline__ uint32_t perm_apart(uint32_t hi, uint32_t lo, uint32_
 }
 
 // The walkers of a wave and what a step does with them around its gathers.
-// QB: q <= 16, so that a residue times q fits a byte.
+// QB: q <= 16, so that a residue times q fits a byte and four are multiplied at
+// once; bytes are cut to four bits as they are loaded, so that one that is no
+// residue does not reach its neighbours (cut at each step: 1% of a sweep).
 template <int KW, int S, bool QB>
 struct Walkers {
     static constexpr int SH = 5 - ilog2(S);  // lane j reduces and decides slot j >> SH
@@ -311,6 +313,7 @@ struct Walkers {
     static constexpr int R = S == 16 ? 2 : 4;
     static_assert((1 << ilog2(S)) == S && S <= 16, "S must be a power of two <= 16");
 
+    static constexpr uint32_t LETTER = QB ? 0x0f0f0f0fu : ~0u;
     static constexpr int NP = (S + 3) / 4;   // residues of a site, four slots to a word
 
     uint32_t st[S][KW];       // residues of sites j + 32k, four to a word
@@ -369,7 +372,7 @@ struct Walkers {
                         transpose4(v[0][d], v[1][d], v[2][d], v[3][d]);
 #pragma unroll
                         for (int g = 0; g < 4; g++)
-                            st[4 * d + g][i] = wfirst + 4 * d + g < end ? v[g][d] : 0u;
+                            st[4 * d + g][i] = wfirst + 4 * d + g < end ? v[g][d] & LETTER : 0u;
                     }
                 }
                 return;
@@ -387,7 +390,7 @@ struct Walkers {
                     uint32_t v = (valid && m < L) ? seq[(size_t)m * ldseq + wfirst + s] : 0u;
                     word |= v << (8 * e);
                 }
-                st[s][i] = word;
+                st[s][i] = word & LETTER;
             }
             asm volatile("" ::: "memory");
         }

@@ -1,4 +1,6 @@
 """Sequences and couplings at the edges of what the engine accepts."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -48,3 +50,30 @@ def test_bicounts_bytes_that_are_no_letter(gpu_ok, tmp_path, L, q, n):
     X = (s[:, :, None] == np.arange(q)).reshape(n, L * q).astype(np.int64)
     want = (X.T @ X).reshape(L, q, L, q).transpose(0, 2, 1, 3).reshape(L, L, q * q)
     np.testing.assert_array_equal(g.getBuf('bicount').read(), want[np.triu_indices(L, 1)])
+
+
+def test_a_byte_that_is_no_letter_stays_in_its_sequence(gpu_ok, tmp_path):
+    """q = 16: the letter 16 (at rows within the staged couplings) changes no other
+    sequence's energy and no other walker's chain."""
+    L, q, N = 40, 16, 2560
+    J = model(L, q, 3)
+    s = seqs_rand(N, L, q - 2, 4)
+    at = np.arange(0, N, 7)
+    res = []
+    for letter in (0, q):
+        g = make_gpu(tmp_path, L, q, N, seed=9, nsteps=L, wgsize=512)
+        dev = np.ascontiguousarray(s.T)
+        dev[3, at] = letter
+        g.setBuf('J', J)
+        _write(g, b'seq main', dev)
+        g.calcEnergies('main')
+        E = g.getBuf('E main').read()
+        g.runMCMC()
+        out = np.empty_like(dev)
+        t = ctypes.c_int()
+        check(g._ctx, lib().mi3_buf_read_async(g._ctx, b'seq main', out.nbytes, 0, ctypes.byref(t)))
+        check(g._ctx, lib().mi3_ticket_wait(g._ctx, t, out.ctypes.data, out.nbytes))
+        rest = np.setdiff1d(np.arange(N), at)
+        res.append((E[rest], out[:, rest]))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    np.testing.assert_array_equal(res[0][1], res[1][1])
