@@ -199,7 +199,10 @@ int mi3_calc_energies(mi3_ctx *ctx, const char *seqbuf, const char *Jbuf, const 
 
 /* "bicount"[pair][a*q+b] = #{n < nseq : s_i = a, s_j = b}, exact uint32.
  * Replaces calcBicounts (mcmcGPU.py:501-518) and countBivariate
- * (mcmc.cl:464-516). */
+ * (mcmc.cl:464-516).  The first count of a sequence buffer takes device memory
+ * of up to 5/8 of its size, which stays with the buffer; it may be captured into
+ * a graph.  (mi3_calc_energies and mi3_weighted_marg of many sequences of up to
+ * 5 letters use the same memory, and do without where there is none.) */
 int mi3_calc_bicounts(mi3_ctx *ctx, const char *seqbuf, uint32_t nseq);
 
 /* Number of parts that mi3_calc_bicounts plans for nseq sequences: with 1, a wave

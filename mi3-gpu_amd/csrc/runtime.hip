@@ -40,6 +40,7 @@ struct Buf {
     void* d = nullptr;
     size_t bytes = 0;
     uint64_t version = 0;
+    uint8_t* packed = nullptr;  // a sequence buffer's residues, packed or folded (packed_of)
 };
 
 struct Pinned {
@@ -96,7 +97,7 @@ struct mi3_ctx {
     uint64_t* wq = nullptr;                   // fixed-point weights
     size_t wq_cap = 0;
     unsigned long long* wacc = nullptr;       // fixed-point weighted-marginal bins
-    uint64_t wacc_cap = 0;
+    unsigned long long* wfold = nullptr;      // those of the folded model
     unsigned long long* probe_out = nullptr;  // sink of mi3_wm_atomic_probe
     uint32_t* wbad = nullptr;
     uint32_t* wm_units = nullptr;
@@ -107,8 +108,6 @@ struct mi3_ctx {
     // the reason in scratch_err, if its address could not be resolved)
     char* scratch = nullptr;
     std::string scratch_err;
-    uint8_t* packed = nullptr;                // residues packed for the bicounts
-    size_t packed_cap = 0;
     uint8_t* seq1 = nullptr;                  // one sequence (fill_seqs)
     // host staging
     std::vector<Pinned> pins;
@@ -229,7 +228,23 @@ int chunked_of(mi3_ctx* c, const char* name, float** out) {
     return MI3_OK;
 }
 
-// The folded model's couplings (k_fold_chunked; its size depends on L and q
+// Device memory of a fixed size, taken at its first use and never moved: a captured
+// graph may hold its address.  The first use may itself be captured, so the calling
+// thread leaves the capture modes that refuse to allocate.
+template <typename T>
+int workspace(mi3_ctx* c, T** p, size_t bytes) {
+    if (*p) return MI3_OK;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIPCHK(c, hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 1));
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return MI3_OK;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return fail(c, MI3_EHIP, "workspace of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
+}
+
+// The folded model's couplings (k_fold_chunked; their size depends on L and q
 // alone), rebuilt when stale.
 int folded_of(mi3_ctx* c, const char* name, float** out) {
     Buf* b;
@@ -241,7 +256,8 @@ int folded_of(mi3_ctx* c, const char* name, float** out) {
     for (uint32_t t = 1; t < k; t++) Q *= c->q;
     const uint32_t chf = chunk_floats(Q), nchunk = (nfold + 31) / 32;
     const uint32_t total = nfold * nchunk * chf;
-    if (!ch.d) HIPCHK(c, hipMalloc(&ch.d, total * sizeof(float)));
+    rc = workspace(c, &ch.d, total * sizeof(float));
+    if (rc) return rc;
     if (ch.version != b->version) {
         Scope s(c, "fold_couplings", total * 4ull);
         hipLaunchKernelGGL(k_fold_chunked, dim3(grid1(total)), dim3(256), 0, c->stream,
@@ -253,17 +269,15 @@ int folded_of(mi3_ctx* c, const char* name, float** out) {
     return MI3_OK;
 }
 
-// Workspace for packed residues, used in stream order; it is kept and grows to the
-// largest call's size.
-int packed_of(mi3_ctx* c, size_t bytes) {
-    if (c->packed_cap >= bytes) return MI3_OK;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    hipFree(c->packed);
-    c->packed = nullptr;
-    c->packed_cap = 0;
-    HIPCHK(c, hipMalloc(&c->packed, bytes));
-    c->packed_cap = bytes;
-    return MI3_OK;
+// Workspace for the residues of sequence buffer b, packed for the bicounts or folded
+// (at most 5/8 of the buffer's size), used in stream order and kept as long as
+// the buffer.
+int packed_of(mi3_ctx* c, Buf* b) {
+    const uint64_t ld = seq_ld(c, b);
+    uint64_t bytes = c->L * ((ld + BC_UNIT - 1) / BC_UNIT) * 16 * bc_planes(c->q);
+    if (const uint32_t k = fold_width(c->q); k > 1)
+        bytes = std::max(bytes, (c->L + k - 1) / k * ((ld + 31) / 32 * 32));
+    return workspace(c, &b->packed, bytes);
 }
 
 int pin_get(mi3_ctx* c, size_t bytes) {
@@ -426,7 +440,10 @@ int mi3_destroy(mi3_ctx* c) {
     if (!c) return MI3_OK;
     hipSetDevice(c->dev);
     if (c->stream) hipStreamSynchronize(c->stream);
-    for (auto& kv : c->bufs) hipFree(kv.second.d);
+    for (auto& kv : c->bufs) {
+        hipFree(kv.second.d);
+        hipFree(kv.second.packed);
+    }
     for (auto& kv : c->chunked) hipFree(kv.second.d);
     for (auto& kv : c->folded) hipFree(kv.second.d);
     for (auto& p : c->pins) hipHostFree(p.h);
@@ -441,10 +458,10 @@ int mi3_destroy(mi3_ctx* c) {
     hipFree(c->red_out);
     hipFree(c->wq);
     hipFree(c->wacc);
+    hipFree(c->wfold);
     hipFree(c->probe_out);
     hipFree(c->wbad);
     hipFree(c->wm_units);
-    hipFree(c->packed);
     hipFree(c->seq1);
     if (c->t0) hipEventDestroy(c->t0);
     if (c->stream) hipStreamDestroy(c->stream);
@@ -813,7 +830,7 @@ int mi3_gen_indep(mi3_ctx* c, const char* seqbuf) {
 int mi3_calc_energies(mi3_ctx* c, const char* seqbuf, const char* Jbuf, const char* Ebuf,
                       uint32_t nseq) {
     if (!c) return MI3_EINVAL;
-    Buf *sb, *eb;
+    Buf *sb, *eb, *jb;
     int rc = need(c, seqbuf, (size_t)c->L, &sb);
     if (rc) return rc;
     size_t ld = seq_ld(c, sb);
@@ -828,24 +845,27 @@ int mi3_calc_energies(mi3_ctx* c, const char* seqbuf, const char* Jbuf, const ch
     a.L = c->L;
     a.q = c->q;
     a.ncu = c->ncu;
-    const uint32_t k = ld % 16 ? 1 : fold_sites(c->q, c->L, nseq, c->ncu);
+    rc = need(c, Jbuf, (size_t)c->nP * c->q * c->q * sizeof(float), &jb);
+    if (rc) return rc;
+    uint32_t k = ld % 16 ? 1 : fold_sites(c->q, c->L, nseq, c->ncu);
+    float* Ju;
+    // (without memory for the folded model or its sequences: the sites as they are)
+    if (k > 1 && (packed_of(c, sb) || folded_of(c, Jbuf, &Ju))) k = 1;
     if (k > 1) {
         a.L = (c->L + k - 1) / k;
         for (uint32_t t = 1; t < k; t++) a.q *= c->q;
         a.ld = (nseq + 31) / 32 * 32;
-        rc = packed_of(c, (size_t)a.L * a.ld);
+    } else {
+        rc = chunked_of(c, Jbuf, &Ju);
         if (rc) return rc;
     }
     a.nchunk = (a.L + 31) / 32;
-    float* Ju;
-    rc = k > 1 ? folded_of(c, Jbuf, &Ju) : chunked_of(c, Jbuf, &Ju);
-    if (rc) return rc;
     a.Ju = Ju;
     Scope s(c, "getEnergies", (size_t)nseq * (c->L + 4));
     if (k > 1) {
         hipLaunchKernelGGL(k_fold_residues, dim3((a.ld / 16 + 255) / 256, a.L), dim3(256), 0, c->stream,
-                           a.seq, (uint32_t)ld, c->L, c->q, k, c->packed, a.ld);
-        a.seq = c->packed;
+                           a.seq, (uint32_t)ld, c->L, c->q, k, sb->packed, a.ld);
+        a.seq = sb->packed;
     }
     HIPCHK(c, launch_energies(a, c->stream));
     eb->version++;
@@ -871,21 +891,20 @@ int mi3_calc_bicounts(mi3_ctx* c, const char* seqbuf, uint32_t nseq) {
     Scope s(c, "calcBicounts", (size_t)nseq * c->L);
     // residues packed to bit planes (16 bytes a plane per 128 sequences of a site)
     const uint32_t planes = bc_planes(c->q), nunits = (nseq + BC_UNIT - 1) / BC_UNIT;
-    const size_t pk_bytes = (size_t)c->L * nunits * 16 * planes;
+    rc = packed_of(c, sb);
+    if (rc) return rc;
     if (ksplit > 1 || nunits == 0 || nunits > BC_PART) {   // no wave stores a whole block
         int frc = fill_u32_dev(c, cb->d, 0u, (uint64_t)c->nP * c->q * c->q);
         if (frc) return frc;
     }
-    rc = packed_of(c, pk_bytes);
-    if (rc) return rc;
     if (nunits) {
         const dim3 grid((nunits * 2 + 255) / 256, c->L);
         if (planes == 3)
             hipLaunchKernelGGL(k_pack_residues<3>, grid, dim3(256), 0, c->stream,
-                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, c->packed);
+                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, sb->packed);
         else
             hipLaunchKernelGGL(k_pack_residues<5>, grid, dim3(256), 0, c->stream,
-                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, c->packed);
+                               (const uint8_t*)sb->d, (uint32_t)ld, nseq, nunits, sb->packed);
     }
     // 128 x 128 blocks where those, times the parts, fill the card's SIMDs with a wave
     // each; below, 64 x 64 blocks, two waves to a SIMD.  The waves that the card holds
@@ -902,7 +921,7 @@ int mi3_calc_bicounts(mi3_ctx* c, const char* seqbuf, uint32_t nseq) {
     const size_t lds = bc_lds_bytes(c->q, tile, stage);
 #define MI3_BC(NT, PL, ST)                                                                     \
     hipLaunchKernelGGL((k_bicounts_fp4<NT, PL, ST>), grid, dim3(64), lds, c->stream,            \
-                       (const uint8_t*)c->packed, nunits, c->L, c->q, nb,                       \
+                       (const uint8_t*)sb->packed, nunits, c->L, c->q, nb,                      \
                        (uint64_t)ntiles * nunits,                                              \
                        (uint32_t*)cb->d)
     if (planes == 5) {
@@ -975,15 +994,26 @@ int mi3_weighted_marg(mi3_ctx* c, const char* seqbuf, const char* wbuf, uint32_t
     if ((uint64_t)c->nP * nseq < (Q * Q << 20)) k = 1;
     uint32_t L = c->L, q = c->q, wld = (uint32_t)ld, n_units = c->n_units, split = c->wm_split;
     const uint8_t* seq = (const uint8_t*)sb->d;
+    uint64_t nacc = nbins;
     if (k > 1) {
-        L = (c->L + k - 1) / k;
-        q = (uint32_t)Q;
-        wld = (nseq + 31) / 32 * 32;
-        rc = packed_of(c, (size_t)L * wld);
-        if (rc) return rc;
-        seq = c->packed;
+        const uint32_t nfold = (c->L + k - 1) / k;
+        const uint64_t folded_bins = (uint64_t)(nfold * (nfold - 1) / 2) * Q * Q;
+        // (without memory for it: the sites as they are)
+        if (packed_of(c, sb) || workspace(c, &c->wfold, folded_bins * sizeof(unsigned long long))) {
+            k = 1;
+        } else {
+            L = nfold;
+            q = (uint32_t)Q;
+            wld = (nseq + 31) / 32 * 32;
+            seq = sb->packed;
+            nacc = folded_bins;
+        }
     }
-    const uint64_t nacc = (uint64_t)(L * (L - 1) / 2) * q * q;
+    if (k == 1) {
+        rc = workspace(c, &c->wacc, nbins * sizeof(unsigned long long));
+        if (rc) return rc;
+    }
+    unsigned long long* acc = k > 1 ? c->wfold : c->wacc;
     size_t lds = (size_t)q * q * WM_COLS * sizeof(unsigned long long);
     if (k > 1) {
         // fewer units, their sequences split: a part's adds take about 5 cycles a
@@ -994,14 +1024,6 @@ int mi3_weighted_marg(mi3_ctx* c, const char* seqbuf, const char* wbuf, uint32_t
         split = (uint32_t)std::sqrt(14.0 * nseq / ((double)n_units * q * q));
         if (split > c->ncu / n_units) split = c->ncu / n_units;
         if (split < 1) split = 1;
-    }
-    if (c->wacc_cap < nacc) {
-        if (c->wacc) HIPCHK(c, hipStreamSynchronize(c->stream));
-        hipFree(c->wacc);
-        c->wacc = nullptr;
-        c->wacc_cap = 0;
-        HIPCHK(c, hipMalloc(&c->wacc, nacc * sizeof(unsigned long long)));
-        c->wacc_cap = nacc;
     }
     HIPCHK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(k_weighted_marg),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1017,23 +1039,23 @@ int mi3_weighted_marg(mi3_ctx* c, const char* seqbuf, const char* wbuf, uint32_t
                        (const float*)wb->d, nseq, (const float*)c->red_out, c->wq, c->wbad);
     if (k > 1)
         hipLaunchKernelGGL(k_fold_residues, dim3((wld / 16 + 255) / 256, L), dim3(256), 0, c->stream,
-                           (const uint8_t*)sb->d, (uint32_t)ld, c->L, c->q, k, c->packed, wld);
+                           (const uint8_t*)sb->d, (uint32_t)ld, c->L, c->q, k, sb->packed, wld);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid1(2 * nacc)), dim3(256), 0, c->stream,
-                       (uint32_t*)c->wacc, 0u, 2 * nacc);
+                       (uint32_t*)acc, 0u, 2 * nacc);
     hipLaunchKernelGGL(k_weighted_marg, dim3(n_units * split), dim3(WM_THREADS), lds, c->stream, seq,
                        wld, nseq, (const uint64_t*)c->wq, L, q, (const uint32_t*)c->wm_units, split,
-                       c->wacc, 0u);
+                       acc, 0u);
     if (k > 1) {
         auto unfold = c->q == 2 ? k_unfold_to_float<2, 3> : c->q == 3 ? k_unfold_to_float<3, 2>
                       : c->q == 4 ? k_unfold_to_float<4, 2> : k_unfold_to_float<5, 2>;
         hipLaunchKernelGGL(unfold, dim3(grid1((uint64_t)(c->L - 1) * c->q * c->q), c->L - 1),
-                           dim3(256), 0, c->stream, (const unsigned long long*)c->wacc,
+                           dim3(256), 0, c->stream, (const unsigned long long*)acc,
                            (float*)bb->d, c->L, L, (const float*)c->red_out,
                            (const uint32_t*)c->wbad);
     }
     else
         hipLaunchKernelGGL(k_fixed_to_float, dim3(grid1(nbins)), dim3(256), 0, c->stream,
-                           (const unsigned long long*)c->wacc, (float*)bb->d, nbins,
+                           (const unsigned long long*)acc, (float*)bb->d, nbins,
                            (const float*)c->red_out, (const uint32_t*)c->wbad);
     HIPCHK(c, hipGetLastError());
     bb->version++;

@@ -1,4 +1,5 @@
-"""Sequences and couplings at the edges of what the engine accepts."""
+"""Sequences and couplings at the edges of what the engine accepts, and its
+calls under graph capture."""
 import ctypes
 
 import numpy as np
@@ -77,3 +78,58 @@ def test_a_byte_that_is_no_letter_stays_in_its_sequence(gpu_ok, tmp_path):
         res.append((E[rest], out[:, rest]))
     np.testing.assert_array_equal(res[0][0], res[1][0])
     np.testing.assert_array_equal(res[0][1], res[1][1])
+
+
+class _Graph:
+    """What a block of calls enqueues on a context's stream, captured."""
+
+    def __init__(self, g):
+        self.s = ctypes.c_void_p()
+        check(g._ctx, lib().mi3_stream(g._ctx, ctypes.byref(self.s)))
+
+    def _hip(self, name, *a):
+        f = getattr(lib(), name)      # from the HIP runtime that the library is linked to
+        f.restype = ctypes.c_int
+        assert f(*a) == 0, name
+
+    def __enter__(self):
+        self._hip('hipStreamBeginCapture', self.s, 1)
+        return self
+
+    def __exit__(self, *exc):
+        self.graph, self.exec = ctypes.c_void_p(), ctypes.c_void_p()
+        f = lib().hipStreamEndCapture
+        f.restype = ctypes.c_int
+        rc = f(self.s, ctypes.byref(self.graph))
+        if exc[0] is None:
+            assert rc == 0
+            self._hip('hipGraphInstantiate', ctypes.byref(self.exec), self.graph, None, None, ctypes.c_size_t(0))
+
+    def launch(self):
+        self._hip('hipGraphLaunch', self.exec, self.s)
+
+    def close(self):
+        self._hip('hipGraphExecDestroy', self.exec)
+        self._hip('hipGraphDestroy', self.graph)
+
+
+@pytest.mark.parametrize("L,q", [(30, 4), (40, 21)])
+def test_bicounts_captured(gpu_ok, tmp_path, L, q):
+    """The context's first count is captured; replays stay right when larger sets are counted between."""
+    from oracle import cboracle
+    N, n = 1024, 9000
+    a, b = seqs_rand(N, L, q, 1), seqs_rand(n, L, q, 2)
+    g = make_gpu(tmp_path, L, q, N)
+    g.initLargeBufs(n)
+    g.setBuf('seq main', a)
+    g.setBuf('seq large', b)
+    with _Graph(g) as cap:
+        g.calcBicounts('main')
+    wa, wb = cboracle.bicounts(a, q), cboracle.bicounts(b, q)
+    for k in range(3):
+        cap.launch()
+        np.testing.assert_array_equal(g.getBuf('bicount').read(), wa)
+        g.calcBicounts('large')
+        g.wait()
+        np.testing.assert_array_equal(g.getBuf('bicount').read(), wb)
+    cap.close()
