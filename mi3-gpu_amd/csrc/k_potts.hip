@@ -951,13 +951,24 @@ template <int KW, int S, int NWAVES, int PF>
 __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(NWAVES / 4, NWAVES / 4))) void
 k_sweep_batch(const BatchModel* __restrict__ models, const BatchTile* __restrict__ tiles,
               uint32_t ntiles, uint32_t* __restrict__ counter) {
-    __shared__ uint32_t s_tile;
+    // the tile's number; two chunks of q > 21 take all of the LDS, so there it goes
+    // through their first word
+    constexpr bool OWN_WORD = PF < 10;
+    uint32_t* s_tile;
+    if constexpr (OWN_WORD) {
+        __shared__ uint32_t word;
+        s_tile = &word;
+    } else {
+        extern __shared__ f4v lds4[];
+        s_tile = reinterpret_cast<uint32_t*>(lds4);
+    }
     for (;;) {
         __syncthreads();   // previous tile's LDS reads done; s_tile free
-        if (threadIdx.x == 0) s_tile = atomicAdd(counter, 1u);
+        if (threadIdx.x == 0) *s_tile = atomicAdd(counter, 1u);
         __syncthreads();
-        const uint32_t t = __builtin_amdgcn_readfirstlane(s_tile);  // uniform: scalar loads below
+        const uint32_t t = __builtin_amdgcn_readfirstlane(*s_tile);  // uniform: scalar loads below
         if (t >= ntiles) break;
+        if constexpr (!OWN_WORD) __syncthreads();   // read by all before a copy overwrites it
         const BatchTile tl = tiles[t];
         const BatchModel m = uniform_model(models[tl.model]);
         const uint64_t step0 = uniform64(*m.step);
