@@ -336,10 +336,12 @@ int mi3_batch_get_seqs(mi3_batch *b, uint32_t model, uint8_t *out);
 int mi3_batch_run(mi3_batch *b, uint32_t nsweeps);
 int mi3_batch_synchronize(mi3_batch *b);
 
-/* Autotuner: for every class, time each allowed walkers-per-tile choice
- * (128, 256, 512; the largest leaves the form to the library, as for
- * mi3_set_wgsize) on nsweeps sweeps of its models and
- * keep the fastest.  The timed sweeps are real MCMC steps of the walkers. */
+/* A class is swept in the form and tile that the library chooses by its walkers,
+ * until mi3_batch_set_tile asks for staged tiles of 128, 256 or 512 walkers (256
+ * at most beyond 512 sites), or the autotuner, which times those and the
+ * library's choice on nsweeps sweeps of the class's models, keeps the fastest.
+ * The timed sweeps are real MCMC steps of the walkers.  mi3_batch_tile tells the
+ * walkers per tile asked for or kept, or the most where the library chooses. */
 int mi3_batch_tune(mi3_batch *b, uint32_t nsweeps);
 int mi3_batch_tile(mi3_batch *b, uint32_t model, uint32_t *wpb);
 int mi3_batch_set_tile(mi3_batch *b, uint32_t model, uint32_t wpb);

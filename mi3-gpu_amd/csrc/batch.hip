@@ -54,7 +54,7 @@ struct ClassKey {
 
 struct ClassRun {
     std::vector<uint32_t> models;
-    uint32_t wpb = 0;        // chosen walkers per tile (the largest: the library's choice)
+    uint32_t wpb = 0;        // walkers per tile asked for, or the most (the library's choice)
     uint32_t run_wpb = 0;    // walkers per tile as run
     bool direct = false;     // swept without staging
     BatchTile* tiles = nullptr;
@@ -117,26 +117,27 @@ std::vector<uint32_t> tile_options(uint32_t kw) {
     return {128, 256, 512};
 }
 
-// Tiles of a class for a walkers-per-tile choice; larger models first so
-// that the tail of the persistent loop is short.  The largest tile stands for
-// the library's choice, as the single-model sweep makes it: no staging for a
-// class of few walkers (more than a single model's, since classes without
-// staging follow one another), else smaller tiles where they leave most of the
-// card free (8 models of 1024-4096 walkers: 4 sweeps took 30.6 ms in
-// tiles of 512, all on the two work-groups of the L=400 model).
+// Tiles of a class of `wpb` walkers, staged, or (0) by the library's choice; larger
+// models first so that the tail of the persistent loop is short.  The choice is the
+// single-model sweep's: no staging for a class of few walkers (more than a single
+// model's, since classes without staging follow one another), else tiles of the
+// most walkers, or smaller where those leave most of the card free (8 models of
+// 1024-4096 walkers: 4 sweeps took 30.6 ms in tiles of 512, all on the two
+// work-groups of the L=400 model).
 int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
-    uint64_t total = 0;
-    uint32_t qmin = MAX_Q;
-    for (uint32_t m : cr.models) {
-        total += b->N[m];
-        qmin = std::min(qmin, b->q[m]);
-    }
-    const uint32_t ncu = b->ncu ? b->ncu : 256;
     cr.direct = false;
-    cr.run_wpb = wpb;
-    if (wpb == tile_options(key.kw).back()) {
+    cr.wpb = cr.run_wpb = wpb;
+    if (wpb == 0) {
+        uint64_t total = 0;
+        uint32_t qmin = MAX_Q;
+        for (uint32_t m : cr.models) {
+            total += b->N[m];
+            qmin = std::min(qmin, b->q[m]);
+        }
+        const uint32_t ncu = b->ncu ? b->ncu : 256;
+        cr.wpb = tile_options(key.kw).back();
         cr.direct = total <= (uint64_t)(qmin <= 8 ? 24 : 32) * ncu;
-        cr.run_wpb = chunk_tile((uint32_t)std::min<uint64_t>(total, 1u << 30), wpb, ncu);
+        cr.run_wpb = chunk_tile((uint32_t)std::min<uint64_t>(total, 1u << 30), cr.wpb, ncu);
     }
     std::vector<BatchTile> t;
     std::vector<uint32_t> order = cr.models;
@@ -149,7 +150,6 @@ int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
     BCHK(b, hipMalloc(&cr.tiles, std::max<size_t>(1, t.size()) * sizeof(BatchTile)));
     BCHK(b, hipMemcpy(cr.tiles, t.data(), t.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
     cr.ntiles = (uint32_t)t.size();
-    cr.wpb = wpb;
     return MI3_OK;
 }
 
@@ -342,8 +342,7 @@ int mi3_batch_create(int device, uint32_t nmodels, const uint32_t* L, const uint
         for (auto& kv : b->classes) {
             if (rc != MI3_OK) break;
             if (hipStreamCreate(&kv.second.side) != hipSuccess) { bad("stream"); break; }
-            // default tile: the largest allowed
-            if (build_tiles(b, kv.first, kv.second, tile_options(kv.first.kw).back()) != MI3_OK)
+            if (build_tiles(b, kv.first, kv.second, 0) != MI3_OK)
                 bad("tiles");
         }
         if (hipStreamSynchronize(b->stream) != hipSuccess) bad("sync");
@@ -470,8 +469,10 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
     for (auto& kv : b->classes) {
         ClassRun& cr = kv.second;
         float best = 1e30f;
-        uint32_t best_w = cr.wpb;
-        for (uint32_t w : tile_options(kv.first.kw)) {
+        uint32_t best_w = 0;
+        std::vector<uint32_t> opts = tile_options(kv.first.kw);
+        opts.push_back(0);   // the library's choice
+        for (uint32_t w : opts) {
             rc = build_tiles(b, kv.first, cr, w);
             if (rc) break;
             // positions for this launch, then the class sweep alone; the

@@ -34,3 +34,37 @@ def test_batch_of_the_largest_alphabets(gpu_ok, tile):
     for m, (L, q, N) in enumerate(models):
         _check_model(b.get_seqs(m), data[m][1], data[m][0], 40 + m, [(0, L), (L + (L & 1), L)])
     b.close()
+
+
+# state words of one to five and more, chunks of each class
+STAGED = [[(20, 4, 20480), (17, 2, 512)], [(24, 21, 17408), (33, 17, 1024)], [(131, 9, 18432)], [(260, 3, 16896)],
+          [(24, 12, 8704), (12, 16, 512)], [(390, 17, 1024)], [(520, 4, 8704)]]
+
+
+@pytest.mark.parametrize("models", STAGED)
+@pytest.mark.parametrize("tile", [None, 128, 256, 512])
+def test_batch_staged_tiles(gpu_ok, models, tile):
+    """Tiles asked for by size, and, for classes of many walkers, the library's choice."""
+    b, data = _batch(models, tile)
+    b.run(1)
+    b.run(1)
+    for m, (L, q, N) in enumerate(models):
+        _check_model(b.get_seqs(m), data[m][1], data[m][0], 40 + m, [(0, L), (L + (L & 1), L)])
+        assert b.tile(m) == min(tile or 512, 256 if L > 512 else 512)
+    b.close()
+
+
+# 2049 to 8192 walkers of more than 8 letters (four to a half-wave), one model or
+# several, state words of one to five; and one to a half-wave
+UNSTAGED = [[(40, 21, 1536), (33, 17, 1536), (37, 21, 512)], [(140, 9, 2560), (129, 16, 1024)], [(260, 12, 2560)],
+            [(390, 21, 2560)], [(520, 9, 2560)], [(30, 25, 1024), (21, 22, 2048)], [(50, 4, 3584), (64, 8, 512)]]
+
+
+@pytest.mark.parametrize("models", UNSTAGED)
+def test_batch_unstaged(gpu_ok, models):
+    b, data = _batch(models)
+    b.run(1)
+    b.run(1)
+    for m, (L, q, N) in enumerate(models):
+        _check_model(b.get_seqs(m), data[m][1], data[m][0], 40 + m, [(0, L), (L + (L & 1), L)])
+    b.close()
