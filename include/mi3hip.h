@@ -336,10 +336,10 @@ int mi3_batch_get_seqs(mi3_batch *b, uint32_t model, uint8_t *out);
 int mi3_batch_run(mi3_batch *b, uint32_t nsweeps);
 int mi3_batch_synchronize(mi3_batch *b);
 
-/* A class is swept in the form and tile that the library chooses by its walkers,
+/* A class is swept in the form and tile that the library chooses for the batch,
  * until mi3_batch_set_tile asks for staged tiles of 128, 256 or 512 walkers (256
- * at most beyond 512 sites), or the autotuner, which times those and the
- * library's choice on nsweeps sweeps of the class's models, keeps the fastest.
+ * at most beyond 512 sites), or the autotuner, which times those and the unstaged
+ * form on nsweeps sweeps of the class's models, keeps what is fastest together.
  * The timed sweeps are real MCMC steps of the walkers.  mi3_batch_tile tells the
  * walkers per tile asked for or kept, or the most where the library chooses. */
 int mi3_batch_tune(mi3_batch *b, uint32_t nsweeps);

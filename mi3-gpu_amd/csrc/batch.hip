@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <map>
 #include <string>
@@ -54,8 +55,8 @@ struct ClassKey {
 
 struct ClassRun {
     std::vector<uint32_t> models;
-    uint32_t wpb = 0;        // walkers per tile asked for, or the most (the library's choice)
-    uint32_t run_wpb = 0;    // walkers per tile as run
+    bool fixed = false;      // form and tile asked for, or kept by the autotuner
+    uint32_t wpb = 0;        // walkers per tile
     bool direct = false;     // swept without staging
     BatchTile* tiles = nullptr;
     uint32_t ntiles = 0;
@@ -117,44 +118,157 @@ std::vector<uint32_t> tile_options(uint32_t kw) {
     return {128, 256, 512};
 }
 
-// Tiles of a class of `wpb` walkers, staged, or (0) by the library's choice; larger
-// models first so that the tail of the persistent loop is short.  The choice is the
-// single-model sweep's: no staging for a class of few walkers (more than a single
-// model's, since classes without staging follow one another), else tiles of the
-// most walkers, or smaller where those leave most of the card free (8 models of
-// 1024-4096 walkers: 4 sweeps took 30.6 ms in tiles of 512, all on the two
-// work-groups of the L=400 model).
-int build_tiles(mi3_batch* b, const ClassKey& key, ClassRun& cr, uint32_t wpb) {
-    cr.direct = false;
-    cr.wpb = cr.run_wpb = wpb;
-    if (wpb == 0) {
-        uint64_t total = 0;
-        uint32_t qmin = MAX_Q;
-        for (uint32_t m : cr.models) {
-            total += b->N[m];
-            qmin = std::min(qmin, b->q[m]);
+uint32_t units(const mi3_batch* b) { return b->ncu ? b->ncu : 256; }
+
+// Walkers up to which a class may be swept unstaged.  Beyond, the rows that its
+// waves read at a time leave the L2s (us a step, unstaged and in tiles of 128:
+// 8192 walkers of L=232 q=21 5.6 and 6.9, L=93 2.5 and 2.8, but L=300 11.0 and
+// 8.6, L=400 19 and 11; 4096 of L=300 4.1 and 8.6, L=600 8.8 and 20).
+bool may_be_unstaged(const mi3_batch* b, const ClassKey& key, const ClassRun& cr) {
+    uint64_t total = 0;
+    for (uint32_t m : cr.models) total += b->N[m];
+    return total <= (uint64_t)(key.pf == 1 ? 24 : key.kw <= 2 ? 32 : 16) * units(b);
+}
+
+// A class whose couplings an XCD's L2 holds (4 MiB).
+bool l2_resident(const mi3_batch* b, const ClassRun& cr) {
+    uint64_t bytes = 0;
+    for (uint32_t m : cr.models) bytes += (uint64_t)b->L[m] * b->nchunk[m] * b->q[m] * b->q[m] * CH * 4;
+    return bytes <= 4u << 20;
+}
+
+// Times of a sweep of a class alone on the card: unstaged; staged, and then its
+// share of the card's CUs.
+struct ClassTimes {
+    double direct, staged, card;
+    bool resident;
+};
+
+// What a batch takes whose classes d are swept unstaged: those run one after
+// another, and the staged ones beside each other, after them or beside those
+// whose couplings the L2s hold (enqueue_round).
+double batch_time(const std::vector<ClassTimes>& t, const std::vector<bool>& d) {
+    double first = 0, beside = 0, longest = 0, card = 0;
+    for (size_t i = 0; i < t.size(); i++) {
+        if (d[i]) {
+            (t[i].resident ? beside : first) += t[i].direct;
+        } else {
+            longest = std::max(longest, t[i].staged);
+            card += t[i].card;
         }
-        const uint32_t ncu = b->ncu ? b->ncu : 256;
-        cr.wpb = tile_options(key.kw).back();
-        cr.direct = total <= (uint64_t)(qmin <= 8 ? 24 : 32) * ncu;
-        cr.run_wpb = chunk_tile((uint32_t)std::min<uint64_t>(total, 1u << 30), cr.wpb, ncu);
     }
+    return first + std::max(std::max(longest, card), beside);
+}
+
+// The classes to sweep unstaged: of those that may be, the first of the longest
+// staged ones, the first two, and so on are tried; times(d) gives the classes'
+// times if the classes d are unstaged.
+template <typename F>
+std::vector<bool> choose_unstaged(const std::vector<bool>& may, F times) {
+    std::vector<bool> d(may.size(), false), best = d;
+    const std::vector<ClassTimes> t = times(d);
+    std::vector<size_t> order;
+    for (size_t i = 0; i < may.size(); i++)
+        if (may[i]) order.push_back(i);
+    std::sort(order.begin(), order.end(),
+              [&](size_t x, size_t y) { return t[x].staged > t[y].staged; });
+    double least = batch_time(t, d);
+    for (size_t i : order) {
+        d[i] = true;
+        const double all = batch_time(times(d), d);
+        if (all < least) {
+            least = all;
+            best = d;
+        }
+    }
+    return best;
+}
+
+// Estimate of those times in tiles of w walkers, in us (within a fifth of what
+// L=40 to 1000 with 512 to 8192 walkers took, to where may_be_unstaged ends).  An
+// unstaged step waits for its gathers, and shares the L2s' lines (as many of a
+// chunk as its 32 sites have letters) with the class's other walkers; a staged
+// step takes the copies of its chunks, or the gathers of the tile's walkers.
+ClassTimes estimate(const mi3_batch* b, const ClassKey& key, const ClassRun& cr, uint32_t w) {
+    static const double per_chunk[4][3] = {
+        {0.37, 0.55, 0.92}, {0.66, 0.70, 1.0}, {0.90, 0.94, 1.05}, {1.15, 1.2, 1.3}};
+    const double chunk = per_chunk[key.pf == 1 ? 0 : key.pf == 4 ? 1 : key.pf == 7 ? 2 : 3]
+                                  [w == 128 ? 0 : w == 256 ? 1 : 2] *
+                         (key.kw >= 5 && key.pf > 1 ? 1.15 : key.kw == 4 && w == 512 ? 1.2 : 1.0);
+    ClassTimes t{0, 0, 0, l2_resident(b, cr)};
+    double gathers = 0, tiles = 0;
+    for (uint32_t m : cr.models) {
+        const double L = b->L[m], q = b->q[m], nc = b->nchunk[m];
+        t.direct = std::max(t.direct, L * (0.55 + 0.05 * nc));
+        gathers += L * nc * b->N[m] * q * (1 - std::pow(1 - 1 / q, 32)) * 4.9e-6;
+        const double step = L * (0.3 + chunk * nc);
+        t.staged = std::max(t.staged, step);
+        tiles += step * (b->N[m] / w);
+    }
+    t.direct += gathers;
+    t.card = tiles / units(b);
+    t.staged = std::max(t.staged, t.card);
+    return t;
+}
+
+// Tiles of a class of w walkers; larger models first so that the tail of the
+// persistent loop is short.
+int build_tiles(mi3_batch* b, ClassRun& cr, uint32_t w, bool direct) {
     std::vector<BatchTile> t;
     std::vector<uint32_t> order = cr.models;
     std::stable_sort(order.begin(), order.end(),
                      [&](uint32_t x, uint32_t y) { return b->L[x] > b->L[y]; });
     for (uint32_t m : order)
-        for (uint32_t blk = 0; blk < b->N[m] / cr.run_wpb; blk++) t.push_back({m, blk});
+        for (uint32_t blk = 0; blk < b->N[m] / w; blk++) t.push_back({m, blk});
     if (cr.tiles) hipFree(cr.tiles);
     cr.tiles = nullptr;
     BCHK(b, hipMalloc(&cr.tiles, std::max<size_t>(1, t.size()) * sizeof(BatchTile)));
     BCHK(b, hipMemcpy(cr.tiles, t.data(), t.size() * sizeof(BatchTile), hipMemcpyHostToDevice));
     cr.ntiles = (uint32_t)t.size();
+    cr.wpb = w;
+    cr.direct = direct;
+    return MI3_OK;
+}
+
+// Forms and tiles of the classes that nobody fixed: tiles of the most walkers, or
+// smaller where all staged classes' together leave most of the card free.
+int choose_tiles(mi3_batch* b) {
+    std::vector<bool> may;
+    for (auto& kv : b->classes) may.push_back(!kv.second.fixed && may_be_unstaged(b, kv.first, kv.second));
+    auto tile = [&](const std::vector<bool>& d) {
+        uint64_t walkers = 0;
+        size_t i = 0;
+        for (auto& kv : b->classes)
+            if (!d[i++])
+                for (uint32_t m : kv.second.models) walkers += b->N[m];
+        // (a third of the card: three batches beside each other find room)
+        return chunk_tile((uint32_t)std::min<uint64_t>(walkers, 1u << 30), 512, units(b) * 4 / 3);
+    };
+    auto class_tile = [](const ClassKey& key, uint32_t w) {
+        return std::min(w, tile_options(key.kw).back());
+    };
+    const std::vector<bool> direct = choose_unstaged(may, [&](const std::vector<bool>& d) {
+        std::vector<ClassTimes> t;
+        const uint32_t w = tile(d);
+        for (auto& kv : b->classes) {
+            const ClassRun& cr = kv.second;
+            t.push_back(estimate(b, kv.first, cr, cr.fixed ? cr.wpb : class_tile(kv.first, w)));
+            if (cr.fixed && cr.direct) t.back().staged = t.back().card = t.back().direct;
+        }
+        return t;
+    });
+    const uint32_t w = tile(direct);
+    size_t i = 0;
+    for (auto& kv : b->classes) {
+        if (!kv.second.fixed)
+            if (const int rc = build_tiles(b, kv.second, class_tile(kv.first, w), direct[i])) return rc;
+        i++;
+    }
     return MI3_OK;
 }
 
 uint32_t class_grid(mi3_batch* b, const ClassRun& cr) {
-    return std::min<uint32_t>(cr.ntiles, b->ncu ? b->ncu : 256);
+    return std::min<uint32_t>(cr.ntiles, units(b));
 }
 
 // The sweep of one class on stream st.
@@ -163,10 +277,10 @@ hipError_t sweep_class(mi3_batch* b, const ClassKey& key, const ClassRun& cr, ui
     if (cr.direct) {
         uint32_t qmin = MAX_Q;
         for (uint32_t m : cr.models) qmin = std::min(qmin, b->q[m]);
-        return launch_sweep_batch_direct(key.kw, qmin, cr.run_wpb, cr.ntiles * cr.run_wpb,
-                                         b->ncu ? b->ncu : 256, b->models, cr.tiles, cr.ntiles, st);
+        return launch_sweep_batch_direct(key.kw, qmin, cr.wpb, cr.ntiles * cr.wpb, units(b), b->models,
+                                         cr.tiles, cr.ntiles, st);
     }
-    return launch_sweep_batch(key.kw, key.pf, cr.run_wpb, b->models, cr.tiles, cr.ntiles, counter,
+    return launch_sweep_batch(key.kw, key.pf, cr.wpb, b->models, cr.tiles, cr.ntiles, counter,
                               class_grid(b, cr), st);
 }
 
@@ -219,21 +333,30 @@ int enqueue_round(mi3_batch* b, std::vector<hipEvent_t>& events) {
                        dim3(256), 0, b->stream, (const BatchModel*)b->models,
                        (uint32_t* const*)b->pos_ptrs);
     BCHK(b, hipGetLastError());
+    // unstaged classes first, one after another: side by side, or beside staged ones,
+    // their waves start or drift apart, the rows they share leave the L2s, and
+    // each takes several times as long (L=301 q=4 and L=400 q=21, 1024 walkers, 4
+    // sweeps: 1.0 and 3.2 ms alone, 9.2 ms together; L=400 and 600 q=21, 2048 walkers, 2
+    // sweeps: 8.7 ms one after another, 16.6 with the first staged beside the second).
+    // Those that the L2s hold follow each other beside the staged ones
+    for (auto& kv : b->classes)
+        if (kv.second.direct && !l2_resident(b, kv.second)) {
+            const hipError_t e = sweep_class(b, kv.first, kv.second, nullptr, b->stream);
+            if (e != hipSuccess)
+                return bfail(b, MI3_EHIP, std::string("batch sweep: ") + hipGetErrorString(e));
+        }
     hipEvent_t fork;
     BCHK(b, hipEventCreateWithFlags(&fork, hipEventDisableTiming));
     events.push_back(fork);
     BCHK(b, hipEventRecord(fork, b->stream));
     uint32_t ci = 0;
     int rc = MI3_OK;
-    // unstaged classes run one after another (on the first one's stream): side
-    // by side their waves drift apart, the rows they share leave the L2s, and
-    // each takes several times as long (L=301 q=4 and L=400 q=21, 1024 walkers,
-    // 4 sweeps: 1.0 and 3.2 ms alone, 9.2 ms together)
-    hipStream_t direct = nullptr;
+    hipStream_t beside = nullptr;
     for (auto& kv : b->classes) {
         ClassRun& cr = kv.second;
-        if (cr.direct && !direct) direct = cr.side;
-        hipStream_t s = cr.direct ? direct : cr.side;
+        if (cr.direct && !l2_resident(b, cr)) continue;
+        if (cr.direct && !beside) beside = cr.side;
+        hipStream_t s = cr.direct ? beside : cr.side;
         if (hipStreamWaitEvent(s, fork, 0) != hipSuccess) { rc = bfail(b, MI3_EHIP, "fork"); break; }
         hipError_t e = sweep_class(b, kv.first, cr, b->counters + ci, s);
         if (e != hipSuccess) {
@@ -341,10 +464,9 @@ int mi3_batch_create(int device, uint32_t nmodels, const uint32_t* L, const uint
                 bad("unpack");
         for (auto& kv : b->classes) {
             if (rc != MI3_OK) break;
-            if (hipStreamCreate(&kv.second.side) != hipSuccess) { bad("stream"); break; }
-            if (build_tiles(b, kv.first, kv.second, 0) != MI3_OK)
-                bad("tiles");
+            if (hipStreamCreate(&kv.second.side) != hipSuccess) bad("stream");
         }
+        if (rc == MI3_OK && choose_tiles(b) != MI3_OK) bad("tiles");
         if (hipStreamSynchronize(b->stream) != hipSuccess) bad("sync");
     }
     if (rc != MI3_OK) {
@@ -466,17 +588,13 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
     BCHK(b, hipEventCreate(&e0));
     BCHK(b, hipEventCreate(&e1));
     uint32_t ci = 0;
+    std::vector<ClassTimes> times;
+    std::vector<bool> may;
     for (auto& kv : b->classes) {
         ClassRun& cr = kv.second;
-        float best = 1e30f;
-        uint32_t best_w = 0;
-        std::vector<uint32_t> opts = tile_options(kv.first.kw);
-        opts.push_back(0);   // the library's choice
-        for (uint32_t w : opts) {
-            rc = build_tiles(b, kv.first, cr, w);
-            if (rc) break;
-            // positions for this launch, then the class sweep alone; the
-            // step counters advance as after any launch
+        // the class sweep alone, in the present tiles; the step counters advance as
+        // after any launch
+        auto sweep_ms = [&](float& ms) {
             hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, b->stream, b->counters + ci, 1u);
             const uint32_t mx = max_steps(b);
             hipLaunchKernelGGL(k_batch_positions,
@@ -488,21 +606,41 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
             hipEventRecord(e1, b->stream);
             hipLaunchKernelGGL(k_batch_advance, dim3((b->n + 255) / 256), dim3(256), 0, b->stream,
                                (const BatchModel*)b->models, b->steps, b->n);
-            if (e != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-                rc = bfail(b, MI3_EHIP, "tuning launch failed");
-                break;
-            }
-            float ms = 0.f;
+            if (e != hipSuccess || hipEventSynchronize(e1) != hipSuccess)
+                return bfail(b, MI3_EHIP, "tuning launch failed");
             hipEventElapsedTime(&ms, e0, e1);
+            return MI3_OK;
+        };
+        float best = 1e30f, ms = 0.f;
+        uint32_t best_w = 0;
+        for (uint32_t w : tile_options(kv.first.kw)) {
+            rc = build_tiles(b, cr, w, false);
+            if (!rc) rc = sweep_ms(ms);
+            if (rc) break;
             if (ms < best) {
                 best = ms;
                 best_w = w;
             }
         }
         if (rc) break;
-        rc = build_tiles(b, kv.first, cr, best_w);
+        may.push_back(may_be_unstaged(b, kv.first, cr));
+        float unstaged = 0.f;
+        if (may.back()) {
+            rc = build_tiles(b, cr, best_w, true);
+            if (!rc) rc = sweep_ms(unstaged);
+            if (rc) break;
+        }
+        rc = build_tiles(b, cr, best_w, false);
         if (rc) break;
+        cr.fixed = true;
+        times.push_back({unstaged, best, best * class_grid(b, cr) / units(b), l2_resident(b, cr)});
         ci++;
+    }
+    if (!rc) {
+        const std::vector<bool> direct =
+            choose_unstaged(may, [&](const std::vector<bool>&) { return times; });
+        size_t i = 0;
+        for (auto& kv : b->classes) kv.second.direct = direct[i++];
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
@@ -512,7 +650,8 @@ int mi3_batch_tune(mi3_batch* b, uint32_t nsweeps) {
 int mi3_batch_tile(mi3_batch* b, uint32_t model, uint32_t* wpb) {
     if (!b || !wpb || model >= b->n) return MI3_EINVAL;
     ClassKey k{state_words(b->L[model]), pf_class(b->q[model])};
-    *wpb = b->classes[k].wpb;
+    const ClassRun& cr = b->classes[k];
+    *wpb = cr.fixed && !cr.direct ? cr.wpb : tile_options(k.kw).back();
     return MI3_OK;
 }
 
@@ -525,7 +664,10 @@ int mi3_batch_set_tile(mi3_batch* b, uint32_t model, uint32_t wpb) {
     hipSetDevice(b->dev);
     BCHK(b, hipStreamSynchronize(b->stream));
     drop_graph(b);
-    return build_tiles(b, k, b->classes[k], wpb);
+    ClassRun& cr = b->classes[k];
+    if (const int rc = build_tiles(b, cr, wpb, false)) return rc;
+    cr.fixed = true;
+    return choose_tiles(b);
 }
 
 int mi3_batch_step_count(mi3_batch* b, uint32_t model, uint64_t* steps) {

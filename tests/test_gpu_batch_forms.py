@@ -68,3 +68,26 @@ def test_batch_unstaged(gpu_ok, models):
     for m, (L, q, N) in enumerate(models):
         _check_model(b.get_seqs(m), data[m][1], data[m][0], 40 + m, [(0, L), (L + (L & 1), L)])
     b.close()
+
+
+# classes that are swept unstaged alone and staged together, and some of each
+MIXED = [[(20, 21, 8192), (130, 21, 8192), (258, 21, 8192)], [(24, 21, 8192), (22, 25, 8192), (20, 16, 512), (33, 4, 6144)],
+         [(20, 21, 2048), (130, 21, 8192), (258, 4, 8192), (300, 21, 1024)]]
+
+
+@pytest.mark.parametrize("models", MIXED)
+@pytest.mark.parametrize("tune", [False, True])
+def test_batch_of_several_classes(gpu_ok, models, tune):
+    b, data = _batch(models)
+    if tune:
+        b.tune(1)
+        for m, (J, s0) in enumerate(data):
+            b.set_seqs(m, s0)
+    start = [b.step_count(m) for m in range(len(models))]
+    b.run(1)
+    b.run(1)
+    for m, (L, q, N) in enumerate(models):
+        t = start[m]
+        _check_model(b.get_seqs(m), data[m][1], data[m][0], 40 + m, [(t, L), (t + L + (L & 1), L)])
+        assert b.tile(m) in (128, 256, 512)
+    b.close()
