@@ -29,10 +29,16 @@ int launched() {
 }
 
 bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-}  // namespace
 
-// 128 x 128 GEMM tiles that fill 256 CUs twice.
-static constexpr int64_t GEMM_LARGE_TILES = 512;
+// Compute units of the current device.
+int compute_units() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+        return 256;
+    return n;
+}
+}  // namespace
 
 extern "C" {
 
@@ -53,11 +59,13 @@ int mi3_gemm_bf16(void* stream, int transA, int transB, int M, int N, int K, flo
     const bf16* a = static_cast<const bf16*>(A);
     const bf16* b = static_cast<const bf16*>(B);
     bf16* cb = static_cast<bf16*>(Cb);
-    // 128 x 128 tiles where they give every CU two; else 64 x 64, which read
-    // LDS twice as often per product but are four times as many (4872 x 512 over
-    // K = 4096: 156 against 616)
+    // 128 x 128 tiles where they give every CU two and have enough products to pay
+    // for their fewer waves; else 64 x 64, which read LDS twice as often per product
+    // but are four times as many, and six instead of two to a CU (us, 128 and 64: 4096
+    // x 4872 over K = 512 64 and 74, 256 49 and 45, 64 38 and 26; 2904 x 3888 over 8 25
+    // and 16; 4872 x 512 over 4096, 156 and 616 tiles, 72 and 62)
     auto tiles = [&](int t) { return (int64_t)((N + t - 1) / t) * ((M + t - 1) / t); };
-    const int t = tiles(128) >= GEMM_LARGE_TILES ? 128 : 64;
+    const int t = K >= 384 && tiles(128) >= 2 * compute_units() ? 128 : 64;
     const dim3 grid((N + t - 1) / t, (M + t - 1) / t);
 #define MI3_G(TA_, TB_)                                                                        \
     if (t == 128)                                                                              \
