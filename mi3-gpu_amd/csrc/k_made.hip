@@ -183,10 +183,11 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, float al
 
 // h1[b][k] = b1[k] + sum_i W1t[(q*i + s_i)*H + k]  (W1t: (L*q, H), masked);
 // h1b = bf16(relu(h1)).  A thread forms V neighbouring units of EMB
-// neighbouring sequences, sites in order: EMB independent sums of V-wide
-// loads keep the gathered rows (bound by L2) in flight.
-constexpr int EMB = 4;
-template <int V>
+// neighbouring sequences, sites in order, four sites' loads in flight.  Bound by
+// their latency while the chip has waves to spare, then by the gathered rows from
+// L2, which wide loads and several sequences to a thread take in fewer
+// instructions.
+template <int V, int EMB>
 __global__ __launch_bounds__(256) void k_made_embed(const uint8_t* __restrict__ seq, uint32_t ld,
                                                     uint32_t B, uint32_t L, uint32_t q, uint32_t H,
                                                     const float* __restrict__ W1t,

@@ -87,15 +87,22 @@ int mi3_made_embed(void* stream, const uint8_t* seq, uint32_t ld, uint32_t B, ui
                    void* h1b) {
     if (!seq || !W1t || !b1 || !h1 || !h1b || ld < B || q < 2 || q > MAX_Q)
         return mfail(MI3_EINVAL, "made_embed: bad arguments");
-    if (B == 0 || H == 0) return MI3_OK;
-    const uint64_t nb = (B + EMB - 1) / EMB;
+    if (B == 0 || H == 0) return mfail(MI3_EHIP, "made_embed: no sequences or no units");
     bf16* hb = static_cast<bf16*>(h1b);
-    if (H % 4 == 0 && al16(W1t) && al16(b1) && al16(h1) && al16(h1b))
-        hipLaunchKernelGGL(k_made_embed<4>, dim3(blocks(nb * (H / 4))), dim3(256), 0, S(stream),
-                           seq, ld, B, L, q, H, W1t, b1, h1, hb);
-    else
-        hipLaunchKernelGGL(k_made_embed<1>, dim3(blocks(nb * H)), dim3(256), 0, S(stream), seq, ld,
-                           B, L, q, H, W1t, b1, h1, hb);
+    // One unit of one sequence to a thread while those are few, else four units of one
+    // or two sequences (us at L=232 q=21, 512 units, by units and sequences of a thread:
+    // 64 sequences 1/1 16, 4/1 26, 4/2 40, 4/4 66; 512 34, 34, 51; 2048 73, 47, 55; 4096
+    // 145, 91, 76; where units are no multiple of 4, 1024 38 and 1/4 47, 2048 73 and 61)
+    const uint64_t n = (uint64_t)B * H;
+#define MI3_EMBED(V, E)                                                                          \
+    hipLaunchKernelGGL((k_made_embed<V, E>), dim3(blocks((uint64_t)((B + E - 1) / E) * (H / V))), \
+                       dim3(256), 0, S(stream), seq, ld, B, L, q, H, W1t, b1, h1, hb)
+    const bool wide = H % 4 == 0 && al16(W1t) && al16(b1) && al16(h1) && al16(h1b);
+    if (wide && n > 5ull << 18) MI3_EMBED(4, 2);
+    else if (wide && n > 3ull << 17) MI3_EMBED(4, 1);
+    else if (n > 3ull << 18) MI3_EMBED(1, 4);
+    else MI3_EMBED(1, 1);
+#undef MI3_EMBED
     return launched();
 }
 

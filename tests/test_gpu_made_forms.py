@@ -25,3 +25,33 @@ def test_gemm_tiles_by_depth(gpu_ok, M, N, K, ta, tb):
     d.sync()
     np.testing.assert_array_equal(d.read('C'), 2 * (A @ B))
     d.close()
+
+
+# one unit of a sequence to a thread; four of one (393216 units on) and of two (1310720);
+# four sequences of a unit where units are no multiple of 4 (786432)
+@pytest.mark.parametrize("L,q,H,B", [(9, 21, 512, 768), (9, 21, 512, 769), (6, 4, 512, 2560), (6, 4, 512, 2563), (5, 25, 4, 98305),
+                                     (7, 3, 250, 3145), (7, 3, 250, 3147), (4, 17, 6, 131073), (300, 21, 64, 17)])
+def test_embedding_by_size(gpu_ok, L, q, H, B):
+    from mi3gpu._lib import lib
+    rng = np.random.default_rng(B)
+    ld = B + 5
+    s = rng.integers(0, q, (L, ld)).astype('u1')
+    W = rng.normal(size=(L * q, H)).astype('f4')
+    b1 = rng.normal(size=H).astype('f4')
+    d = _arrays(s=s, W=W, b1=b1, h=np.zeros((B, H), 'f4'), hb=np.zeros((B, H), 'u2'))
+    assert lib().mi3_made_embed(d.stream, d['s'], ld, B, L, q, H, d['W'], d['b1'], d['h'], d['hb']) == 0
+    d.sync()
+    h = np.repeat(b1[None], B, axis=0)      # float32, sites in order, as the kernel adds
+    for i in range(L):
+        h += W[i * q + s[i, :B].astype(int)]
+    np.testing.assert_array_equal(d.read('h'), h)
+    np.testing.assert_array_equal(d.read('hb'), _to_bf16_bits(np.maximum(h, 0)))
+    d.close()
+
+
+def test_embedding_of_nothing_is_refused(gpu_ok):
+    from mi3gpu._lib import lib
+    d = _arrays(s=np.zeros((2, 16), 'u1'), W=np.zeros((8, 4), 'f4'), b=np.zeros(4, 'f4'), h=np.zeros(4, 'f4'))
+    for B, H in ((0, 4), (4, 0)):
+        assert lib().mi3_made_embed(d.stream, d['s'], 16, B, 2, 4, H, d['W'], d['b'], d['h'], d['h']) < 0
+    d.close()
