@@ -12,6 +12,8 @@
 // site-major (L rows of `ld` bytes), the engine's walker layout.
 #include "common.h"
 
+#include <type_traits>
+
 namespace mi3 {
 
 typedef __bf16 bf16;
@@ -262,52 +264,61 @@ __global__ __launch_bounds__(64 * EG_WAVES) void k_made_embed_grad(
     for (int x = 0; x < EG_LPW; x++) acc[x] = (fv)0.f;
     for (uint32_t c0 = 0; c0 < B; c0 += EG_CHUNK) {
         const uint32_t n = B - c0 < EG_CHUNK ? B - c0 : EG_CHUNK;
-        // ranks within groups of 64 (sequences past the batch: letter q)
-        uint32_t s[EG_GROUPS / EG_WAVES], rank[EG_GROUPS / EG_WAVES];
+        // (a whole chunk with its number of groups known to the compiler: 4% of 4096 x 232
+        // x 512)
+        auto sort = [&](auto full) __attribute__((always_inline)) {
+            // groups, dealt to the waves in turn
+            const uint32_t ng = decltype(full)::value ? (uint32_t)EG_GROUPS : (n + 63) / 64;
+            // ranks within groups of 64 (sequences past the batch: letter q)
+            uint32_t s[EG_GROUPS / EG_WAVES], rank[EG_GROUPS / EG_WAVES];
 #pragma unroll
-        for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
-            const uint32_t g = wave * (EG_GROUPS / EG_WAVES) + x, b = g * 64 + lane;
-            s[x] = q;
-            if (b < n) {
-                s[x] = si[c0 + b];
-                if (s[x] >= q) s[x] = q - 1;
+            for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
+                const uint32_t g = EG_WAVES * x + wave, b = g * 64 + lane;
+                s[x] = q;
+                if (!decltype(full)::value && g >= ng) continue;
+                if (b < n) {
+                    s[x] = si[c0 + b];
+                    if (s[x] >= q) s[x] = q - 1;
+                }
+                rank[x] = 0;
+                uint32_t c = 0;
+                for (uint32_t a = 0; a < q; a++) {
+                    const uint64_t m = __ballot(s[x] == a);
+                    const uint32_t r = __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                    rank[x] = s[x] == a ? r : rank[x];
+                    c = lane == a ? (uint32_t)__popcll(m) : c;
+                }
+                if (lane < 32) cnt[g][lane] = c;
             }
-            rank[x] = 0;
-            uint32_t c = 0;
-            for (uint32_t a = 0; a < q; a++) {
-                const uint64_t m = __ballot(s[x] == a);
-                const uint32_t r = __builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-                rank[x] = s[x] == a ? r : rank[x];
-                c = lane == a ? (uint32_t)__popcll(m) : c;
+            __syncthreads();
+            // places: letters in order, within a letter the groups in order
+            if (threadIdx.x < 32) {
+                uint32_t t = 0;
+                for (uint32_t g = 0; g < ng; g++) t += cnt[g][threadIdx.x];
+                uint32_t before = 0;
+                for (uint32_t a = 0; a < q; a++) {
+                    const uint32_t ta = __shfl(t, a, 32);
+                    before += a < threadIdx.x ? ta : 0u;
+                }
+                off[threadIdx.x] = before;
+                for (uint32_t g = 0; g < ng; g++) {
+                    const uint32_t c = cnt[g][threadIdx.x];
+                    cnt[g][threadIdx.x] = before;
+                    before += c;
+                }
+                if (threadIdx.x == 31) off[32] = before;
             }
-            if (lane < 32) cnt[g][lane] = c;
-        }
-        __syncthreads();
-        // places: letters in order, within a letter the groups in order
-        if (threadIdx.x < 32) {
-            uint32_t t = 0;
-            for (uint32_t g = 0; g < EG_GROUPS; g++) t += cnt[g][threadIdx.x];
-            uint32_t before = 0;
-            for (uint32_t a = 0; a < q; a++) {
-                const uint32_t ta = __shfl(t, a, 32);
-                before += a < threadIdx.x ? ta : 0u;
-            }
-            off[threadIdx.x] = before;
-            for (uint32_t g = 0; g < EG_GROUPS; g++) {
-                const uint32_t c = cnt[g][threadIdx.x];
-                cnt[g][threadIdx.x] = before;
-                before += c;
-            }
-            if (threadIdx.x == 31) off[32] = before;
-        }
-        __syncthreads();
+            __syncthreads();
 #pragma unroll
-        for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
-            const uint32_t g = wave * (EG_GROUPS / EG_WAVES) + x;
-            if (s[x] < q) list[cnt[g][s[x]] + rank[x]] = (uint16_t)(g * 64 + lane);
-        }
-        __syncthreads();
+            for (int x = 0; x < EG_GROUPS / EG_WAVES; x++) {
+                const uint32_t g = EG_WAVES * x + wave;
+                if (s[x] < q) list[cnt[g][s[x]] + rank[x]] = (uint16_t)(g * 64 + lane);
+            }
+            __syncthreads();
+        };
+        if (n == EG_CHUNK) sort(std::true_type{});
+        else sort(std::false_type{});
 #pragma unroll
         for (int x = 0; x < EG_LPW; x++) {
             const uint32_t a = wave + EG_WAVES * x;
@@ -340,6 +351,41 @@ __global__ __launch_bounds__(64 * EG_WAVES) void k_made_embed_grad(
         const uint32_t a = wave + EG_WAVES * x;
         if (a < q) *reinterpret_cast<fv*>(dW1t + (size_t)(q * i + a) * H + k) = acc[x];
     }
+}
+
+// The same for few sequences: one work-group per (site, 256 units), a thread keeps
+// its unit's sums of every letter in an LDS column of its own and walks the batch,
+// eight sequences' letters and gradients loaded before their additions.  No
+// sort, whose passes over the letters come to 4 us (rule at the launch).
+constexpr int EGF_T = 256;
+__global__ __launch_bounds__(EGF_T) void k_made_embed_grad_few(
+    const uint8_t* __restrict__ seq, uint32_t ld, uint32_t B, uint32_t q, uint32_t H,
+    const float* __restrict__ dh1, float* __restrict__ dW1t) {
+    __shared__ float sum[EG_QMAX][EGF_T];
+    const uint32_t nkb = (H + EGF_T - 1) / EGF_T, t = threadIdx.x;
+    const uint32_t i = blockIdx.x / nkb, k = (blockIdx.x % nkb) * EGF_T + t;
+    if (k >= H) return;
+    const uint8_t* si = seq + (size_t)i * ld;
+    for (uint32_t a = 0; a < q; a++) sum[a][t] = 0.f;
+    constexpr uint32_t U = 8;
+    auto add = [&](uint32_t letter, float g) {
+        const uint32_t a = __builtin_amdgcn_readfirstlane(letter);
+        sum[a < q ? a : q - 1][t] += g;
+    };
+    uint32_t b = 0;
+    for (; b + U <= B; b += U) {
+        uint32_t s[U];
+        float g[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            s[u] = si[b + u];
+            g[u] = dh1[(size_t)(b + u) * H + k];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) add(s[u], g[u]);
+    }
+    for (; b < B; b++) add(si[b], dh1[(size_t)b * H + k]);
+    for (uint32_t a = 0; a < q; a++) dW1t[(size_t)(q * i + a) * H + k] = sum[a][t];
 }
 
 // Per sequence b (one work-group): nll[b] = -sum_j log softmax(logits_j)[s_j]

@@ -55,3 +55,23 @@ def test_embedding_of_nothing_is_refused(gpu_ok):
     for B, H in ((0, 4), (4, 0)):
         assert lib().mi3_made_embed(d.stream, d['s'], 16, B, 2, 4, H, d['W'], d['b'], d['h'], d['h']) < 0
     d.close()
+
+
+# up to 7 q sequences without a sort; groups of 64 and chunks of 2048 sorted
+@pytest.mark.parametrize("L,q,H,B", [(5, 2, 1, 1), (7, 21, 260, 147), (7, 21, 260, 148), (7, 21, 257, 149), (3, 25, 256, 175),
+                                     (3, 25, 66, 176), (9, 4, 512, 28), (9, 4, 512, 29), (4, 4, 64, 63), (4, 4, 64, 65),
+                                     (4, 9, 300, 2047), (4, 9, 64, 2049)])
+def test_embedding_gradient_by_size(gpu_ok, L, q, H, B):
+    from mi3gpu._lib import lib
+    rng = np.random.default_rng(B)
+    ld = B + 5
+    s = rng.integers(0, q, (L, ld)).astype('u1')
+    dh = rng.normal(size=(B, H)).astype('f4')
+    d = _arrays(s=s, dh=dh, dW=np.ones((L * q, H), 'f4'))
+    assert lib().mi3_made_embed_grad(d.stream, d['s'], ld, B, L, q, H, d['dh'], d['dW']) == 0
+    d.sync()
+    dW = np.zeros((L * q, H), 'f4')      # float32, in batch order, as the kernels add
+    for b in range(B):
+        dW[np.arange(L) * q + s[:, b]] += dh[b]
+    np.testing.assert_array_equal(d.read('dW'), dW)
+    d.close()
