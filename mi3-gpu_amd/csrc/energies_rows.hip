@@ -31,6 +31,10 @@ hipError_t run_shape(const EnergyArgs& a, hipStream_t st, uint32_t stage_kb) {
 //              of L=232 q=8 alone: 405 against 833)
 //   up to 128: 8 x 8: 16384 sequences of L=93 24 / 57, 26 / 55 for 4 x 4; 32768 35 / 58,
 //              36 / 86 for 16 x 8
+//   up to 256 in rows of up to 32 KB of 8 KB chunks: 8 x 16: 46000 sequences of L=93 q=8
+//              58 / 104, 58 / 114 for 16 x 8 (56 / 103 chunk-staged); 65536 75 / 106, 61 /
+//              115 (75 / 109); L=128 q=7 116 / 159, 111 / 178 (114 / 168).  Longer rows 16 x 8
+//              (65536 of L=150 q=8 168 / 274, 240 / 242 for 8 x 16)
 //   beyond:    16 x 8 for up to two state words (65536 sequences of L=93 56 / 87, 69 / 80
 //              for 8 x 8; 2^18 alone 276, of L=232 1253; chunk-staged 327 and 1649),
 //              16 x 16 for wide rows (L=232 q=8: 1464 against 2249 alone); 8 x 16 for
@@ -40,6 +44,8 @@ hipError_t run_kw(const EnergyArgs& a, hipStream_t st) {
     const bool wide = 4ull * a.nchunk * NPC * 1024 > 163840;
     if (a.nseq <= 32 * a.ncu && !wide) return run_shape<KW, 4, 4, NPC>(a, st, 16);
     if (a.nseq <= 128 * a.ncu) return run_shape<KW, 8, 8, NPC>(a, st, 32);
+    if constexpr (KW == 1 && NPC == 8)
+        if (a.nseq <= 256 * a.ncu && a.nchunk <= 4) return run_shape<KW, 8, 16, NPC>(a, st, 32);
     if constexpr (KW <= 2)
         return wide ? run_shape<KW, 16, 16, NPC>(a, st, 64) : run_shape<KW, 16, 8, NPC>(a, st, 32);
     else
