@@ -319,7 +319,7 @@ struct Walkers {
     uint32_t st[S][KW];       // residues of sites j + 32k, four to a word
     // this step's current residues, byte s % 4 of word s / 4, kept for its end;
     // fetched again there where the state leaves no registers for them
-    static constexpr bool KEEP = KW * S < 64;
+    static constexpr bool KEEP = KW * S <= 48;
     uint32_t kept[KEEP ? NP : 1];
     uint32_t Xe, Xo;          // this lane's draws (steps 2h, 2h+1 of its own pair)
     int remap;                // bpermute address: row lane e <- the lane deciding slot e
