@@ -82,7 +82,10 @@ __global__ __launch_bounds__(256) void k_pack_residues(const uint8_t* __restrict
 // (5 units, else 3) whose buffers fit 40 KiB, so that four waves share a CU.
 constexpr uint32_t BC_PLANES_Q = 7;   // largest q of three planes
 constexpr uint32_t BC_UNIT = 128;     // sequences
-constexpr uint32_t BC_PART = 65536;   // most units that a wave sums in float32 (2^23 sequences)
+// most units that a wave sums in float32 (2^23 sequences; whole numbers are exact to
+// 2^24).  Parts reach it from 2^28 sequences on for few blocks (32 parts), and
+// from 2^23 on where a wave takes whole blocks (L=255 q=25)
+constexpr uint32_t BC_PART = 65536;
 inline uint32_t bc_planes(uint32_t q) { return q <= BC_PLANES_Q ? 3 : 5; }
 inline size_t bc_lds_bytes(uint32_t q, uint32_t tile, uint32_t stage) {
     const uint32_t sites = 2 * (tile / q + 2);

@@ -296,7 +296,8 @@ int pin_get(mi3_ctx* c, size_t bytes) {
 
 // Parts of the sequence range of a 128 x 128 block of the bicount kernel: enough
 // that there are about four waves for each SIMD (one fits at a time), of at
-// least 2048 sequences each, and below 2^24 (a wave sums in float32).
+// least 2048 sequences each.  (How many a wave sums at a time is the kernel's
+// business: BC_PART.)
 uint32_t bicount_split(const mi3_ctx* c, uint32_t nseq) {
     const uint32_t Lq = c->L * c->q;
     const uint32_t nblk = (Lq + 127) / 128;
@@ -308,7 +309,6 @@ uint32_t bicount_split(const mi3_ctx* c, uint32_t nseq) {
     if (ksplit > kmax) ksplit = kmax;
     if (ksplit > 32) ksplit = 32;
     if (ksplit < 1) ksplit = 1;
-    while ((uint64_t)((ksteps + ksplit - 1) / ksplit) * 32 >= (1ull << 24)) ksplit++;
     return ksplit;
 }
 
