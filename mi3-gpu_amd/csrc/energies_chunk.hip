@@ -45,8 +45,10 @@ hipError_t run_pf(const EnergyArgs& a, hipStream_t st) {
 
 template <>
 hipError_t launch_energies_chunks<MI3_KW>(const EnergyArgs& a, hipStream_t st) {
+    // (up to 8 letters and two state words always take staged rows)
+    if constexpr (MI3_KW > 2)
+        if (pf_class(a.q) == 1) return run_pf<MI3_KW, 1>(a, st);
     switch (pf_class(a.q)) {
-        case 1: return run_pf<MI3_KW, 1>(a, st);
         case 4: return run_pf<MI3_KW, 4>(a, st);
         case 7: return run_pf<MI3_KW, 7>(a, st);
         case 10: return run_pf<MI3_KW, 10>(a, st);

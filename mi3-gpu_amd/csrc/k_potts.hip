@@ -1096,10 +1096,9 @@ __global__ __launch_bounds__(64 * NWAVES) void k_energies(
 
     // the padded chunk is PF float4 per thread of the first DMA_T threads
     // (the chunk layout's unit); waves beyond them take no part in staging
-    constexpr int DMA_T = NT < 512 ? NT : 512;
-    // (a tile of fewer than 512 threads copies a chunk in several passes)
-    constexpr int PASS = 512 / DMA_T;
-    constexpr uint32_t chb = PF * 512 * 16;  // padded chunk (bytes)
+    constexpr int DMA_T = 512;
+    static_assert(NT >= DMA_T, "a chunk is copied in one pass");
+    constexpr uint32_t chb = PF * DMA_T * 16;  // padded chunk (bytes)
     const int tid = threadIdx.x;
     const uint32_t lane = tid & 63;
     const uint32_t j = lane & 31;
@@ -1146,7 +1145,7 @@ __global__ __launch_bounds__(64 * NWAVES) void k_energies(
         barrier_copies_in_flight();
     } else {
         // first unit: row 0, chunk 0
-        if (stage) chunk_dma<PF * PASS, DMA_T>(rJ, voff, 0, ldsb, wave);
+        if (stage) chunk_dma<PF, DMA_T>(rJ, voff, 0, ldsb, wave);
         wait_vmem();
         __syncthreads();
     }
@@ -1184,7 +1183,7 @@ __global__ __launch_bounds__(64 * NWAVES) void k_energies(
                         const uint32_t ni = last_chunk ? i + 1 : i;
                         const uint32_t nc = last_chunk ? ((i + 2) >> 5) : (uint32_t)k + 1;
                         if (stage)
-                            chunk_dma<PF * PASS, DMA_T>(rJ, voff, (ni * nchunk + nc) * chb,
+                            chunk_dma<PF, DMA_T>(rJ, voff, (ni * nchunk + nc) * chb,
                                                         ldsb + (buf ^ 1) * chb, wave);
                     }
                     cb = ldsb + buf * chb;

@@ -46,8 +46,9 @@ struct SweepDisp {
             if (w <= 128) return sweep_kws<KW, PF, 8, 8>(a, st);
             if (w <= 256) return sweep_kws<KW, PF, 8, 16>(a, st);
             // four state words do not fit 16 slots in 128 registers; the
-            // spills still pay for q > 8, not for the small chunks of q <= 8
-            if constexpr (KW == 4 && PF == 1)
+            // spills still pay for q > 8, not for the small chunks of q <= 8 (which
+            // come here in tiles of 512 for three words and four alone)
+            if constexpr (KW != 3 && PF == 1)
                 return sweep_kws<KW, PF, 8, 16>(a, st);
             else
                 return sweep_kws<KW, PF, 16, 16>(a, st);
