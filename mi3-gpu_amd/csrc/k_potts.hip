@@ -1300,8 +1300,8 @@ __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(4, 
 }
 
 // No staging: one wave per work-group, ROWS neighbouring rows at a time (of one
-// chunk, so that they share its partners), all their gathers in flight, summed
-// row by row as the staged forms do.  Lanes whose partner does not count read the row all the same, and
+// chunk, so that they share its partners), all their gathers of a chunk in
+// flight.  Lanes whose partner does not count read the row all the same, and
 // select its couplings away (as a 0 factor, an infinite one would make NaN of
 // the energies of sequences that do not hold it, or hold it in a row that counts).
 template <int NC>
@@ -1319,31 +1319,28 @@ __global__ __launch_bounds__(64) void k_energies_direct(
     for (uint32_t i0 = 0; i0 + 1 < L; i0 += ROWS) {
         const uint32_t kp = i0 >> 5;
         uint32_t base[ROWS][S];
-        // whether a coupling counts: in the row's own chunk those of partners past it,
-        // then all; none in rows past the last, which repeat it
-        bool all[ROWS], own[ROWS];
+        // whether a coupling counts: in the first chunk those of partners past the
+        // row, then all; none in rows past the last, which repeat it
+        bool all[ROWS], counts[ROWS];
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
             const uint32_t i = i0 + r + 1 < L ? i0 + r : L - 2;
             w.row_bases(i, lane, q, j * 4 + i * NC * chb, base[r]);
             all[r] = i == i0 + r;
-            own[r] = all[r] && j > (i & 31);
+            counts[r] = all[r] && j > (i & 31);
         }
-        float v[NC][ROWS];
 #pragma unroll
         for (int k = 0; k < NC; k++) {
             if ((uint32_t)k < kp) continue;
+            float v[ROWS];
 #pragma unroll
             for (int r = 0; r < ROWS; r++)
-                v[k][r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
                     rJ, base[r][0] + byte_x128(w.st[0][k >> 2], k & 3), k * chb, 0));
-        }
 #pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-#pragma unroll
-            for (int k = 0; k < NC; k++) {
-                if ((uint32_t)k < kp) continue;
-                acc[0] += ((uint32_t)k == kp ? own[r] : all[r]) ? v[k][r] : 0.f;
+            for (int r = 0; r < ROWS; r++) {
+                acc[0] += counts[r] ? v[r] : 0.f;
+                counts[r] = all[r];
             }
         }
     }

@@ -23,22 +23,3 @@ def test_energy_shapes(gpu_ok, tmp_path, L, q, n):
     E = g.getBuf('E large').read()
     # float32 sums of L(L-1)/2 terms: 1e-5 of the sum of magnitudes, as for the other sizes
     assert (np.abs(E - cboracle.energies(s, J)) / cboracle.energies(s, np.abs(J))).max() < 1e-5
-
-
-# unstaged, rows and chunks staged: each count another form or tile
-@pytest.mark.parametrize("L,q", [(40, 7), (93, 6), (130, 21), (300, 8), (600, 9)])
-def test_energies_do_not_depend_on_the_count(gpu_ok, tmp_path, L, q):
-    """The same bits for a sequence whatever set it is in (more than 5 letters)."""
-    N = 20000
-    J = model(L, q, 3)
-    s = seqs_rand(N, L, q, 4)
-    g = make_gpu(tmp_path, L, q, 512, wgsize=512)
-    g.initLargeBufs(N)
-    g.setBuf('J', J)
-    got = []
-    for n in (N, 9001, 4097, 2048, 513, 1):
-        g.setBuf('seq large', s[:n])
-        g.calcEnergies('large')
-        got.append(g.getBuf('E large').read())
-    for E in got[1:]:
-        np.testing.assert_array_equal(E, got[0][:len(E)])
