@@ -659,7 +659,9 @@ __global__ __launch_bounds__(MF_THREADS, KS > 2 ? 4 : 5) void k_made_fused(
         asm volatile("" : "+v"(tid));
         lr = tid & 15;
         lg = (tid >> 4) & 3;
-        // uniforms of sites j .. j + MF_T - 1
+        // uniforms of sites j .. j + MF_T - 1, one per thread (their last reads, in
+        // (D) of site j - 1, lie before the barrier that follows it; the next ones, in
+        // (D) of this site, after those of (A) and (C))
         if (draw && j % MF_T == 0) {
             const uint4 r = philox4x32_10(
                 make_uint4(j + ((uint32_t)tid >> 4), walker_base + tile0 + (tid & 15), counter,
@@ -694,10 +696,9 @@ __global__ __launch_bounds__(MF_THREADS, KS > 2 ? 4 : 5) void k_made_fused(
         made_product(sm.h2, w3r, H, sm.part[wave], lr, lg, wave);
         __syncthreads();
         load_w2(j + 1, 0);
-        // (D) softmax and the letter: 16 lanes per walker (walker tid / 16;
-        // lane l holds letters l and l + 16), max, sum and the inverse-CDF
-        // search by 16-lane shuffles and one ballot; wave 1 then draws the
-        // next site's uniforms
+        // (D) softmax and the letter: 16 lanes per walker (walker tid / 16; lane l
+        // holds letters l and l + 16): max by row rotations, prefix sums by row
+        // shifts, the inverse-CDF search by a ballot for each half of the letters
         float zs, mxs, ses;   // this lane's logit if the letter is s % 16, max, sum
         uint32_t ls;
         {
