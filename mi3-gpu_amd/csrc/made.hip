@@ -90,15 +90,16 @@ int mi3_made_embed(void* stream, const uint8_t* seq, uint32_t ld, uint32_t B, ui
     if (B == 0 || H == 0) return mfail(MI3_EHIP, "made_embed: no sequences or no units");
     bf16* hb = static_cast<bf16*>(h1b);
     // One unit of one sequence to a thread while those are few, else four units of one
-    // or two sequences (us at L=232 q=21, 512 units, by units and sequences of a thread:
-    // 64 sequences 1/1 16, 4/1 26, 4/2 40, 4/4 66; 512 34, 34, 51; 2048 73, 47, 55; 4096
-    // 145, 91, 76; where units are no multiple of 4, 1024 38 and 1/4 47, 2048 73 and 61)
+    // sequence, then of four (us alone at L=232 q=21, 512 units, by units and sequences
+    // of a thread: 64 sequences 1/1 16, 4/1 26, 4/4 66; 512 34, 34, 72; 2048 73, 47, 68;
+    // 4096 145, 91, 83, and 76 of 4/2, which beside other contexts' steps cost 4 more
+    // than 4/4; where units are no multiple of 4, 1024 38 and 1/4 47, 2048 73 and 61)
     const uint64_t n = (uint64_t)B * H;
 #define MI3_EMBED(V, E)                                                                          \
     hipLaunchKernelGGL((k_made_embed<V, E>), dim3(blocks((uint64_t)((B + E - 1) / E) * (H / V))), \
                        dim3(256), 0, S(stream), seq, ld, B, L, q, H, W1t, b1, h1, hb)
     const bool wide = H % 4 == 0 && al16(W1t) && al16(b1) && al16(h1) && al16(h1b);
-    if (wide && n > 5ull << 18) MI3_EMBED(4, 2);
+    if (wide && n > 3ull << 19) MI3_EMBED(4, 4);
     else if (wide && n > 3ull << 17) MI3_EMBED(4, 1);
     else if (n > 3ull << 18) MI3_EMBED(1, 4);
     else MI3_EMBED(1, 1);

@@ -27,9 +27,9 @@ def test_gemm_tiles_by_depth(gpu_ok, M, N, K, ta, tb):
     d.close()
 
 
-# one unit of a sequence to a thread; four of one (393216 units on) and of two (1310720);
+# one unit of a sequence to a thread; four of one (393216 units on) and of four (1572864);
 # four sequences of a unit where units are no multiple of 4 (786432)
-@pytest.mark.parametrize("L,q,H,B", [(9, 21, 512, 768), (9, 21, 512, 769), (6, 4, 512, 2560), (6, 4, 512, 2563), (5, 25, 4, 98305),
+@pytest.mark.parametrize("L,q,H,B", [(9, 21, 512, 768), (9, 21, 512, 769), (6, 4, 512, 3072), (6, 4, 512, 3075), (5, 25, 4, 98305),
                                      (7, 3, 250, 3145), (7, 3, 250, 3147), (4, 17, 6, 131073), (300, 21, 64, 17)])
 def test_embedding_by_size(gpu_ok, L, q, H, B):
     from mi3gpu._lib import lib
