@@ -3,6 +3,7 @@
 // own allocator and stream (the training step's framework) own the memory.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 
 #include "k_made.hip"
@@ -114,14 +115,19 @@ int mi3_made_embed_grad(void* stream, const uint8_t* seq, uint32_t ld, uint32_t 
     if (!seq || !dh1 || !dW1t || ld < B || q < 2 || q > MAX_Q)
         return mfail(MI3_EINVAL, "made_embed_grad: bad arguments");
     if (L == 0 || H == 0) return MI3_OK;
-    // sorting takes longer by the letters, summing in LDS by the sequences (us, sorted
-    // and not: 64 sequences of L=232 q=21, 512 units 10.6 and 7.4, 128 12.3 and 11.2,
-    // 256 14.1 and 18.1; q=25, 200 sequences of L=100 12.6 and 12.6; q=4, 64 sequences of
-    // L=93 4.9 and 5.1)
-    if (B <= 7 * q)
+    // sorting takes longer by the letters, and by the work-groups that share a CU, summing
+    // in LDS by the sequences (us, sorted and not: 64 sequences of L=232 q=21, 512 units
+    // 10.6 and 7.4, 128 12.3 and 11.2, 256 14.1 and 18.1; q=25, 200 sequences of L=100 12.6
+    // and 12.6; q=4, 64 sequences of L=93 4.9 and 5.1; L=318 in 6 work-groups a site,
+    // 359 units, 128 sequences q=2 11.5 and 9.9, q=25 22.6 and 12.4, 256 17.1 and 17.4,
+    // 25.2 and 20.2)
+    const bool wide = H % 4 == 0 && al16(dh1) && al16(dW1t);
+    const int64_t groups = (int64_t)L * (wide ? (H + 255) / 256 : (H + 63) / 64);
+    const int64_t few = 7 * q + std::max<int64_t>(0, groups - 4 * compute_units()) / 4;
+    if (B <= few)
         hipLaunchKernelGGL(k_made_embed_grad_few, dim3(L * ((H + EGF_T - 1) / EGF_T)), dim3(EGF_T), 0,
                            S(stream), seq, ld, B, q, H, dh1, dW1t);
-    else if (H % 4 == 0 && al16(dh1) && al16(dW1t))
+    else if (wide)
         hipLaunchKernelGGL(k_made_embed_grad<4>, dim3(L * ((H + 255) / 256)), dim3(64 * EG_WAVES), 0,
                            S(stream), seq, ld, B, L, q, H, dh1, dW1t);
     else

@@ -57,10 +57,11 @@ def test_embedding_of_nothing_is_refused(gpu_ok):
     d.close()
 
 
-# up to 7 q sequences without a sort; groups of 64 and chunks of 2048 sorted
+# up to 7 q sequences without a sort, more where there are many work-groups (the last
+# two); groups of 64 and chunks of 2048 sorted
 @pytest.mark.parametrize("L,q,H,B", [(5, 2, 1, 1), (7, 21, 260, 147), (7, 21, 260, 148), (7, 21, 257, 149), (3, 25, 256, 175),
                                      (3, 25, 66, 176), (9, 4, 512, 28), (9, 4, 512, 29), (4, 4, 64, 63), (4, 4, 64, 65),
-                                     (4, 9, 300, 2047), (4, 9, 64, 2049)])
+                                     (4, 9, 300, 2047), (4, 9, 64, 2049), (200, 3, 515, 215), (200, 3, 515, 216)])
 def test_embedding_gradient_by_size(gpu_ok, L, q, H, B):
     from mi3gpu._lib import lib
     rng = np.random.default_rng(B)
