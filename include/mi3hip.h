@@ -309,9 +309,10 @@ int mi3_reg_SCADddE(mi3_ctx *ctx, float gamma, float pc, float lam, float r);
  * Many independent Potts models of uneven L and q, each with its own
  * couplings, walkers and random streams (model m is keyed by seed + m and
  * runs exactly the chains a single-model context created with that seed
- * would), swept together: one persistent kernel per class of models sharing
- * the register layout (ceil(L/128) state words, the chunk class of q), the
- * classes on parallel branches of one HIP graph per round.  No counterpart
+ * would), swept together by class of models sharing the register layout
+ * (ceil(L/128) state words, the chunk class of q): classes of few walkers one
+ * after another without staging, the others side by side with a persistent
+ * kernel each, in one HIP graph per round.  No counterpart
  * in the reference, which runs one model per process. */
 typedef struct mi3_batch mi3_batch;
 

@@ -1,8 +1,9 @@
 // libmi3hip.so, batched models: many independent Potts models of uneven L
 // and q, each with its own walkers, couplings and random streams, swept by
-// one persistent kernel per (state words, chunk class) class.  One round
-// (positions of every model, the class sweeps on parallel branches, the
-// step-counter advance) is captured once into a HIP graph and replayed.
+// (state words, chunk class) class: unstaged, one class after another, or by a
+// persistent kernel per class on parallel branches.  One round (positions of
+// every model, the class sweeps, the step-counter advance) is captured once into
+// a HIP graph and replayed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

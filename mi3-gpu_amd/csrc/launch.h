@@ -83,9 +83,9 @@ struct BatchTile {
 inline uint32_t direct_walkers(uint32_t q, uint32_t ncu) { return (q <= 8 ? 12 : 6) * ncu; }
 
 // Largest sequence count whose energies are taken without staging, by the same
-// measure (us, three contexts at once / one alone: L=232 q=21, 2048 sequences 187 /
-// 163 against 324 / 960, 4096 770 / 266 against 321 / 950; L=93 q=4, 4096 sequences
-// 14 / 17 against 18 / 48, 8192 27 / 32 against 19 / 48).
+// measure (us, three contexts at once / one alone: L=232 q=21, 1024 sequences 83 /
+// 133, 2048 200-330 / 165 against 324 / 960, 4096 770 / 266 against 321 / 950; L=93
+// q=4, 4096 sequences 13 / 18 against 18 / 48, 8192 27 / 32 against 19 / 48).
 inline uint32_t direct_sequences(uint32_t q, uint32_t ncu) { return (q <= 8 ? 16 : 8) * ncu; }
 
 // Sites that the energies of many sequences take together as one of q^k letters
@@ -94,10 +94,10 @@ inline uint32_t direct_sequences(uint32_t q, uint32_t ncu) { return (q <= 8 ? 16
 // to stay within MAX_Q letters, and for q = 2 three sites (8 letters, whole rows
 // staged) take as long as four at half the cost of their table.  The table is formed
 // anew when the couplings change (15 us at L=93 q=4 against 8 without folding), so
-// few sequences and short chains are left as they are.  us, before / folded, table
-// included: L=93 q=4, 2^18 sequences 283 / 192, 2^17 154 / 104, 2^16 104 / 100, 2^14
-// 68 / 78; L=232 q=4, 2^18 1381 / 578, 2^16 489 / 297; L=93 q=2, 2^18 273 / 89; L=93
-// q=5, 2^18 296 / 235; L=17 q=4, 2^18 44 / 41.  The error against 64 bits is about
+// few sequences and short chains are left as they are.  us, unfolded / folded, table
+// included: L=93 q=4, 2^18 sequences 247 / 160, 2^17 132 / 87, 2^16 90 / 85, 2^14
+// 61 / 69; L=232 q=4, 2^18 1245 / 518, 2^16 454 / 270; L=93 q=2, 2^18 242 / 78; L=93
+// q=5, 2^18 262 / 222; L=17 q=4, 2^18 35 / 32.  The error against 64 bits is about
 // half (fewer additions).
 inline uint32_t fold_width(uint32_t q) { return q == 2 ? 3 : q <= 5 ? 2 : 1; }
 inline uint32_t fold_sites(uint32_t q, uint32_t L, uint32_t nseq, uint32_t ncu) {

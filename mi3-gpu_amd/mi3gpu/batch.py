@@ -4,9 +4,11 @@ Each model has its own couplings (the reference's packed (L(L-1)/2, q*q)
 float32 layout), walkers and random streams: model m is keyed by seed + m
 and runs exactly the chains a single-model MCMCGPU with that seed would.
 A round (`run(nsweeps)`) is one replay of a HIP graph holding the site lists
-of every model, one persistent sweep kernel per class of models that share
-the register layout, on parallel branches, and the step-counter advance.
-`tune()` picks the walkers per work-group tile of each class by timing.
+of every model, the sweeps of the classes of models that share the register
+layout (those of few walkers one after another, without staging; a persistent
+kernel each for the others, side by side) and the step-counter advance.
+`tune()` picks the form and the walkers per work-group tile of each class by
+timing; `set_tile` asks for a staged tile.
 
 The reference runs one model per process; this module has no counterpart
 there.
@@ -88,8 +90,8 @@ class PottsBatch:
         _check(self._b, lib().mi3_batch_synchronize(self._b))
 
     def tune(self, nsweeps=1):
-        """Time every allowed tile per class on nsweeps real sweeps (the
-        walkers move on) and keep the fastest."""
+        """Time every allowed tile and the unstaged form per class on nsweeps
+        real sweeps (the walkers move on) and keep what is fastest together."""
         _check(self._b, lib().mi3_batch_tune(self._b, int(nsweeps)))
 
     def tile(self, m):
