@@ -185,7 +185,7 @@ std::vector<bool> choose_unstaged(const std::vector<bool>& may, F times) {
     return best;
 }
 
-// Estimate of those times in tiles of w walkers, in us (within a fifth of what
+// Estimate of those times in tiles of w walkers, in us (within a third of what
 // L=40 to 1000 with 512 to 8192 walkers took, to where may_be_unstaged ends).  An
 // unstaged step waits for its gathers, and shares the L2s' lines (as many of a
 // chunk as its 32 sites have letters) with the class's other walkers; a staged
